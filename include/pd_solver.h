@@ -296,6 +296,14 @@ int pd_update(pd_ctx* ctx, const pd_step_params* prm);
 int pd_backup(pd_ctx* ctx);
 int pd_restore(pd_ctx* ctx);
 
+/* The longest wait, in seconds (0 to 60, 2 by default), of the resident
+ * solve that steps systems of up to about 16,000 particles: its workgroups
+ * run at once and await each other's sums.  Where a wait runs out (another
+ * process holds the device's room) the step is solved by the general
+ * kernels, with identical results, and so are the context's later steps
+ * until this is called again. */
+int pd_set_wait_limit(pd_ctx* ctx, double seconds);
+
 /* Wait for all work on the context stream. */
 int pd_synchronize(pd_ctx* ctx);
 

@@ -173,6 +173,17 @@ struct pd_ctx {
   double op_t_mf = 0.0;     // recomputing product
   double op_t_store = 0.0;  // the storing first product of a stored-block step
   double op_t_st = 0.0;     // a streaming product of stored blocks
+
+  // the resident solve of small systems (pd_small.hip); scratch allocated on
+  // its first step
+  int32_t max_cap = 0;             // longest bond list
+  int small_lanes_ok = 0;          // lanes the device was found to hold (-1: not)
+  bool small_off = false;          // a wait ran out in this context: not again
+  unsigned long long spin_ticks = 200000000ull;  // 2 s of the 100 MHz clock
+  double* small_ex = nullptr;      // [2][n][6]
+  double* small_part = nullptr;    // [9][PD_SMALL_UNITS]
+  unsigned int* small_abort = nullptr;
+  unsigned int* h_small_abort = nullptr;  // pinned
 };
 
 struct pd_trainer {
@@ -635,6 +646,50 @@ int enqueue_contact(pd_ctx* c, const pd_step_params* prm) {
   return PD_OK;
 }
 
+// One resident solve at a time per device: two of them could each hold part
+// of the chip and wait for workgroups that find no room.
+std::mutex g_small_mu[64];
+
+// Lanes per row of the small-system step, or 0: the general kernels.  They
+// stay for mixed precision, the learned preconditioner, gap tracking and
+// steps that time their products, and for systems past the unit count
+// where a row per lane fills the chip.
+int small_step_lanes(pd_ctx* c, const pd_step_params* prm) {
+  if (c->small_off || c->n <= 0 || prm->precision != 0 || prm->precond == 2 || prm->track_gap ||
+      prm->timing || c->device >= 64)
+    return 0;
+  const int lanes = pd::small_lanes(c->nslices, c->max_cap);
+  if (!lanes) return 0;
+  if (c->small_lanes_ok != lanes && c->small_lanes_ok != -lanes)
+    c->small_lanes_ok = pd::small_resident(lanes, c->device) >= PD_SMALL_UNITS ? lanes : -lanes;
+  return c->small_lanes_ok == lanes ? lanes : 0;
+}
+
+int small_args(pd_ctx* c, const pd_step_params* prm, int lanes, pd::SmallArgs* g) {
+  if (!c->small_ex) {
+    if (int e = dalloc(c, &c->small_ex, (size_t)c->n * 12)) return e;
+    if (int e = dalloc(c, &c->small_part, 9 * PD_SMALL_UNITS)) return e;
+    if (int e = dalloc(c, &c->small_abort, 1)) return e;
+    if (hipHostMalloc((void**)&c->h_small_abort, sizeof(unsigned int), hipHostMallocDefault) !=
+        hipSuccess)
+      return fail(c, PD_ERR_HIP, "hipHostMalloc failed");
+  }
+  g->units = c->nslices * (lanes / 8);
+  g->nslices = c->nslices;
+  g->ex = c->small_ex;
+  g->start = c->small_part;
+  g->part = c->small_part + 3 * PD_SMALL_UNITS;
+  g->rtol = prm->rtol;
+  g->max_iter = prm->max_iter;
+  g->spin_ticks = c->spin_ticks;
+  g->counters = c->counters;
+  g->aborted = c->small_abort;
+  g->h_aborted = c->h_small_abort;
+  g->h_st = c->h_st;
+  g->h_cnt = c->h_cnt;
+  return PD_OK;
+}
+
 int ensure_rec(pd_ctx* c) {
   if (!c->rec)
     if (int e = dalloc(c, &c->rec, (size_t)c->n * 6)) return e;
@@ -670,8 +725,10 @@ int ensure_blocks(pd_ctx* c) {
 // start is the block-Jacobi one; run_solve_pc replaces z = M r and its
 // partial once the learned blocks exist (launch_pc_infer_start), or keeps it for a
 // block-Jacobi probe.
+// small_lanes != 0: the small-system assembly (fuse, no gap tracking).
 int enqueue_assemble(pd_ctx* c, const pd_step_params* prm,
-                     const pd_step_consts* consts = nullptr, bool fuse = false) {
+                     const pd_step_consts* consts = nullptr, bool fuse = false,
+                     int small_lanes = 0) {
   if (prm->precision == 1)
     if (int e = ensure_mixed(c)) return e;
   pd::launch_reset_counters(c->counters, c->stream);
@@ -684,7 +741,7 @@ int enqueue_assemble(pd_ctx* c, const pd_step_params* prm,
   const bool defer = defer_blocks(prm);
   // the record: positions and p for the matrix-free FP64 products,
   // positions and x for the mixed solve's FP64 residual
-  const bool rec = prm->matrix_free || defer || prm->precision == 1;
+  const bool rec = !small_lanes && (prm->matrix_free || defer || prm->precision == 1);
   if (rec)
     if (int e = ensure_rec(c)) return e;
   {  // the assembly record, the Dirichlet start values (fuse), the range flag
@@ -716,7 +773,7 @@ int enqueue_assemble(pd_ctx* c, const pd_step_params* prm,
   pd::AsmArgs a;
   a.d0 = c->d0;
   a.arec = c->arec;
-  a.rec = prm->matrix_free || defer ? c->rec : nullptr;
+  a.rec = rec && (prm->matrix_free || defer) ? c->rec : nullptr;
   c->mf = prm->matrix_free ? 1 : 0;
   c->blocks_deferred = defer;
   c->blocks32_deferred = prm->precision == 1;  // launch_mx_spmv_store writes them
@@ -767,6 +824,15 @@ int enqueue_assemble(pd_ctx* c, const pd_step_params* prm,
   a.counters = c->counters;
   a.consts = consts;
   a.bond_stats = c->bond_stats;
+  if (small_lanes) {
+    pd::SmallArgs g;
+    if (int e = small_args(c, prm, small_lanes, &g)) return e;
+    pd::launch_small_assemble(small_lanes, a, g, c->stream);
+    CHECK_LAUNCH(c, "assemble");
+    c->mat_prec = 0;
+    c->asm_fresh = true;
+    return PD_OK;  // the solve copies the counters out
+  }
   pd::launch_assemble(a, c->stream);
   CHECK_LAUNCH(c, "assemble");
   c->mat_prec = prm->precision;
@@ -806,6 +872,31 @@ void read_assemble_stats(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st
 // CG on the device; the host waits once per chunk of iterations.
 int run_solve_mixed(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int resumed,
                     bool fused);
+
+// The batch summary of a finished FP64 solve (h_st): most iterations (also
+// returned), all converged, worst relative residual.
+int solve_summary(pd_ctx* c, pd_step_stats* st) {
+  int it = 0, worst = 0;
+  bool conv = true;
+  for (int k = 0; k < c->nspec; ++k) {
+    const pd_cg_state& h = c->h_st[k];
+    it = std::max(it, h.iter);
+    conv = conv && h.converged;
+    const pd_cg_state& w = c->h_st[worst];
+    if (h.rnorm * w.bnorm > w.rnorm * h.bnorm) worst = k;
+  }
+  c->last_iters = it;
+  c->last_converged = conv;
+  c->last_solve_prec = 0;
+  if (st) {
+    st->cg_iterations = it;
+    st->converged = conv ? 1 : 0;
+    st->residual_norm = c->h_st[worst].rnorm;
+    st->b_norm = c->h_st[worst].bnorm;
+    st->refinements = 0;
+  }
+  return it;
+}
 
 // resumed > 0: a captured step already ran the start and `resumed`
 // iterations; the device state is in h_st / h_mx.  No per-launch timing then.
@@ -881,25 +972,8 @@ int run_solve(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int resum
       chunk = next;
     }
   }
-  // the batch summary: most iterations, all converged, worst relative residual
-  int it = 0, worst = 0;
-  bool conv = true;
-  for (int k = 0; k < ns; ++k) {
-    const pd_cg_state& h = c->h_st[k];
-    it = std::max(it, h.iter);
-    conv = conv && h.converged;
-    const pd_cg_state& w = c->h_st[worst];
-    if (h.rnorm * w.bnorm > w.rnorm * h.bnorm) worst = k;
-  }
-  c->last_iters = it;
-  c->last_converged = conv;
-  c->last_solve_prec = 0;
+  const int it = solve_summary(c, st);
   if (st) {
-    st->cg_iterations = it;
-    st->converged = conv ? 1 : 0;
-    st->residual_norm = c->h_st[worst].rnorm;
-    st->b_norm = c->h_st[worst].bnorm;
-    st->refinements = 0;
     st->host_syncs += syncs;
     if (timing) {
       double tot = 0.0;
@@ -1083,7 +1157,7 @@ int run_solve_mixed(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int
 }
 
 int enqueue_update(pd_ctx* c, const pd_step_params* prm,
-                   const pd_step_consts* consts = nullptr) {
+                   const pd_step_consts* consts = nullptr, const unsigned int* skip = nullptr) {
   if (int e = ensure_blocks(c)) return e;  // from the positions they belong to
   double lo[3], hi[3];
   for (int k = 0; k < 3; ++k) {
@@ -1091,7 +1165,7 @@ int enqueue_update(pd_ctx* c, const pd_step_params* prm,
     hi[k] = prm->bmax[k] - prm->wall_radius;
   }
   pd::launch_update(c->n, c->x, c->v, c->sol, c->act, prm->integrator, prm->dt, prm->walls, lo, hi,
-                    prm->restitution, consts, c->stream);
+                    prm->restitution, consts, c->stream, skip);
   CHECK_LAUNCH(c, "update");
   c->asm_fresh = false;
   return PD_OK;
@@ -1438,9 +1512,62 @@ void zero_timing(pd_step_stats* st) {
   st->contact_grid = 0;
 }
 
+// The same step for a system that fits the chip at once: three launches and
+// the update, one wait.  Captured steps (graph) take it too: it has no
+// launches left to save.
+int run_step_small(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int lanes) {
+  if (prm->contact_radius > 0.0) {
+    if (int e = enqueue_contact(c, prm)) return e;
+    if (st) st->contact_grid = c->last_grid;
+  }
+  if (int e = enqueue_assemble(c, prm, nullptr, true, lanes)) return e;
+  std::swap(c->s, c->s_new);  // core/simulator.cuh:2612
+  c->last_learned = false;
+  pd::SmallArgs g;
+  if (int e = small_args(c, prm, lanes, &g)) return e;
+  pd::CgArgs a = cg_args(c, prm->precond);
+  if (prm->matrix_free) a.vals = nullptr;  // else the blocks are written on the way
+  *c->h_small_abort = 0u;
+  const bool deferred = c->blocks_deferred;
+  {
+    std::lock_guard<std::mutex> lock(g_small_mu[c->device]);
+    pd::launch_small_solve(lanes, a, g, c->stream);
+    CHECK_LAUNCH(c, "resident solve");
+    c->blocks_deferred = false;
+    if (int e = enqueue_update(c, prm, nullptr, c->small_abort)) return e;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  }
+  int syncs = 1;
+  if (*c->h_small_abort) {  // no room for all its workgroups at once
+    c->small_off = true;
+    c->blocks_deferred = deferred;
+    pd::launch_small_undo(c->n, c->arec, c->sol, c->stream);
+    CHECK_LAUNCH(c, "solve start");
+    if (int e = run_solve_pc(c, prm, st)) return e;
+    if (int e = enqueue_update(c, prm)) return e;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+  } else {
+    const int it = solve_summary(c, st);
+    if (prm->precond == 1) {
+      c->bj_iters = it;
+      c->pc_since_probe = 0;
+    }
+  }
+  read_assemble_stats(c, prm, st);
+  if (st) {
+    st->host_syncs += syncs;
+    st->operator_mf = c->mf;
+  }
+  if (!c->last_converged)
+    return fail(c, PD_ERR_NOT_CONVERGED, "CG reached the iteration limit before rtol");
+  return PD_OK;
+}
+
 // One step (contact, assembly, stretch commit, solve, update) with the
 // operator prm->matrix_free (0 or 1) names.
 int run_step(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st) {
+  if (!prm->graph || !(prm->contact_radius > 0.0))  // graph and contact: an error below
+    if (const int lanes = small_step_lanes(c, prm)) return run_step_small(c, prm, st, lanes);
   if (prm->graph) {
     const int e = run_step_graph(c, prm, st);
     if (st) st->operator_mf = c->mf;
@@ -1628,6 +1755,8 @@ int pd_ctx_destroy(pd_ctx* c) {
   destroy_graphs(c);
   dfree(c->consts);
   if (c->h_consts) (void)hipHostFree(c->h_consts);
+  dfree(c->small_ex); dfree(c->small_part); dfree(c->small_abort);
+  if (c->h_small_abort) (void)hipHostFree(c->h_small_abort);
   dfree(c->bond_stats); dfree(c->pc_feat); dfree(c->pc_p); dfree(c->pc_w);
   dfree(c->pc_minv); dfree(c->pc_minv32);
   if (c->h_mx) (void)hipHostFree(c->h_mx);
@@ -1752,6 +1881,7 @@ int pd_build_bonds(pd_ctx* c, pd_bond_stats* stats) {
   c->mat_prec = -1;
   c->last_iters = 0;
   c->h_cap = counts;
+  c->max_cap = mxc;
   c->d0_valid = false;
   c->blocks_deferred = false;  // new bond lists: no matrix to keep
   c->blocks32_deferred = false;
@@ -1810,6 +1940,7 @@ int pd_set_bonds(pd_ctx* c, const int32_t* counts, const int32_t* lists, int32_t
   c->mat_prec = -1;
   c->last_iters = 0;
   c->h_cap = cap;
+  c->max_cap = n > 0 ? *std::max_element(cap.begin(), cap.end()) : 0;
   c->d0_valid = false;
   c->blocks_deferred = false;  // new bond lists: no matrix to keep
   c->blocks32_deferred = false;
@@ -1954,8 +2085,10 @@ int pd_step(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st) {
   pd_step_stats local;
   pd_step_stats* s = st ? st : &local;
   zero_timing(s);
-  q.matrix_free = auto_operator(c, prm);
-  const bool measure = q.precision == 0 && !q.graph &&
+  // the resident solve keeps the blocks it forms: nothing to choose or time
+  const bool small = small_step_lanes(c, prm) != 0;
+  q.matrix_free = small ? 1 : auto_operator(c, prm);
+  const bool measure = !small && q.precision == 0 && !q.graph &&
                        (q.matrix_free ? c->op_t_mf <= 0.0 : c->op_t_store <= 0.0);
   if (measure) q.timing = 1;
   const int e = run_step(c, &q, s);
@@ -2012,6 +2145,14 @@ int pd_restore(pd_ctx* c) {
   c->asm_fresh = false;
   HIPCHK(c, hipMemcpyAsync(c->v, c->v_bak, n * 32, hipMemcpyDeviceToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  return PD_OK;
+}
+
+int pd_set_wait_limit(pd_ctx* c, double seconds) {
+  if (!c) return fail(nullptr, PD_ERR_ARG, "null context");
+  if (!(seconds >= 0.0 && seconds <= 60.0)) return fail(c, PD_ERR_ARG, "seconds outside [0, 60]");
+  c->spin_ticks = (unsigned long long)(seconds * 1e8);
+  c->small_off = false;
   return PD_OK;
 }
 

@@ -211,6 +211,32 @@ struct MxArgs {
   SpmvView A64;
 };
 
+// The step of a system whose rows fit the chip at once (pd_small.hip).
+#define PD_SMALL_THREADS 512
+#define PD_SMALL_UNITS 256     // workgroups, one per CU
+#define PD_SMALL_MAX_BONDS 120 // longest list whose blocks a row's lanes hold
+struct SmallArgs {
+  int32_t units;    // workgroups: slices << log2(lanes / 8)
+  int32_t nslices;
+  double* ex;       // [2][n][6] z and the direction, by parity of the iteration
+  double* start;    // [3][units] the start's partials <r,z>, <r,r>, <Sb,Sb>
+  double* part;     // [6][units] <y,p>, <r,z>, <r,r> by parity
+  double rtol;
+  int32_t max_iter;
+  unsigned long long spin_ticks;  // longest wait, 100 MHz clock
+  const pd_step_counters* counters;
+  unsigned int* aborted;    // device word: a wait ran out
+  unsigned int* h_aborted;  // the same on the host, pinned
+  pd_cg_state* h_st;        // pinned results, one per specimen
+  pd_step_counters* h_cnt;  // pinned copy of the assembly's counters
+};
+// lanes per row (8, 16, 32), or 0 where the general kernels take the step
+int small_lanes(int32_t nslices, int32_t max_cap);
+int small_resident(int lanes, int device);
+void launch_small_assemble(int lanes, const AsmArgs& a, const SmallArgs& g, hipStream_t s);
+void launch_small_solve(int lanes, const CgArgs& a, const SmallArgs& g, hipStream_t s);
+void launch_small_undo(int32_t n, const double* arec, double4* x, hipStream_t s);
+
 // Learned block preconditioner: a 16-64-64-8 MLP (BF16 weights, FP32
 // accumulation on MFMA) maps per-particle features to S_p = L L^T + eps I,
 // and M_p = C_p^{-T} S_p C_p^{-1} with D_p = C_p C_p^T (S = I is block Jacobi).
@@ -376,11 +402,12 @@ void launch_mx_apply(const MxArgs& a, hipStream_t s);
 // mixed assembly), and y32 = A32 x32
 void launch_spmv_wide(const MxArgs& a, const double4* x, double4* y, hipStream_t s);
 void launch_spmv_f32(const MxArgs& a, const float4* x, float4* y, hipStream_t s);
-// consts non-null: dt from there
+// consts non-null: dt from there; skip non-null and set: nothing is done
 void launch_update(int32_t n, double4* x, double4* v, const double4* sol,
                    const int32_t* act, int32_t integrator, double dt, int32_t walls,
                    const double* lo, const double* hi, double restitution,
-                   const pd_step_consts* consts, hipStream_t s);
+                   const pd_step_consts* consts, hipStream_t s,
+                   const unsigned int* skip = nullptr);
 void launch_copy(double* dst, const double* src, int32_t n, hipStream_t s);
 // Compares shared-reciprocal quotients with IEEE division on `samples`
 // random operand pairs; *bad counts the differing ones.

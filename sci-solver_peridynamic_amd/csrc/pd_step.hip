@@ -1300,9 +1300,11 @@ struct UpdArgs {
   double hi[3];
   double rest;
   const pd_step_consts* consts;
+  const unsigned int* skip;
 };
 
 __global__ __launch_bounds__(PD_BLOCK) void k_update(UpdArgs a) {
+  if (a.skip && *a.skip) return;
   const int p = blockIdx.x * PD_BLOCK + threadIdx.x;
   if (p >= a.n || a.act[p] == PD_INVISIBLE) return;
   if (a.consts) a.dt = a.consts->dt;
@@ -1338,8 +1340,9 @@ __global__ __launch_bounds__(PD_BLOCK) void k_update(UpdArgs a) {
 void launch_update(int32_t n, double4* x, double4* v, const double4* sol,
                    const int32_t* act, int32_t integrator, double dt, int32_t walls,
                    const double* lo, const double* hi, double restitution,
-                   const pd_step_consts* consts, hipStream_t s) {
+                   const pd_step_consts* consts, hipStream_t s, const unsigned int* skip) {
   UpdArgs a;
+  a.skip = skip;
   a.consts = consts;
   a.n = n;
   a.x = x;

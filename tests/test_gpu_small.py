@@ -1,0 +1,119 @@
+"""The resident step of small systems (up to 256 slices of 64 rows, lists of
+at most 120 bonds) against the oracle, bit for bit: row counts at the edges
+of a unit, of a slice, of the lane counts 32 / 16 / 8 and of its range,
+lists broken in the middle and to the end, both integrators and operators,
+specimens, and a wait that runs out."""
+import ctypes
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as orc
+from pdhelpers import lattice, make_pair, material
+
+pytestmark = pytest.mark.gpu
+pds = pytest.importorskip("pdsolver")
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def pair(n, pull=6.0, factor=3.0):
+    """n rows of a jittered lattice, the first layer fixed, the last pulled."""
+    w = 4 if n < 2000 else 12
+    x4 = lattice(w, w, -(-n // (w * w)), 0.01, 0.05, n)[:n]
+    k = np.arange(n) // (w * w)
+    bc = ((k == 0) | (k == k[-1])).astype(np.int32) if n > w * w else np.zeros(n, np.int32)
+    vbc = np.zeros((n, 4))
+    vbc[(k == k[-1]) & (bc == 1), 2] = pull
+    return make_pair(x4, [material(0.01, factor)], v4=vbc.copy(), bc=bc, vbc=vbc)
+
+
+def compare(S, ctx, steps, **kw):
+    broken = 0
+    for k in range(1, steps + 1):
+        p = dict(dict(dt=1e-4, clock_scale=min(k, 10) / 10.0, precond=1, rtol=1e-8), **kw)
+        so = S.step(orc.make_params(**p))
+        sg = ctx.step(pds.make_params(**p))
+        assert (so.cg_iterations, so.broken_bonds) == (sg.cg_iterations, sg.broken_bonds), k
+        for f, want in (("position", S.x), ("velocity", S.v), ("new_stretch", S.s)):
+            got = ctx.download("stretch" if f == "new_stretch" else f)
+            same = np.array_equal(got[:, :3], want[:, :3]) if got.ndim > 1 else np.array_equal(got, want)
+            assert same, (f, k)
+        broken += sg.broken_bonds
+    assert np.array_equal(ctx.download("bond_top"), S.top)
+    return broken
+
+
+# 1, 63..65: a slice's edge; 4096 / 4097 and 8192 / 8193: the lane counts;
+# 16384 / 16385: the last resident size and the first general one
+@pytest.mark.parametrize("n", [1, 15, 63, 64, 65, 257, 1000, 4096, 4097, 8192, 8193, 16384, 16385])
+def test_sizes_match_oracle(n):
+    say("case small n", n)
+    S, ctx = pair(n)
+    broken = compare(S, ctx, 12 if n < 4000 else 6)
+    say(dict(n=n, broken=broken))
+    ctx.close()
+
+
+@pytest.mark.parametrize("kw", [dict(matrix_free=1), dict(matrix_free=2), dict(precond=0),
+                                dict(integrator=1), dict(max_iter=3), dict(rtol=1e10),
+                                dict(graph=1)])
+def test_options_match_oracle(kw):
+    say("case small", kw)
+    S, ctx = pair(900)
+    o = {k: v for k, v in kw.items() if k not in ("matrix_free", "graph")}
+    for k in range(1, 25):
+        p = dict(dict(dt=1e-4, clock_scale=min(k, 10) / 10.0, precond=1, rtol=1e-8), **o)
+        so = S.step(orc.make_params(**p))
+        sg = ctx.step(pds.make_params(**dict(p, **kw)), allow_fail=True)
+        assert (so.cg_iterations, bool(so.converged), so.broken_bonds) == \
+            (sg.cg_iterations, bool(sg.converged), sg.broken_bonds), k
+        assert np.array_equal(ctx.download("position")[:, :3], S.x[:, :3]), k
+    ctx.close()
+
+
+@pytest.mark.parametrize("factor", [2.5, 3.1, 3.3])
+def test_list_lengths(factor):
+    """Longest lists below and above the 120 blocks a row's lanes hold, and
+    rows that lose most of their bonds."""
+    say("case small horizon", factor)
+    S, ctx = pair(1700, pull=12.0, factor=factor)
+    say(dict(longest=int(ctx.download("bond_top").max()) + 1))
+    assert compare(S, ctx, 20) > 0
+    ctx.close()
+
+
+def test_wait_that_runs_out_falls_back():
+    """A wait limit of zero: every workgroup gives up at its first wait and
+    the general kernels solve the step, with the same results."""
+    say("case small wait limit")
+    L = pds.lib()
+    L.pd_set_wait_limit.argtypes = [ctypes.c_void_p, ctypes.c_double]
+    S, ctx = pair(8000)
+    assert L.pd_set_wait_limit(ctx._h, 0.0) == pds.PD_OK
+    compare(S, ctx, 2)
+    assert L.pd_set_wait_limit(ctx._h, 2.0) == pds.PD_OK
+    compare_from = S.x.copy()
+    for k in range(3, 6):
+        p = dict(dt=1e-4, clock_scale=k / 10.0, precond=1, rtol=1e-8)
+        S.step(orc.make_params(**p))
+        ctx.step(pds.make_params(**p))
+    assert np.array_equal(ctx.download("position")[:, :3], S.x[:, :3])
+    assert not np.array_equal(compare_from, S.x)
+    assert L.pd_set_wait_limit(ctx._h, -1.0) == pds.PD_ERR_ARG
+    ctx.close()
+
+
+def test_operands_out_of_range_take_ieee_forms():
+    """A coordinate outside the shared-reciprocal range: IEEE quotients."""
+    say("case small range flag")
+    x4 = lattice(6, 6, 8, 0.01, 0.0, 3)
+    x4[:, :3] -= x4[0, :3]
+    x4[5, 1] = 1e-200
+    S, ctx = make_pair(x4, [material(0.01)])
+    compare(S, ctx, 6)
+    ctx.close()
