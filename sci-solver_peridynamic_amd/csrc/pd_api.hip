@@ -177,11 +177,12 @@ struct pd_ctx {
   // the resident solve of small systems (pd_small.hip); scratch allocated on
   // its first step
   int32_t max_cap = 0;             // longest bond list
-  int small_lanes_ok = 0;          // lanes the device was found to hold (-1: not)
+  int small_lanes_ok = 0;          // lanes the device holds (negative: does not)
+  int small_fit = -1;              // the units' neighbours fit LDS (-1: not counted yet)
   bool small_off = false;          // a wait ran out in this context: not again
   unsigned long long spin_ticks = 200000000ull;  // 2 s of the 100 MHz clock
   double* small_ex = nullptr;      // [2][n][6]
-  double* small_part = nullptr;    // [9][PD_SMALL_UNITS]
+  double* small_part = nullptr;    // [9][PD_SMALL_ROW]
   unsigned int* small_abort = nullptr;
   unsigned int* h_small_abort = nullptr;  // pinned
 };
@@ -662,13 +663,25 @@ int small_step_lanes(pd_ctx* c, const pd_step_params* prm) {
   if (!lanes) return 0;
   if (c->small_lanes_ok != lanes && c->small_lanes_ok != -lanes)
     c->small_lanes_ok = pd::small_resident(lanes, c->device) >= PD_SMALL_UNITS ? lanes : -lanes;
-  return c->small_lanes_ok == lanes ? lanes : 0;
+  if (c->small_lanes_ok != lanes) return 0;
+  if (lanes == 8 && c->small_fit < 0) {  // once per bond set
+    int* longest = nullptr;
+    int h = 0;
+    if (dalloc(c, &longest, 1) != PD_OK) return 0;
+    pd::launch_small_union(c->n, c->nslices, c->slice_off, c->cap, c->col, longest, c->stream);
+    const bool ok = hipMemcpyAsync(&h, longest, sizeof(int), hipMemcpyDeviceToHost, c->stream) ==
+                        hipSuccess &&
+                    hipStreamSynchronize(c->stream) == hipSuccess;
+    dfree(longest);
+    c->small_fit = ok && h <= PD_SMALL_UNION ? 1 : 0;
+  }
+  return lanes != 8 || c->small_fit == 1 ? lanes : 0;
 }
 
 int small_args(pd_ctx* c, const pd_step_params* prm, int lanes, pd::SmallArgs* g) {
   if (!c->small_ex) {
     if (int e = dalloc(c, &c->small_ex, (size_t)c->n * 12)) return e;
-    if (int e = dalloc(c, &c->small_part, 9 * PD_SMALL_UNITS)) return e;
+    if (int e = dalloc(c, &c->small_part, 9 * PD_SMALL_ROW)) return e;
     if (int e = dalloc(c, &c->small_abort, 1)) return e;
     if (hipHostMalloc((void**)&c->h_small_abort, sizeof(unsigned int), hipHostMallocDefault) !=
         hipSuccess)
@@ -678,7 +691,7 @@ int small_args(pd_ctx* c, const pd_step_params* prm, int lanes, pd::SmallArgs* g
   g->nslices = c->nslices;
   g->ex = c->small_ex;
   g->start = c->small_part;
-  g->part = c->small_part + 3 * PD_SMALL_UNITS;
+  g->part = c->small_part + 3 * PD_SMALL_ROW;
   g->rtol = prm->rtol;
   g->max_iter = prm->max_iter;
   g->spin_ticks = c->spin_ticks;
@@ -1882,6 +1895,7 @@ int pd_build_bonds(pd_ctx* c, pd_bond_stats* stats) {
   c->last_iters = 0;
   c->h_cap = counts;
   c->max_cap = mxc;
+  c->small_fit = -1;
   c->d0_valid = false;
   c->blocks_deferred = false;  // new bond lists: no matrix to keep
   c->blocks32_deferred = false;
@@ -1941,6 +1955,7 @@ int pd_set_bonds(pd_ctx* c, const int32_t* counts, const int32_t* lists, int32_t
   c->last_iters = 0;
   c->h_cap = cap;
   c->max_cap = n > 0 ? *std::max_element(cap.begin(), cap.end()) : 0;
+  c->small_fit = -1;
   c->d0_valid = false;
   c->blocks_deferred = false;  // new bond lists: no matrix to keep
   c->blocks32_deferred = false;

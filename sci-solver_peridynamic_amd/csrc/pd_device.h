@@ -120,12 +120,51 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
 }
 
+// v + (v of the lane M away by xor), the level M of a wave's butterfly sum.
+// Within a row of 16 lanes through DPP moves, across rows through the lane
+// swaps of gfx950 (both operands of the swap hold v, so in every lane their
+// sum is the level's).  A level through the LDS crossbar (__shfl_xor) waits
+// about 130 cycles, this one about 30.
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  const int64_t b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
+}
+template <int M>
+__device__ __forceinline__ double xor_add(double v) {
+  if constexpr (M == 1) return v + dpp_mov<0xb1>(v);                  // quad_perm 1 0 3 2
+  if constexpr (M == 2) return v + dpp_mov<0x4e>(v);                  // quad_perm 2 3 0 1
+  if constexpr (M == 4) return v + dpp_mov<0x1b>(dpp_mov<0x141>(v));  // i ^ 7, then i ^ 3
+  if constexpr (M == 8) return v + dpp_mov<0x128>(v);                 // row_ror 8
+  if constexpr (M >= 16) {
+    const int64_t b = __double_as_longlong(v);
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    const unsigned int l = (unsigned int)b, h = (unsigned int)(b >> 32);
+    u2 sl, sh;
+    if constexpr (M == 16) {
+      sl = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+      sh = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    } else {
+      sl = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+      sh = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+    }
+    const double a = __longlong_as_double(((int64_t)sh.x << 32) | sl.x);
+    const double c = __longlong_as_double(((int64_t)sh.y << 32) | sl.y);
+    return a + c;
+  }
+}
+
 // Sum of a double over the 64 lanes by the xor butterfly m = 32..1; every
 // lane ends with the same value (the order fixed by the oracle's orc_dot).
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);
-  return v;
+  v = xor_add<32>(v);
+  v = xor_add<16>(v);
+  v = xor_add<8>(v);
+  v = xor_add<4>(v);
+  v = xor_add<2>(v);
+  return xor_add<1>(v);
 }
 
 // Tile reduction of one value per thread of a 256-thread workgroup:

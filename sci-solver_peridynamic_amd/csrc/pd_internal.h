@@ -215,12 +215,14 @@ struct MxArgs {
 #define PD_SMALL_THREADS 512
 #define PD_SMALL_UNITS 256     // workgroups, one per CU
 #define PD_SMALL_MAX_BONDS 120 // longest list whose blocks a row's lanes hold
+#define PD_SMALL_ROW 1024      // doubles of a row of partials (padded)
+#define PD_SMALL_UNION 1888    // neighbours of a unit held in LDS (8 lanes per row)
 struct SmallArgs {
   int32_t units;    // workgroups: slices << log2(lanes / 8)
   int32_t nslices;
   double* ex;       // [2][n][6] z and the direction, by parity of the iteration
-  double* start;    // [3][units] the start's partials <r,z>, <r,r>, <Sb,Sb>
-  double* part;     // [6][units] <y,p>, <r,z>, <r,r> by parity
+  double* start;    // [3][PD_SMALL_ROW] the start's partials <r,z>, <r,r>, <Sb,Sb>
+  double* part;     // [6][PD_SMALL_ROW] <y,p>, <r,z>, <r,r> by parity
   double rtol;
   int32_t max_iter;
   unsigned long long spin_ticks;  // longest wait, 100 MHz clock
@@ -235,6 +237,9 @@ int small_lanes(int32_t nslices, int32_t max_cap);
 int small_resident(int lanes, int device);
 void launch_small_assemble(int lanes, const AsmArgs& a, const SmallArgs& g, hipStream_t s);
 void launch_small_solve(int lanes, const CgArgs& a, const SmallArgs& g, hipStream_t s);
+// *longest raised to the longest neighbour list of a unit of 64 rows
+void launch_small_union(int32_t n, int32_t nslices, const int64_t* slice_off, const int32_t* cap,
+                        const int32_t* col, int* longest, hipStream_t s);
 void launch_small_undo(int32_t n, const double* arec, double4* x, hipStream_t s);
 
 // Learned block preconditioner: a 16-64-64-8 MLP (BF16 weights, FP32

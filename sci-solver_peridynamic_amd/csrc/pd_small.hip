@@ -16,8 +16,9 @@
 //   * the workgroups exchange z, p and the partial sums through global
 //     memory without leaving the kernel.
 // Measured at 8,000 rows, 11 iterations: assembly 93 -> 31 us, solve about
-// 590 (44 launches) -> 247 us, the step 744 -> 315 us; at 288 rows the step
-// 400 -> 147 us.
+// 590 (44 launches) -> 140 us, the step 744 -> 217 us; at 288 rows the step
+// 400 -> 124 us.  An iteration at 4,553 rows (143 workgroups): 9.1 us, of
+// which the products and their sums 2.9, the waits for the two sums 3.9.
 #include <math.h>
 
 #include "pd_bond.h"
@@ -33,6 +34,12 @@ constexpr int kThreads = PD_SMALL_THREADS;
 // (i << K) + c of the slice.  The xor butterfly of a slice's wave sum pairs
 // lanes 32, 16, .. 1 apart; a unit holds whole subtrees of its first 6 - K
 // levels, and the remaining K levels join the slice's units.
+// Longest neighbour list of a unit that the solve keeps in LDS.  With 16 and
+// 32 lanes no unit can have more (its rows, their bonds and row 0).
+constexpr int small_union(int lanes) {
+  return lanes == 8 ? PD_SMALL_UNION : kThreads / lanes * (PD_SMALL_MAX_BONDS + 1) + 1;
+}
+
 template <int L>
 struct Unit {
   static constexpr int R = kThreads / L;
@@ -43,10 +50,18 @@ struct Unit {
 // Sum over the first R lanes (R = 16, 32 or 64), the butterfly's levels.
 template <int R>
 __device__ __forceinline__ double unit_sum(double v) {
-#pragma unroll
-  for (int m = R / 2; m >= 1; m >>= 1) v = v + __shfl_xor(v, m, 64);
-  return v;
+  if constexpr (R > 32) v = xor_add<32>(v);
+  if constexpr (R > 16) v = xor_add<16>(v);
+  v = xor_add<8>(v);
+  v = xor_add<4>(v);
+  v = xor_add<2>(v);
+  return xor_add<1>(v);
 }
+
+// Where unit u's partial lies in its row: eight to a 64-byte line, the lines
+// 256 bytes apart so that the polls of all units spread over the memory
+// channels.
+__device__ __forceinline__ int small_slot(int u) { return (u >> 3) * 32 + (u & 7); }
 
 // A partial that no unit has written yet: a signalling NaN, which no
 // arithmetic returns (every partial is the result of an addition).
@@ -63,55 +78,118 @@ __device__ __forceinline__ double get(const double* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Every store of this wave has reached the point where all XCDs see it:
+// stores that others read are agent-scope ones (written through), so their
+// acknowledgement is all there is to wait for.  A release fence writes the
+// whole L2 back on top, 1.5 to 2 us here.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Fold of one partial row over tiles [t0, t0 + nt), nt <= 64, by one wave:
-// fold_partials' tree.  Lane t joins the units of tile t's four slices
-// (levels 2^(K-1) .. 1 of the butterfly within a slice, then (w0 + w1) +
-// (w2 + w3)); tiles beyond nt add 0.0.  WAIT: the partials are written by
-// running workgroups, each is awaited until it is set or `until` (100 MHz
-// clock) has passed; then *late is raised.
-template <int K, bool WAIT>
-__device__ __forceinline__ double fold_units(const double* part, int t0, int nt, int nslices,
-                                             int lane, unsigned long long until, bool* late) {
-  constexpr int U = 1 << K;
-  double w[4][U];
-  const bool mine = lane < nt;
-  bool ready = false;
-  for (unsigned spin = 0; !ready; ++spin) {
-    ready = true;
+// Fold of NV partial rows over tiles [t0, t0 + nt), nt <= 64 >> K, by one
+// wave: fold_partials' tree.  The units' partials are read 64 at a time, one
+// per lane (a lane per tile reading its units one after another asked for
+// eight times the lines, 5 us a fold at 250 units); the lanes of a slice,
+// then those of a tile join through xor levels (2^(K-1) .. 1 within the
+// slice, then (w0 + w1) + (w2 + w3)), and tile t's sum moves to lane t.
+// WAIT: the partials are written by running workgroups, each is awaited
+// until it is set, `until` (100 MHz clock) has passed or another unit has
+// given up (*aborted); then *late is raised.
+template <int K, int NV, bool WAIT>
+__device__ __forceinline__ void fold_units(const double* part, int64_t stride, int t0, int nt,
+                                           int nslices, int lane, unsigned long long until,
+                                           const unsigned int* aborted, bool* late,
+                                           double* out) {
+  const int first = (t0 * 4) << K;
+  const int nu = min(nt * 4, nslices - t0 * 4) << K;  // at most 256
+  double v[NV][4];
+  for (unsigned spin = 0;; ++spin) {
+    bool ready = true;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int s = (t0 + lane) * 4 + j;
-      const bool in = mine && s < nslices;
+    for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int c = 0; c < U; ++c) {
-        w[j][c] = in ? get(part + (s << K) + c) : 0.0;
-        if (WAIT && is_unset(w[j][c])) ready = false;
+      for (int k = 0; k < NV; ++k) {
+        v[k][r] = r * 64 + lane < nu ? get(part + k * stride + small_slot(first + r * 64 + lane))
+                                     : 0.0;
+        if (WAIT) ready = ready && !is_unset(v[k][r]);
       }
-    }
-    if (!WAIT) break;
-    ready = __all(ready);
-    if (!ready && (spin & 15) == 15 && wall_clock64() > until) {
+    if (!WAIT || __all(ready)) break;
+    if ((spin & 15) == 15 &&
+        (wall_clock64() > until ||
+         __hip_atomic_load(aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
       *late = true;
       break;
     }
   }
-  double ws[4];
+  constexpr int TPR = 16 >> K;  // tiles per 64 units
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if constexpr (K == 0) ws[j] = w[j][0];
-    if constexpr (K == 1) ws[j] = w[j][0] + w[j][1];
-    if constexpr (K == 2) ws[j] = (w[j][0] + w[j][2]) + (w[j][1] + w[j][3]);
+  for (int k = 0; k < NV; ++k) {
+    double acc = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      double x = v[k][r];
+      if constexpr (K == 2) x = xor_add<1>(xor_add<2>(x));
+      if constexpr (K == 1) x = xor_add<1>(x);
+      x = xor_add<2 << K>(xor_add<1 << K>(x));
+      const double y = __shfl(x, (lane % TPR) << (2 + K), 64);
+      if (lane / TPR == r && lane < nt) acc = acc + y;
+    }
+    const double w = wave_sum(acc);
+    out[k] = (w + 0.0) + (0.0 + 0.0);
   }
-  double acc = 0.0;
-  if (mine) acc = acc + ((ws[0] + ws[1]) + (ws[2] + ws[3]));
-  const double v = wave_sum(acc);
-  return (v + 0.0) + (0.0 + 0.0);
+}
+
+// acc + t[0] + t[1] + .. + t[n - 1], left to right; the next eight terms are
+// on their way from LDS while eight are added.
+__device__ __forceinline__ double chain_add(double acc, const double* t, int n) {
+  double h[8];
+  int e = 0;
+  if (n >= 8) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) h[u] = t[u];
+    for (; e + 16 <= n; e += 8) {
+      double k[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) k[u] = t[e + 8 + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += h[u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) h[u] = k[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += h[u];
+    e += 8;
+  }
+  for (; e < n; ++e) acc += t[e];
+  return acc;
+}
+
+// The same over t[0 .. n), n <= N wave-uniform, in steps of 16 terms with
+// each term read 16 terms ahead (the terms past a list's end hold -0.0,
+// which changes no sum).  An LDS read costs the same with one lane as with
+// 64: a chain in three lanes of every wave took 32 cycles an addition, all
+// eight waves reading; the chains of all rows side by side in one to three
+// waves take about 10, the latency of the addition.
+template <int N>
+__device__ __forceinline__ double chain_wide(double acc, const double* t, int n) {
+  static_assert(N % 16 == 0 || N % 8 == 0, "whole steps");
+  double h[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) h[u] = u < N ? t[u] : -0.0;
+#pragma unroll
+  for (int e = 0; e < N; e += 16) {
+    if (e >= n) break;  // uniform
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      if (e + u < N) acc += h[u];
+      if (e + 16 + u < N) h[u] = t[e + 16 + u];
+    }
+  }
+  return acc;
 }
 
 }  // namespace
@@ -331,14 +409,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
         double v = acc[k];
         int e = 0;
         if (role < 13) {
-          for (; e + 8 <= m; e += 8) {
-            double x[8];
-#pragma unroll
-            for (int w = 0; w < 8; ++w) x[w] = t[e + w];
-#pragma unroll
-            for (int w = 0; w < 8; ++w) v += x[w];
-          }
-          for (; e < m; ++e) v += t[e];
+          v = chain_add(v, t, m);
         } else if (role == 13) {
           for (; e < m; ++e) v = t[e] < v ? t[e] : v;
         } else {
@@ -478,11 +549,12 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
     live += __shfl_xor(live, m, 64);
   }
   if (threadIdx.x == 0) {
-    g.start[unit] = v0;
-    g.start[g.units + unit] = v1;
-    g.start[2 * g.units + unit] = v2;
+    const int at = small_slot(unit);
+    g.start[at] = v0;
+    g.start[PD_SMALL_ROW + at] = v1;
+    g.start[2 * PD_SMALL_ROW + at] = v2;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) g.part[k * g.units + unit] = unset();
+    for (int k = 0; k < 6; ++k) g.part[k * PD_SMALL_ROW + at] = unset();
     if (broken) atomicAdd(&a.counters->broken, broken);
     if (live) atomicAdd(&a.counters->live, live);
     if (unit == 0) *g.aborted = 0u;
@@ -499,36 +571,49 @@ __global__ __launch_bounds__(kThreads) void k_small_assemble(AsmArgs a, SmallArg
 }
 
 // ---------------------------------------------------------------------------
-// The CG solve of a step in one launch, every workgroup resident: CUSP's loop as the general kernels run it (k_cg_spmv,
-// k_cg_update, k_cg_beta, k_cg_dir), the same sums in the same order.
+// The CG solve of a step in one launch, every workgroup resident: CUSP's
+// loop as the general kernels run it (k_cg_spmv, k_cg_update, k_cg_beta,
+// k_cg_dir), the same sums in the same order.
 //
-// An iteration: every lane gathers z and the previous direction of its
-// slots' neighbours, forms p = z + beta p, multiplies its blocks and leaves
-// the terms in LDS; lanes 0..2 of a row add them in list order on top of
-// the diagonal term.  The first R threads then own a row each: <y, p>, and
+// An iteration: the workgroup forms p = z + beta p of its rows' neighbours
+// in LDS, every lane multiplies its blocks by it and leaves the terms in
+// LDS, and the first wave adds them in list order on top of the diagonal
+// terms.  Its first R lanes then own a row each: <y, p>, and
 // once every unit's partial is there alpha, x, r, z; once <r, z> and <r, r>
 // are there, beta and the monitor test.  A unit's partial doubles as its
 // arrival: partials are awaited until they are set, and those of the
 // phase before are unset again once the next phase's are complete (all
-// units have read them by then).  z and p go through global memory with an
-// agent release ahead of the partial and an agent acquire after the wait,
-// by one wave per workgroup (by all eight, the cache maintenance alone took
-// 30 to 60 us per round; by one it is not seen).
+// units have read them by then).  z and p go through global memory, by
+// agent-scope stores that are awaited ahead of the partial and an agent
+// acquire after the wait, by one wave per workgroup (fences in all eight
+// took 30 to 60 us per round; in one they are not seen).
 //
 // Every wait ends: after g.spin_ticks of the 100 MHz clock a workgroup
 // raises *g.aborted and leaves.  The position update behind it then does
 // nothing, and the host puts the start values back (the assembly record
 // holds them) and solves with the general kernels.
 // ---------------------------------------------------------------------------
-template <int L, int M, int MC>
+// M slots per lane, the blocks of the first MR in registers and of the rest
+// in LDS; MC slots per chunk.
+template <int L, int M, int MR, int MC>
 __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g) {
   constexpr int R = Unit<L>::R, K = Unit<L>::K;
   constexpr int CH = MC * L, CP = CH + 3;  // slots per chunk, padded stride
-  __shared__ double T[R * 3 * CP];         // terms
-  __shared__ double Y[R * 3];
-  __shared__ double Mi[6 * R];  // the rows' inverse blocks
+  __shared__ double T[R * 3 * CP];  // terms
+  __shared__ double Y[3 * R];
+  __shared__ double Di[6 * R];  // the rows' diagonal blocks
+  __shared__ int longest;
+  __shared__ int own_l[R];  // each row's p in V
+  // the owners' x and r wait in LDS where the blocks leave no registers
+  constexpr bool kStateLds = L == 8;
+  __shared__ double Sl[kStateLds ? 6 * R : 1];
+  __shared__ double Mi[6 * R];  // and their inverses
+  // the unit's neighbours: the rows its blocks touch and its own, ascending
+  constexpr int UC = small_union(L);
+  __shared__ unsigned short list[UC];
+  __shared__ double V[3 * UC];  // their p of this iteration
+  __shared__ dbl2v Bl[M > MR ? (M - MR) * 3 * kThreads : 1];
   __shared__ double ctl[2];     // beta, and whether the loop goes on
-  const int units = g.units;
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int s = unit >> K, cl = unit & ((1 << K) - 1);
   const int i = threadIdx.x / L, j = threadIdx.x % L;
@@ -543,9 +628,9 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
   if (unit == 0 && threadIdx.x == 0) *g.h_cnt = *g.counters;
   // a tile between specimens: its rows are invisible, nobody awaits its sums
   if ((s >> 2) >= t0 + nt) return;
-  // the slots' blocks (zero past the list's end, where nothing adds them)
+  // the slots' blocks (past the list's end anything: nothing adds them)
   int q[M];
-  double B[M][6];
+  double B[MR][6];
   {
     const int64_t base = a.A.slice_off[s];
     const int* __restrict__ cp = a.A.col + base * 64 + pl;
@@ -560,50 +645,118 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
       const int k = m * L + j;
       q[m] = k <= top ? ntl(cp + (int64_t)k * 64) : -1;
     }
+    // groups of GS slots: their loads go out together
+    constexpr int GS = 4;
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const int k = m * L + j;
+    for (int m0 = 0; m0 < M; m0 += GS) {
+      double l0[GS];
+      double4 xq[GS];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) B[m][c] = 0.0;
-      if (q[m] >= 0) {
-        const double l0 = ntl(lp + (int64_t)k * 64);
-        const double4 xq = a.A.pos[q[m]];
+      for (int u = 0; u < GS; ++u) {
+        if (m0 + u >= M) break;
+        const int m = m0 + u;
+        l0[u] = q[m] >= 0 ? ntl(lp + (int64_t)(m * L + j) * 64) : 1.0;
+        xq[u] = a.A.pos[q[m] >= 0 ? q[m] : pc];
+      }
+#pragma unroll
+      for (int u = 0; u < GS; ++u) {
+        if (m0 + u >= M) break;
+        const int m = m0 + u;
         double e0, e1, e2, dij, F00, F01, F02, F11, F12, F22;
         if (shared) {
-          bond_dir<true, true>(pos_p, xq, e0, e1, e2, dij);
-          bond_jac<true>(e0, e1, e2, dij, l0, cb, F00, F01, F02, F11, F12, F22);
+          bond_dir<true, true>(pos_p, xq[u], e0, e1, e2, dij);
+          bond_jac<true>(e0, e1, e2, dij, l0[u], cb, F00, F01, F02, F11, F12, F22);
         } else {
-          bond_dir(pos_p, xq, e0, e1, e2, dij);
-          bond_jac(e0, e1, e2, dij, l0, cb, F00, F01, F02, F11, F12, F22);
+          bond_dir(pos_p, xq[u], e0, e1, e2, dij);
+          bond_jac(e0, e1, e2, dij, l0[u], cb, F00, F01, F02, F11, F12, F22);
         }
-        B[m][0] = (F00 * -1.0) * dt2;
-        B[m][1] = (F01 * -1.0) * dt2;
-        B[m][2] = (F02 * -1.0) * dt2;
-        B[m][3] = (F11 * -1.0) * dt2;
-        B[m][4] = (F12 * -1.0) * dt2;
-        B[m][5] = (F22 * -1.0) * dt2;
-        if (a.vals)
-          store_block(a.vals, base + k, pl, B[m][0], B[m][1], B[m][2], B[m][3], B[m][4],
-                      B[m][5]);
-      } else {
-        q[m] = pc;  // a gather in bounds, its term unused
+        const double b0 = (F00 * -1.0) * dt2, b1 = (F01 * -1.0) * dt2, b2 = (F02 * -1.0) * dt2,
+                     b3 = (F11 * -1.0) * dt2, b4 = (F12 * -1.0) * dt2, b5 = (F22 * -1.0) * dt2;
+        if (m < MR) {
+          B[m < MR ? m : 0][0] = b0;
+          B[m < MR ? m : 0][1] = b1;
+          B[m < MR ? m : 0][2] = b2;
+          B[m < MR ? m : 0][3] = b3;
+          B[m < MR ? m : 0][4] = b4;
+          B[m < MR ? m : 0][5] = b5;
+        } else {
+          dbl2v* o = Bl + (m - MR) * 3 * kThreads + threadIdx.x;
+          o[0] = dbl2v{b0, b1};
+          o[kThreads] = dbl2v{b2, b3};
+          o[2 * kThreads] = dbl2v{b4, b5};
+        }
+        if (q[m] < 0)
+          q[m] = pc;  // past the list's end: a gather in bounds, its term unused
+        else if (a.vals)
+          store_block(a.vals, base + m * L + j, pl, b0, b1, b2, b3, b4, b5);
       }
     }
   }
-  // lanes 0..2 of a row: row j of the diagonal block
-  double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-  if (j < 3) {
-    const double* dg = a.A.diag + (int64_t)s * 384 + pl;
-    g0 = dg[j == 0 ? 0 : j == 1 ? 64 : 128];
-    g1 = dg[j == 0 ? 64 : j == 1 ? 192 : 256];
-    g2 = dg[j == 0 ? 128 : j == 1 ? 256 : 320];
+  // the union of the gathered rows as a bitmap, its ranks the local indices
+  int own_at, nlist;
+  unsigned int at2[(M + 1) / 2];  // slots' places in V, two to a word
+  static_assert(3 * small_union(L) <= 65536, "16-bit places");
+  {
+    unsigned int* bits = (unsigned int*)T;       // [kThreads]: 16,384 rows
+    unsigned int* rank = bits + kThreads;        // [kThreads] ones before the word
+    unsigned int* wsum = rank + kThreads;        // [kThreads / 64]
+    static_assert(sizeof(T) >= (2 * kThreads + kThreads / 64) * sizeof(unsigned int), "scratch");
+    static_assert(PD_SMALL_UNITS * 64 <= kThreads * 32, "a bit per row");
+    const int t = threadIdx.x, wl = t & 63;
+    const int pc = row ? p : 0;
+    bits[t] = 0u;
+    if (t == 0) longest = 0;
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < M; ++m) atomicOr(bits + (q[m] >> 5), 1u << (q[m] & 31));
+    if (j == 0) atomicOr(bits + (pc >> 5), 1u << (pc & 31));
+    __syncthreads();
+    const unsigned int mine = bits[t];
+    int incl = __popc(mine);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (wl >= d) incl += v;
+    }
+    if (wl == 63) wsum[t >> 6] = incl;
+    __syncthreads();
+    int before = 0;
+    nlist = 0;
+#pragma unroll
+    for (int k = 0; k < kThreads / 64; ++k) {
+      if (k < (t >> 6)) before += wsum[k];
+      nlist += wsum[k];
+    }
+    const int ex0 = before + incl - __popc(mine);
+    rank[t] = ex0;
+    unsigned int left = mine;
+    for (int k = ex0; left; ++k) {
+      if (k < UC) list[k] = (unsigned short)(t * 32 + __ffs((int)left) - 1);
+      left &= left - 1;
+    }
+    __syncthreads();
+    auto local = [&](int r) {
+      return 3 * (int)(rank[r >> 5] + __popc(bits[r >> 5] & ((1u << (r & 31)) - 1u)));
+    };
+#pragma unroll
+    for (int m = 0; m < M; m += 2) {
+      unsigned int h = (unsigned int)local(q[m]);
+      if (m + 1 < M) h |= (unsigned int)local(q[m + 1]) << 16;
+      at2[m / 2] = h;
+    }
+    own_at = local(pc);
+    __syncthreads();
+  }
+  nlist = min(nlist, UC);  // the host found that no unit has more (k_small_union)
+  if (j == 0) {
+    own_l[i] = own_at;
+    atomicMax(&longest, top + 1);
   }
   // the first R threads own a row each
   const int ol = (threadIdx.x << K) + cl;
   const int op = s * 64 + ol;
   const bool own = threadIdx.x < R && op < a.A.n;
   double x0 = 0.0, x1 = 0.0, x2 = 0.0, r0 = 0.0, r1 = 0.0, r2 = 0.0;
-  double z0 = 0.0, z1 = 0.0, z2 = 0.0, p0 = 0.0, p1 = 0.0, p2 = 0.0;
   bool fr = false;
   if (own) {
     const double4 xx = a.x[op], rr = a.r[op];
@@ -613,17 +766,28 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
     r0 = rr.x;
     r1 = rr.y;
     r2 = rr.z;
-    const double* e = g.ex + 6 * (int64_t)op;
-    z0 = e[0];
-    z1 = e[1];
-    z2 = e[2];
     fr = a.bc[op] == 0;
-    if (a.precond) {
-      const double* m = a.minv + (int64_t)s * 384 + ol;
+    const int64_t blk = (int64_t)s * 384 + ol;
 #pragma unroll
-      for (int c = 0; c < 6; ++c) Mi[c * R + threadIdx.x] = m[c * 64];
+    for (int c = 0; c < 6; ++c) {
+      Di[c * R + threadIdx.x] = a.A.diag[blk + c * 64];
+      if (a.precond) Mi[c * R + threadIdx.x] = a.minv[blk + c * 64];
     }
   }
+  auto state = [&](bool load) {
+    if constexpr (kStateLds) {
+      double* o = Sl + threadIdx.x;
+      double* v[6] = {&x0, &x1, &x2, &r0, &r1, &r2};
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        if (load)
+          *v[k] = o[k * R];
+        else
+          o[k * R] = *v[k];
+      }
+    }
+  };
+  if (own) state(false);
   const int lane = threadIdx.x & 63;
   const bool lead = threadIdx.x < 64;  // the wave of the owners
   bool late = false;
@@ -632,9 +796,11 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
   int iter = 0;
   bool done = false, conv = false;
   if (lead) {
-    rz = fold_units<K, false>(g.start, t0, nt, g.nslices, lane, 0, &late);
-    rr = fold_units<K, false>(g.start + units, t0, nt, g.nslices, lane, 0, &late);
-    const double bb = fold_units<K, false>(g.start + 2 * units, t0, nt, g.nslices, lane, 0, &late);
+    double v[3];
+    fold_units<K, 3, false>(g.start, PD_SMALL_ROW, t0, nt, g.nslices, lane, 0, nullptr, &late, v);
+    rz = v[0];
+    rr = v[1];
+    const double bb = v[2];
     bnorm = sqrt(bb);
     tol = g.rtol * bnorm;
     rnorm = sqrt(rr);
@@ -651,92 +817,103 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
   }
   __syncthreads();
   const int64_t exn = 6 * (int64_t)a.A.n;
+  const int most = __builtin_amdgcn_readfirstlane(longest);  // slots in use
+  const int chain_c = threadIdx.x / R, chain_row = threadIdx.x % R;
+  const int at = small_slot(unit);
+  constexpr int PR = PD_SMALL_ROW;
   double* P_yp = g.part;
-  double* P_rz = g.part + 2 * units;
-  double* P_rr = g.part + 4 * units;
+  double* P_rz = g.part + 2 * PR;  // and <r, r> two rows on
   for (int it = 0; ctl[1] != 0.0; ++it) {
     const double bt = ctl[0];
     const double* ex = g.ex + (it & 1 ? exn : 0);
-    double acc = 0.0;
-    if (j < 3 && row) {
-      const double* e = ex + 6 * (int64_t)p;
-      double v0 = e[0], v1 = e[1], v2 = e[2];
+    // p = z + beta p of the neighbours (z in the first iteration), once each
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nlist; k += kThreads) {
+      const dbl2v* e = (const dbl2v*)(ex + 6 * (int64_t)list[k]);
+      const dbl2v ea = e[0], eb = e[1], ec = e[2];
+      double v0 = ea.x, v1 = ea.y, v2 = eb.x;
       if (it > 0) {
-        v0 = v0 + bt * e[3];
-        v1 = v1 + bt * e[4];
-        v2 = v2 + bt * e[5];
+        v0 = v0 + bt * eb.y;
+        v1 = v1 + bt * ec.x;
+        v2 = v2 + bt * ec.y;
       }
-      acc = g0 * v0 + g1 * v1 + g2 * v2;
+      V[3 * k] = v0;
+      V[3 * k + 1] = v1;
+      V[3 * k + 2] = v2;
+    }
+    __syncthreads();
+    double acc = 0.0;
+    if (threadIdx.x < 3 * R) {  // the diagonal term comes first
+      const double* v = V + own_l[chain_row];
+      const double* d = Di + chain_row;
+      acc = d[chain_c * R] * v[0] + d[(chain_c == 0 ? 1 : chain_c + 2) * R] * v[1] +
+            d[(chain_c == 0 ? 2 : chain_c + 3) * R] * v[2];
     }
 #pragma unroll
     for (int m0 = 0; m0 < M; m0 += MC) {
 #pragma unroll
       for (int m = m0; m < m0 + MC; ++m) {
-        if (m >= M) break;
-        const dbl2v* e = (const dbl2v*)(ex + 6 * (int64_t)q[m]);
-        const dbl2v ea = e[0], eb = e[1], ec = e[2];
-        double v0 = ea.x, v1 = ea.y, v2 = eb.x;
-        if (it > 0) {
-          v0 = v0 + bt * eb.y;
-          v1 = v1 + bt * ec.x;
-          v2 = v2 + bt * ec.y;
+        if (m >= M) {  // the last chunk's slots that no list reaches
+          double* o = T + i * 3 * CP + (m - m0) * L + j;
+          o[0] = -0.0;
+          o[CP] = -0.0;
+          o[2 * CP] = -0.0;
+          continue;
         }
         double u0, u1, u2;
-        blk6(B[m][0], B[m][1], B[m][2], B[m][3], B[m][4], B[m][5],
-             make_double4(v0, v1, v2, 0.0), u0, u1, u2);
-        double* o = T + i * 3 * CP + (m - m0) * L + j;
-        o[0] = u0;
-        o[CP] = u1;
-        o[2 * CP] = u2;
-      }
-      wave_fence();
-      if (j < 3) {
-        const double* t = T + (i * 3 + j) * CP;
-        const int cnt = min(CH, top + 1 - m0 * L);
-        int e = 0;
-        for (; e + 8 <= cnt; e += 8) {
-          double h[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) h[u] = t[e + u];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) acc += h[u];
+        const double* v = V + (m & 1 ? at2[m / 2] >> 16 : at2[m / 2] & 0xffffu);
+        const double4 v4 = make_double4(v[0], v[1], v[2], 0.0);
+        if (m < MR) {
+          const double* k = B[m < MR ? m : 0];
+          blk6(k[0], k[1], k[2], k[3], k[4], k[5], v4, u0, u1, u2);
+        } else {
+          const dbl2v* k = Bl + (m - MR) * 3 * kThreads + threadIdx.x;
+          const dbl2v ka = k[0], kb = k[kThreads], kc = k[2 * kThreads];
+          blk6(ka.x, ka.y, kb.x, kb.y, kc.x, kc.y, v4, u0, u1, u2);
         }
-        for (; e < cnt; ++e) acc += t[e];
+        const bool in = m * L + j <= top;
+        double* o = T + i * 3 * CP + (m - m0) * L + j;
+        o[0] = in ? u0 : -0.0;
+        o[CP] = in ? u1 : -0.0;
+        o[2 * CP] = in ? u2 : -0.0;
       }
-      wave_fence();
+      __syncthreads();
+      if (threadIdx.x < 3 * R) {  // a lane per row and component
+        const int n = most - m0 * L;
+        if (n > 0) acc = chain_wide<CH>(acc, T + (chain_row * 3 + chain_c) * CP, n);
+      }
+      if (m0 + MC < M) __syncthreads();
     }
-    if (j < 3) Y[i * 3 + j] = acc;
+    if (threadIdx.x < 3 * R) Y[threadIdx.x] = acc;
     __syncthreads();
     if (lead) {
       const int b = it & 1;
-      double t_yp = 0.0, y0 = 0.0, y1 = 0.0, y2 = 0.0;
+      double t_yp = 0.0, y0 = 0.0, y1 = 0.0, y2 = 0.0, p0 = 0.0, p1 = 0.0, p2 = 0.0;
       if (own) {
-        y0 = Y[threadIdx.x * 3];
-        y1 = Y[threadIdx.x * 3 + 1];
-        y2 = Y[threadIdx.x * 3 + 2];
-        if (it > 0) {
-          p0 = z0 + bt * p0;
-          p1 = z1 + bt * p1;
-          p2 = z2 + bt * p2;
-        } else {
-          p0 = z0;
-          p1 = z1;
-          p2 = z2;
-        }
+        y0 = Y[threadIdx.x];
+        y1 = Y[R + threadIdx.x];
+        y2 = Y[2 * R + threadIdx.x];
+        const double* v = V + own_l[threadIdx.x];
+        p0 = v[0];
+        p1 = v[1];
+        p2 = v[2];
         t_yp = (y0 * p0 + y1 * p1) + y2 * p2;
       }
       const double vy = unit_sum<R>(t_yp);
-      if (lane == 0) put(P_yp + b * units + unit, vy);
-      if (own) {  // the direction the next iteration gathers
-        double* e = g.ex + (b ? 0 : exn) + 6 * (int64_t)op;
-        e[3] = p0;
-        e[4] = p1;
-        e[5] = p2;
+      if (lane == 0) put(P_yp + b * PR + at, vy);
+      // the record that the next iteration gathers
+      double* e = g.ex + (b ? 0 : exn) + 6 * (int64_t)op;
+      if (own) {
+        put(e + 3, p0);
+        put(e + 4, p1);
+        put(e + 5, p2);
       }
-      yp = fold_units<K, true>(P_yp + b * units, t0, nt, g.nslices, lane, until, &late);
+      fold_units<K, 1, true>(P_yp + b * PR, 0, t0, nt, g.nslices, lane, until, g.aborted,
+                             &late, &yp);
       alpha = rz / yp;
       double t_rz = 0.0, t_rr = 0.0;
       if (own) {
+        state(true);
         x0 = alpha * p0 + x0;
         x1 = alpha * p1 + x1;
         x2 = alpha * p2 + x2;
@@ -746,9 +923,7 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
           r1 = na * y1 + r1;
           r2 = na * y2 + r2;
         }
-        z0 = r0;
-        z1 = r1;
-        z2 = r2;
+        double z0 = r0, z1 = r1, z2 = r2;
         if (a.precond) {
           const double* m = Mi + threadIdx.x;
           const double m00 = m[0], m01 = m[R], m02 = m[2 * R], m11 = m[3 * R], m12 = m[4 * R],
@@ -757,29 +932,31 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
           z1 = m01 * r0 + m11 * r1 + m12 * r2;
           z2 = m02 * r0 + m12 * r1 + m22 * r2;
         }
-        double* e = g.ex + (b ? 0 : exn) + 6 * (int64_t)op;
-        e[0] = z0;
-        e[1] = z1;
-        e[2] = z2;
+        put(e, z0);
+        put(e + 1, z1);
+        put(e + 2, z2);
         t_rz = (r0 * z0 + r1 * z1) + r2 * z2;
         t_rr = (r0 * r0 + r1 * r1) + r2 * r2;
+        state(false);
       }
       const double vz = unit_sum<R>(t_rz), vr = unit_sum<R>(t_rr);
       if (lane == 0 && it > 0) {  // all units have read the previous <r, z>
-        put(P_rz + (b ^ 1) * units + unit, unset());
-        put(P_rr + (b ^ 1) * units + unit, unset());
+        put(P_rz + (b ^ 1) * PR + at, unset());
+        put(P_rz + (2 + (b ^ 1)) * PR + at, unset());
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      stores_done();
       if (lane == 0) {
-        put(P_rz + b * units + unit, vz);
-        put(P_rr + b * units + unit, vr);
+        put(P_rz + b * PR + at, vz);
+        put(P_rz + (2 + b) * PR + at, vr);
       }
-      const double nrz =
-          fold_units<K, true>(P_rz + b * units, t0, nt, g.nslices, lane, until, &late);
-      rr = fold_units<K, true>(P_rr + b * units, t0, nt, g.nslices, lane, until, &late);
+      double sums[2];
+      fold_units<K, 2, true>(P_rz + b * PR, 2 * PR, t0, nt, g.nslices, lane, until,
+                             g.aborted, &late, sums);
+      const double nrz = sums[0];
+      rr = sums[1];
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       // all units have read this iteration's <y, p>
-      if (lane == 0) put(P_yp + b * units + unit, unset());
+      if (lane == 0) put(P_yp + b * PR + at, unset());
       beta = nrz / rz;
       rz = nrz;
       ++iter;
@@ -806,6 +983,7 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
     return;
   }
   if (own) {
+    state(true);
     a.x[op] = make_double4(x0, x1, x2, 0.0);
   }
   if (threadIdx.x == 0 && s == 4 * t0 && cl == 0) {  // the specimen's first unit
@@ -825,6 +1003,40 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
     st->max_iter = g.max_iter;
     st->upd_it = iter - 1;
   }
+}
+
+// The longest of the units' neighbour lists, over all the slots a list may
+// hold (its capacity): with 8 lanes per row it may exceed what LDS holds.
+template <int L>
+__global__ __launch_bounds__(kThreads) void k_small_union(int n, const int64_t* slice_off,
+                                                          const int32_t* cap, const int32_t* col,
+                                                          int* longest) {
+  constexpr int K = Unit<L>::K;
+  __shared__ unsigned int bits[kThreads];
+  __shared__ int total;
+  const int unit = blockIdx.x, s = unit >> K;
+  const int pl = ((threadIdx.x / L) << K) + (unit & ((1 << K) - 1)), p = s * 64 + pl;
+  bits[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) total = 0;
+  __syncthreads();
+  if (p < n) {
+    const int* c = col + slice_off[s] * 64 + pl;
+    for (int k = threadIdx.x % L; k < cap[p]; k += L) {
+      const int q = c[(int64_t)k * 64];
+      atomicOr(bits + (q >> 5), 1u << (q & 31));
+    }
+    atomicOr(bits + (p >> 5), 1u << (p & 31));
+  }
+  __syncthreads();
+  atomicAdd(&total, __popc(bits[threadIdx.x]));
+  __syncthreads();
+  if (threadIdx.x == 0) atomicMax(longest, total + 1);  // row 0 stands in for absent ones
+}
+
+void launch_small_union(int32_t n, int32_t nslices, const int64_t* slice_off, const int32_t* cap,
+                        const int32_t* col, int* longest, hipStream_t s) {
+  hipLaunchKernelGGL(k_small_union<8>, dim3(nslices), dim3(kThreads), 0, s, n, slice_off, cap,
+                     col, longest);
 }
 
 // the solve's start values back into x, after a solve that gave up
@@ -849,10 +1061,12 @@ void launch_small_assemble(int lanes, const AsmArgs& a, const SmallArgs& g, hipS
   }
 }
 
-// blocks per lane (L * M >= PD_SMALL_MAX_BONDS) and slots per chunk
-#define SOLVE8 k_small_solve<8, 15, 3>
-#define SOLVE16 k_small_solve<16, 8, 8>
-#define SOLVE32 k_small_solve<32, 4, 4>
+// slots per lane (L * M >= PD_SMALL_MAX_BONDS), those in registers, slots
+// per chunk (its gathers are in flight together).  More than eleven slots in
+// registers spill beside a chunk's gathers, so four go to LDS.
+#define SOLVE8 k_small_solve<8, 15, 13, 4>
+#define SOLVE16 k_small_solve<16, 8, 8, 4>
+#define SOLVE32 k_small_solve<32, 4, 4, 4>
 static_assert(8 * 15 >= PD_SMALL_MAX_BONDS && 16 * 8 >= PD_SMALL_MAX_BONDS &&
                   32 * 4 >= PD_SMALL_MAX_BONDS,
               "a row's blocks fit its lanes");
