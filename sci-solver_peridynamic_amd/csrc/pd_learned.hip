@@ -640,20 +640,48 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
   if (l == 0) part[PC_NWEIGHT] = ls;
 }
 
-// fold the per-wave gradients in wave order, Adam, bf16 refresh; thread i
-// owns weight i
+// Fold the per-wave gradients in wave order, Adam, bf16 refresh; the last
+// column of the partials is the loss.  A workgroup takes 32 columns: its
+// 256 threads bring 256 waves' rows of them to LDS, 32 independent loads
+// each, and a thread per column adds them in order.  (A thread per column
+// reading its 256 rows one after another took 102 us per step at 256 waves,
+// the latency of the loads; this takes 7.)
+#define ADAM_COLS 32
 __global__ __launch_bounds__(PD_BLOCK) void k_pc_adam(const float* partial, int nwaves, float* p,
                                                      float* m, float* v, __bf16* w, int step,
                                                      float lr, float* loss_out) {
-  const int i = blockIdx.x * PD_BLOCK + threadIdx.x;
-  if (i == 0 && loss_out) {
-    float s = 0.0f;
-    for (int k = 0; k < nwaves; ++k) s += partial[(int64_t)k * (PC_NWEIGHT + 1) + PC_NWEIGHT];
-    loss_out[0] = s;
-  }
-  if (i >= PC_NWEIGHT) return;
+  __shared__ float rows[PD_BLOCK][ADAM_COLS + 1];
+  constexpr int STEP = PD_BLOCK / ADAM_COLS;  // rows per pass
+  const int c = threadIdx.x % ADAM_COLS, r0 = threadIdx.x / ADAM_COLS;
+  const int i = blockIdx.x * ADAM_COLS + c;
   float gsum = 0.0f;
-  for (int k = 0; k < nwaves; ++k) gsum += partial[(int64_t)k * (PC_NWEIGHT + 1) + i];
+  for (int k0 = 0; k0 < nwaves; k0 += PD_BLOCK) {
+    float t[ADAM_COLS];
+#pragma unroll
+    for (int u = 0; u < ADAM_COLS; ++u) {
+      const int k = k0 + r0 + STEP * u;
+      t[u] = k < nwaves && i <= PC_NWEIGHT ? partial[(int64_t)k * (PC_NWEIGHT + 1) + i] : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < ADAM_COLS; ++u) rows[r0 + STEP * u][c] = t[u];
+    __syncthreads();
+    if (r0 == 0) {
+      const int n = min(PD_BLOCK, nwaves - k0);
+      int k = 0;
+      for (; k + 16 <= n; k += 16) {
+        float h[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) h[u] = rows[k + u][c];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) gsum += h[u];
+      }
+      for (; k < n; ++k) gsum += rows[k][c];
+    }
+    __syncthreads();
+  }
+  if (r0 != 0) return;
+  if (i == PC_NWEIGHT && loss_out) loss_out[0] = gsum;
+  if (i >= PC_NWEIGHT) return;
   const float b1 = 0.9f, b2 = 0.999f;
   const float mi = b1 * m[i] + (1.0f - b1) * gsum;
   const float vi = b2 * v[i] + (1.0f - b2) * gsum * gsum;
@@ -672,32 +700,31 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_to_bf16(const float* p, __bf16*
   if (i < PC_NWEIGHT) w[i] = (__bf16)p[i];
 }
 
-// one workgroup: feature means and inverse standard deviations
+// feature means and inverse standard deviations, a workgroup per feature
 __global__ __launch_bounds__(PD_BLOCK) void k_pc_norm(const float* samples, int64_t ns, float* p) {
   __shared__ double sm[PD_BLOCK], sq[PD_BLOCK];
-  for (int k = 0; k < PC_NIN; ++k) {
-    double s = 0.0, q = 0.0;
-    for (int64_t i = threadIdx.x; i < ns; i += PD_BLOCK) {
-      const double f = samples[i * PC_SAMPLE + k];
-      s += f;
-      q += f * f;
+  const int k = blockIdx.x;
+  double s = 0.0, q = 0.0;
+#pragma unroll 8
+  for (int64_t i = threadIdx.x; i < ns; i += PD_BLOCK) {
+    const double f = samples[i * PC_SAMPLE + k];
+    s += f;
+    q += f * f;
+  }
+  sm[threadIdx.x] = s;
+  sq[threadIdx.x] = q;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double S = 0.0, Q = 0.0;
+    for (int t = 0; t < PD_BLOCK; ++t) {
+      S += sm[t];
+      Q += sq[t];
     }
-    sm[threadIdx.x] = s;
-    sq[threadIdx.x] = q;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      double S = 0.0, Q = 0.0;
-      for (int t = 0; t < PD_BLOCK; ++t) {
-        S += sm[t];
-        Q += sq[t];
-      }
-      const double mean = ns > 0 ? S / (double)ns : 0.0;
-      const double var = ns > 0 ? Q / (double)ns - mean * mean : 0.0;
-      const double sd = var > 0.0 ? sqrt(var) : 0.0;
-      p[PC_OFF_MEAN + k] = (float)mean;
-      p[PC_OFF_ISTD + k] = sd > 1e-6 ? (float)(1.0 / sd) : 0.0f;
-    }
-    __syncthreads();
+    const double mean = ns > 0 ? S / (double)ns : 0.0;
+    const double var = ns > 0 ? Q / (double)ns - mean * mean : 0.0;
+    const double sd = var > 0.0 ? sqrt(var) : 0.0;
+    p[PC_OFF_MEAN + k] = (float)mean;
+    p[PC_OFF_ISTD + k] = sd > 1e-6 ? (float)(1.0 / sd) : 0.0f;
   }
 }
 
@@ -731,14 +758,14 @@ void launch_pc_train(const PcTrainArgs& a, hipStream_t s) {
 }
 void launch_pc_adam(const float* partial, int32_t nwaves, float* p, float* m, float* v, __bf16* w,
                     int32_t step, float lr, float* loss_out, hipStream_t s) {
-  hipLaunchKernelGGL(k_pc_adam, dim3(blocks_of(PC_NWEIGHT)), dim3(PD_BLOCK), 0, s, partial, nwaves,
-                     p, m, v, w, step, lr, loss_out);
+  hipLaunchKernelGGL(k_pc_adam, dim3((PC_NWEIGHT + 1 + ADAM_COLS - 1) / ADAM_COLS),
+                     dim3(PD_BLOCK), 0, s, partial, nwaves, p, m, v, w, step, lr, loss_out);
 }
 void launch_pc_to_bf16(const float* p, __bf16* w, hipStream_t s) {
   hipLaunchKernelGGL(k_pc_to_bf16, dim3(blocks_of(PC_NWEIGHT)), dim3(PD_BLOCK), 0, s, p, w);
 }
 void launch_pc_norm(const float* samples, int64_t nsamples, float* p, hipStream_t s) {
-  hipLaunchKernelGGL(k_pc_norm, dim3(1), dim3(PD_BLOCK), 0, s, samples, nsamples, p);
+  hipLaunchKernelGGL(k_pc_norm, dim3(PC_NIN), dim3(PD_BLOCK), 0, s, samples, nsamples, p);
 }
 
 }  // namespace pd
