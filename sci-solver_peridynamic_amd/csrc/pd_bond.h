@@ -26,24 +26,31 @@ typedef double vpair __attribute__((ext_vector_type(2)));
 // two Newton steps y += y (1 - bs y); q = as y; the Markstein correction
 // fma(as - bs q, y, q) (div_fmas); div_fixup for special operands and the
 // sign.  When no operand needs scaling (div_scale leaves both unchanged and
-// div_fmas applies no 2^64 factor) and no special case applies, that is
-// exactly rcp_nr(b) then div_rcp(a, b, y) below, so quotients by one
-// denominator can share y.  No scaling happens when b and 1/b are normal,
-// a is 0 or |a| >= 2^-969, a / b is normal and exponent(a) - exponent(b) <
-// 768.  Every denominator here is positive: then a = +0 gives +0 as IEEE
-// division does, but a = -0 would give +0 where it gives -0, so no caller
-// passes -0 (a coordinate difference is -0 only for a -0 coordinate less a
-// +0 one, and the range flag admits no -0 coordinate; the other numerators
-// are positive or a difference horizon - d0 with a positive horizon, which
-// is never -0).  range_ok_* state sufficient ranges; callers take this path
-// only when the assembly found every operand inside them.
+// div_fmas applies no 2^64 factor) and no special case applies, the quotient
+// is fma(a - b q, y, q) with q = a y for a y within half an ulp of 1 / b and
+// an excess of 2^-16 ulp, so quotients by one denominator can share y, which
+// may come from any such refinement.  No scaling happens when b and
+// 1/b are normal, a is 0 or |a| >= 2^-969, a / b is normal and exponent(a) -
+// exponent(b) < 768.  (Two refinements can only give different quotients for
+// a / b within 1.5 2^-53 ulp of a rounding boundary, a few numerators in 2^52
+// for each b, and only where the two y differ, 2^-16 of all b or fewer.)
+// Every denominator here is positive: then a = +0 gives
+// +0 as IEEE division does, but a = -0 would give +0 where it gives -0, so no
+// caller passes -0 (a coordinate difference is -0 only for a -0 coordinate
+// less a +0 one, and the range flag admits no -0 coordinate; the other
+// numerators are positive or a difference horizon - d0 with a positive
+// horizon, which is never -0).  range_ok_* state sufficient ranges; callers
+// take this path only when the assembly found every operand inside them.
+//
+// 1 / b from an estimate y0 of relative error t = 1 - b y0 (rcp: 2^-23):
+// y0 (1 + t + t^2), whose remaining error t^3 is below 2^-68, in three
+// operations where two Newton steps take four.
+__device__ __forceinline__ double rcp_from(double b, double y0) {
+  const double t = __builtin_fma(-b, y0, 1.0);
+  return __builtin_fma(y0, __builtin_fma(t, t, t), y0);
+}
 __device__ __forceinline__ double rcp_nr(double b) {
-  double y = __builtin_amdgcn_rcp(b);
-  double t = __builtin_fma(-b, y, 1.0);
-  y = __builtin_fma(y, t, y);
-  t = __builtin_fma(-b, y, 1.0);
-  y = __builtin_fma(y, t, y);
-  return y;
+  return rcp_from(b, __builtin_amdgcn_rcp(b));
 }
 __device__ __forceinline__ double div_rcp(double a, double b, double y) {
   const double q = a * y;
@@ -56,7 +63,9 @@ __device__ __forceinline__ double div_rcp(double a, double b, double y) {
 // together by one coupled Newton step, then two Markstein corrections
 // s += (x - s^2) h.  The same operations in the same order, so the same
 // bits.  x = 0 gives NaN: callers exclude it.
-__device__ __forceinline__ double sqrt_nr(double x) {
+// yi: 1 / s on the way, from 2 h (relative error below 2^-44) by one Newton
+// step: no second reciprocal instruction (16 cycles against 4).
+__device__ __forceinline__ double sqrt_rcp(double x, double& yi) {
   const double g = __builtin_amdgcn_rsq(x);
   double s = x * g;
   double h = g * 0.5;
@@ -66,7 +75,10 @@ __device__ __forceinline__ double sqrt_nr(double x) {
   double d = __builtin_fma(-s, s, x);
   s = __builtin_fma(d, h, s);
   d = __builtin_fma(-s, s, x);
-  return __builtin_fma(d, h, s);
+  s = __builtin_fma(d, h, s);
+  const double y = h + h;
+  yi = __builtin_fma(y, __builtin_fma(-s, y, 1.0), y);
+  return s;
 }
 
 // A coordinate +0 or of magnitude in [2^-300, 2^100]: a difference of two
@@ -74,7 +86,7 @@ __device__ __forceinline__ double sqrt_nr(double x) {
 //  * it divided by the bond length fd = max(|d|, 1e-10) (at most 2^102, a
 //    float) needs no scaling;
 //  * the squared length of a bond is 0 or in [2^-704, 2^204], inside
-//    sqrt_nr's range when it is not 0, and the length dij is 0 or in
+//    sqrt_rcp's range when it is not 0, and the length dij is 0 or in
 //    [2^-352, 2^102].
 __device__ __forceinline__ bool range_ok_coord(double v) {
   const double m = fabs(v);
@@ -92,34 +104,44 @@ __device__ __forceinline__ bool range_ok_stiff(double c) {
   return c >= 0x1p-300 && c <= 0x1p300;
 }
 
+// Bond lengths up to this (cg_solver.cuh:256's floor, as a float) divide
+// by it instead of by themselves.
+__device__ __forceinline__ float small_len() { return (float)1.0e-10; }
+
 // Current geometry of bond (p, q), cg_solver.cuh:253-256: the unit vector e
 // (the difference divided by the float-rounded length max(|d|, SMALL)) and
 // the current length dij.  SHARED: the three quotients share one
-// reciprocal, and the square root is sqrt_nr, behind a test for a zero
-// length unless NONZERO (the caller knows every bond length is nonzero):
-// identical results inside the ranges above.
-template <bool SHARED = false, bool NONZERO = false>
+// reciprocal, refined from 1 / dij (yi; the rounded length is within 2^-24 of
+// dij), and the square root is sqrt_rcp, behind tests for a length up to
+// SMALL unless LONG (the caller knows every bond is longer): identical
+// results inside the ranges above.
+template <bool SHARED = false, bool LONG = false>
 __device__ __forceinline__ void bond_dir(const double4 pos_p, const double4 xq, double& e0,
-                                         double& e1, double& e2, double& dij) {
+                                         double& e1, double& e2, double& dij, double& yi) {
   e0 = xq.x - pos_p.x;
   e1 = xq.y - pos_p.y;
   e2 = xq.z - pos_p.z;
   const double ss = e0 * e0 + e1 * e1 + e2 * e2;
-  if constexpr (!SHARED)
-    dij = sqrt(ss);
-  else if constexpr (NONZERO)
-    dij = sqrt_nr(ss);
-  else
-    dij = ss == 0.0 ? 0.0 : sqrt_nr(ss);
-  const float dij_f = (float)dij;
-  const float small_f = (float)1.0e-10;
-  const double fd = (double)(dij_f > small_f ? dij_f : small_f);
   if constexpr (SHARED) {
-    const double y = rcp_nr(fd);
+    dij = sqrt_rcp(ss, yi);
+    if constexpr (!LONG) dij = ss == 0.0 ? 0.0 : dij;
+    float dij_f = (float)dij;
+    double y0 = yi;
+    if constexpr (!LONG) {
+      const bool s = !(dij_f > small_len());
+      dij_f = s ? small_len() : dij_f;
+      y0 = s ? 1.0 / (double)small_len() : y0;  // a constant
+    }
+    const double fd = (double)dij_f;
+    const double y = rcp_from(fd, y0);
     e0 = div_rcp(e0, fd, y);
     e1 = div_rcp(e1, fd, y);
     e2 = div_rcp(e2, fd, y);
   } else {
+    dij = sqrt(ss);
+    yi = 0.0;
+    const float dij_f = (float)dij;
+    const double fd = (double)(dij_f > small_len() ? dij_f : small_len());
     e0 /= fd;
     e1 /= fd;
     e2 /= fd;
@@ -134,35 +156,44 @@ __device__ __forceinline__ double ref_len(const double4 opos_p, const double4 oq
 
 // The bond's 3x3 Jacobian F (six distinct entries), cg_solver.cuh:292-299:
 // (c / d0) [(1 - d0/dij) I + (d0/dij) e e^T], with the factor sc = c / d0
-// given.  SHARED: d0 / dij through rcp_nr(dij) (identical inside the ranges
+// given.  SHARED: d0 / dij through yi = 1 / dij (identical inside the ranges
 // above for a nonzero dij; a zero dij makes every entry NaN either way).
-template <bool SHARED = false>
+// PLUS0: the off-diagonal entries' "0.0 +", which turns -0 into +0 and
+// changes nothing else: entries that are stored keep it, entries that only
+// go into a sum do without it.
+template <bool SHARED = false, bool PLUS0 = true>
 __device__ __forceinline__ void bond_jac_sc(double e0, double e1, double e2, double dij,
-                                            double d0, double sc, double& F00, double& F01,
-                                            double& F02, double& F11, double& F12,
+                                            double yi, double d0, double sc, double& F00,
+                                            double& F01, double& F02, double& F11, double& F12,
                                             double& F22) {
-  const double ratio = SHARED ? div_rcp(d0, dij, rcp_nr(dij)) : d0 / dij;
+  const double ratio = SHARED ? div_rcp(d0, dij, yi) : d0 / dij;
   const double dg = 1.0 - ratio;
+  double o01 = (e0 * e1) * ratio, o02 = (e0 * e2) * ratio, o12 = (e1 * e2) * ratio;
+  if constexpr (PLUS0) {
+    o01 = 0.0 + o01;
+    o02 = 0.0 + o02;
+    o12 = 0.0 + o12;
+  }
   F00 = (dg + (e0 * e0) * ratio) * sc;
-  F01 = (0.0 + (e0 * e1) * ratio) * sc;
-  F02 = (0.0 + (e0 * e2) * ratio) * sc;
+  F01 = o01 * sc;
+  F02 = o02 * sc;
   F11 = (dg + (e1 * e1) * ratio) * sc;
-  F12 = (0.0 + (e1 * e2) * ratio) * sc;
+  F12 = o12 * sc;
   F22 = (dg + (e2 * e2) * ratio) * sc;
 }
 
 // The same from c: SHARED forms c / d0 through rcp_nr (identical results
 // inside the ranges above).
-template <bool SHARED = false>
-__device__ __forceinline__ void bond_jac(double e0, double e1, double e2, double dij, double d0,
-                                         double c_bond, double& F00, double& F01, double& F02,
-                                         double& F11, double& F12, double& F22) {
+template <bool SHARED = false, bool PLUS0 = true>
+__device__ __forceinline__ void bond_jac(double e0, double e1, double e2, double dij, double yi,
+                                         double d0, double c_bond, double& F00, double& F01,
+                                         double& F02, double& F11, double& F12, double& F22) {
   double sc;
   if constexpr (SHARED)
     sc = div_rcp(c_bond, d0, rcp_nr(d0));
   else
     sc = c_bond / d0;
-  bond_jac_sc<SHARED>(e0, e1, e2, dij, d0, sc, F00, F01, F02, F11, F12, F22);
+  bond_jac_sc<SHARED, PLUS0>(e0, e1, e2, dij, yi, d0, sc, F00, F01, F02, F11, F12, F22);
 }
 
 __device__ __forceinline__ void blk6(double a00, double a01, double a02, double a11,
@@ -182,8 +213,8 @@ __device__ __forceinline__ void blk6(double a00, double a01, double a02, double 
 // arithmetic, not by HBM.  REC: the neighbour's position and x come from
 // A.rec (x must be the CG direction p the record holds): three 16-byte
 // loads instead of four.  SHARED: quotients share reciprocals and square
-// roots take sqrt_nr with no zero test (the assembly found every operand in
-// range and no live bond of zero length).
+// roots take sqrt_rcp with no length test (the assembly found every operand
+// in range and every live bond longer than SMALL).
 typedef double dbl2v __attribute__((ext_vector_type(2)));
 
 // One bond block into the pair planes of vals (the assembly's layout).
@@ -224,6 +255,7 @@ __device__ __forceinline__ void spmv_row_mf(const SpmvView& A, const double4* __
                                             int p, double& y0, double& y1, double& y2,
                                             const double* __restrict__ rec = nullptr,
                                             double* __restrict__ vals = nullptr) {
+  constexpr bool PLUS0 = STORE || !SHARED;
   const int s = p >> 6;
   const int lane = p & 63;
   const double* dg = A.diag + (int64_t)s * 6 * 64 + lane;
@@ -258,13 +290,18 @@ __device__ __forceinline__ void spmv_row_mf(const SpmvView& A, const double4* __
       double4 xq[V], vq[V];
 #pragma unroll
       for (int u = 0; u < V; ++u) gather_mf<REC>(A, rec, x, q[u], xq[u], vq[u]);
+      // all of the trip's loads before its arithmetic: left to itself the
+      // scheduler moves some of them behind the first bonds' chains to save
+      // registers, and their latency is paid in line (five slots at 10^6
+      // rows: 860 us against 480)
+      __builtin_amdgcn_sched_barrier(0);
       double t[V][3];
 #pragma unroll
       for (int u = 0; u < V; ++u) {
-        double e0, e1, e2, dij;
-        bond_dir<SHARED, SHARED>(pos_p, xq[u], e0, e1, e2, dij);
+        double e0, e1, e2, dij, yi;
+        bond_dir<SHARED, SHARED>(pos_p, xq[u], e0, e1, e2, dij, yi);
         double F00, F01, F02, F11, F12, F22;
-        bond_jac<SHARED>(e0, e1, e2, dij, l0[u], cb, F00, F01, F02, F11, F12, F22);
+        bond_jac<SHARED, PLUS0>(e0, e1, e2, dij, yi, l0[u], cb, F00, F01, F02, F11, F12, F22);
         const double b00 = (F00 * -1.0) * dt2, b01 = (F01 * -1.0) * dt2,
                      b02 = (F02 * -1.0) * dt2, b11 = (F11 * -1.0) * dt2,
                      b12 = (F12 * -1.0) * dt2, b22 = (F22 * -1.0) * dt2;
@@ -282,11 +319,11 @@ __device__ __forceinline__ void spmv_row_mf(const SpmvView& A, const double4* __
       const int q0 = ntl(cp + (int64_t)bnd * 64);
       double4 xq, vq;
       gather_mf<REC>(A, rec, x, q0, xq, vq);
-      double e0, e1, e2, dij;
-      bond_dir<SHARED, SHARED>(pos_p, xq, e0, e1, e2, dij);
+      double e0, e1, e2, dij, yi;
+      bond_dir<SHARED, SHARED>(pos_p, xq, e0, e1, e2, dij, yi);
       double F00, F01, F02, F11, F12, F22;
-      bond_jac<SHARED>(e0, e1, e2, dij, ntl(lp + (int64_t)bnd * 64), cb, F00, F01, F02, F11,
-                       F12, F22);
+      bond_jac<SHARED, PLUS0>(e0, e1, e2, dij, yi, ntl(lp + (int64_t)bnd * 64), cb, F00, F01,
+                              F02, F11, F12, F22);
       const double b00 = (F00 * -1.0) * dt2, b01 = (F01 * -1.0) * dt2, b02 = (F02 * -1.0) * dt2,
                    b11 = (F11 * -1.0) * dt2, b12 = (F12 * -1.0) * dt2, b22 = (F22 * -1.0) * dt2;
       if constexpr (STORE) store_block(vals, base + bnd, lane, b00, b01, b02, b11, b12, b22);

@@ -93,8 +93,8 @@ struct pd_step_counters {
   unsigned long long live;
   // bit 0: some position, reference length, bond stiffness, horizon or
   // radius lies outside the ranges of the shared-reciprocal quotients and
-  // of sqrt_nr (set ahead of the assembly); bit 1: a live bond has zero
-  // length (set by the assembly).  Nonzero: the matrix-free operator
+  // of sqrt_rcp (set ahead of the assembly); bit 1: a live bond is no longer
+  // than (float)1e-10 (set by the assembly).  Nonzero: the matrix-free operator
   // divides one quotient at a time and takes IEEE square roots.
   unsigned int range_bad;
   unsigned int pad;

@@ -174,10 +174,10 @@ __device__ __forceinline__ void row_f32(const MxArgs& A, const float4* __restric
 template <bool SHARED>
 __device__ __forceinline__ void bond_block32(const double4 pos_p, const double4 xq, double d0,
                                              double cb, double dt2, float v[6]) {
-  double e0, e1, e2, dij;
-  bond_dir<SHARED, SHARED>(pos_p, xq, e0, e1, e2, dij);
+  double e0, e1, e2, dij, yi;
+  bond_dir<SHARED, SHARED>(pos_p, xq, e0, e1, e2, dij, yi);
   double F00, F01, F02, F11, F12, F22;
-  bond_jac<SHARED>(e0, e1, e2, dij, d0, cb, F00, F01, F02, F11, F12, F22);
+  bond_jac<SHARED>(e0, e1, e2, dij, yi, d0, cb, F00, F01, F02, F11, F12, F22);
   v[0] = (float)((F00 * -1.0) * dt2);
   v[1] = (float)((F01 * -1.0) * dt2);
   v[2] = (float)((F02 * -1.0) * dt2);
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_mx_resid(MxArgs a) {
     if (!a.A64.rec)
       spmv_row_mf<3, true, false, false>(a.A64, a.x, p, y0, y1, y2);
     else if (*a.A64.range_bad == 0)  // uniform over the grid
-      spmv_row_mf<4, true, true, true>(a.A64, a.x, p, y0, y1, y2, a.A64.rec);
+      spmv_row_mf<5, true, true, true>(a.A64, a.x, p, y0, y1, y2, a.A64.rec);
     else
       spmv_row_mf<2, true, true, false>(a.A64, a.x, p, y0, y1, y2, a.A64.rec);
     const double4 bp = a.b[p];

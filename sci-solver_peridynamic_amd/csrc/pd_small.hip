@@ -236,7 +236,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
   double* __restrict__ len = a.d0 + base * 64 + pl;
   const double hr = mt.horizon - mt.radius;
   const double yr = SHARED ? rcp_nr(mt.radius) : 0.0;
-  bool zero_len = false;
+  bool short_len = false;
   double acc[NR];
 #pragma unroll
   for (int k = 0; k < NR; ++k) acc[k] = j + k * L == 14 ? -INFINITY : 0.0;
@@ -244,7 +244,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
   // geometry, stretch and breaking test of slot k (k <= top)
   struct Bond {
     double4 u;
-    double d0, e0, e1, e2, dij, yd, dr;
+    double d0, e0, e1, e2, dij, yi, yd, dr;
     bool brk;
   };
   auto measure = [&](int q, double d0, Bond& b) {
@@ -256,7 +256,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
     sq = r1.y;
     b.u = make_double4(r2.x, r2.y, r3.x, 0.0);
     b.d0 = d0;
-    bond_dir<SHARED>(pos_p, xq, b.e0, b.e1, b.e2, b.dij);
+    bond_dir<SHARED>(pos_p, xq, b.e0, b.e1, b.e2, b.dij, b.yi);
     b.yd = SHARED ? rcp_nr(d0) : 0.0;
     b.dr = (SHARED ? div_rcp(b.dij, d0, b.yd) : b.dij / d0) - 1.0;
     const float sq_f = (float)sq;
@@ -285,7 +285,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
       for (int u = 0; u < 2; ++u) {
         const bool in = c0 + u * L + j <= top;
         measure(q[u], l0[u], b[u]);
-        if (in && SHARED) zero_len = zero_len || b[u].dij == 0.0;
+        if (in && SHARED) short_len = short_len || !((float)b[u].dij > small_len());
         brk = brk || (in && b[u].brk);
       }
       const unsigned long long any = __ballot(brk);
@@ -300,7 +300,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
         if (in) {
           Bond t;
           measure(col[(int64_t)k * 64], len[(int64_t)k * 64], t);
-          if (SHARED) zero_len = zero_len || t.dij == 0.0;
+          if (SHARED) short_len = short_len || !((float)t.dij > small_len());
           bk = t.brk;
         }
         const unsigned long long bits =
@@ -380,7 +380,8 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
       const double kk = t.dr * vscale;
       double F00, F01, F02, F11, F12, F22;
       const double sc = SHARED ? div_rcp(mt.c_bond, t.d0, t.yd) : mt.c_bond / t.d0;
-      bond_jac_sc<SHARED>(t.e0, t.e1, t.e2, t.dij, t.d0, sc, F00, F01, F02, F11, F12, F22);
+      bond_jac_sc<SHARED, false>(t.e0, t.e1, t.e2, t.dij, t.yi, t.d0, sc, F00, F01, F02, F11,
+                                 F12, F22);
       const double b00 = (F00 * -1.0) * a.dt2, b01 = (F01 * -1.0) * a.dt2,
                    b02 = (F02 * -1.0) * a.dt2, b11 = (F11 * -1.0) * a.dt2,
                    b12 = (F12 * -1.0) * a.dt2, b22 = (F22 * -1.0) * a.dt2;
@@ -428,7 +429,7 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
     if (j + k * L < ROLES) sum[i * 16 + j + k * L] = acc[k];
   int* tops = (int*)(lds + R * 16);  // [R]
   if (j == 0) tops[i] = top;
-  const bool zany = __any(zero_len);
+  const bool zany = __any(short_len);
   if (SHARED && zany && (threadIdx.x & 63) == 0) atomicOr(&a.counters->range_bad, 2u);
   __syncthreads();
   if (threadIdx.x >= 64) return;
@@ -662,13 +663,13 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
       for (int u = 0; u < GS; ++u) {
         if (m0 + u >= M) break;
         const int m = m0 + u;
-        double e0, e1, e2, dij, F00, F01, F02, F11, F12, F22;
+        double e0, e1, e2, dij, yi, F00, F01, F02, F11, F12, F22;
         if (shared) {
-          bond_dir<true, true>(pos_p, xq[u], e0, e1, e2, dij);
-          bond_jac<true>(e0, e1, e2, dij, l0[u], cb, F00, F01, F02, F11, F12, F22);
+          bond_dir<true, true>(pos_p, xq[u], e0, e1, e2, dij, yi);
+          bond_jac<true>(e0, e1, e2, dij, yi, l0[u], cb, F00, F01, F02, F11, F12, F22);
         } else {
-          bond_dir(pos_p, xq[u], e0, e1, e2, dij);
-          bond_jac(e0, e1, e2, dij, l0[u], cb, F00, F01, F02, F11, F12, F22);
+          bond_dir(pos_p, xq[u], e0, e1, e2, dij, yi);
+          bond_jac(e0, e1, e2, dij, yi, l0[u], cb, F00, F01, F02, F11, F12, F22);
         }
         const double b0 = (F00 * -1.0) * dt2, b1 = (F01 * -1.0) * dt2, b2 = (F02 * -1.0) * dt2,
                      b3 = (F11 * -1.0) * dt2, b4 = (F12 * -1.0) * dt2, b5 = (F22 * -1.0) * dt2;

@@ -7,6 +7,8 @@
 // square root, and the two float roundings of cg_solver.cuh:256,264.
 #include <math.h>
 
+#include <type_traits>
+
 #include "pd_bond.h"
 
 namespace pd {
@@ -48,10 +50,10 @@ __device__ __forceinline__ void gather_asm(const AsmArgs& a, int q, double4& xq,
 // the quotients by the float-rounded length (bond_dir), by the reference
 // length (dij / d0, c / d0), by the current length (d0 / dij) and by the
 // radius (the volume scale) share reciprocals and the square root is
-// sqrt_nr; both variants are launched and the one that does not match bit 0
+// sqrt_rcp; both variants are launched and the one that does not match bit 0
 // of the range flag (k_asm_prep) returns at once.  The SHARED variant sets
-// bit 1 when a live bond has zero length (the matrix-free products then
-// leave the shared forms).
+// bit 1 when a live bond is no longer than SMALL (the matrix-free products
+// then leave the shared forms).
 // FUSE and GAP: a.fuse and a.track_gap as compile-time choices.
 template <bool MIXED, bool SHARED, bool FUSE, bool GAP>
 __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int p = tile * PD_BLOCK + threadIdx.x;
   unsigned long long broken = 0, live = 0;
-  bool zero_len = false;  // SHARED: a bond of zero current length
+  bool short_len = false;  // SHARED: a bond no longer than SMALL
   double t_rr = 0.0, t_rz = 0.0, t_r32 = 0.0, t_bb = 0.0;  // fused residual partials
   if (p < a.n && a.act[p] != PD_INVISIBLE) {
     const pd_mat_dev mt = a.mat[a.body[p]];
@@ -88,17 +90,20 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     const double yr = SHARED ? rcp_nr(mt.radius) : 0.0;  // 1 / radius for vscale
     // A bond's geometry, stretch and breaking threshold, cg_solver.cuh:253-264
     // (yd: SHARED, 1 / d0 for dij / d0 and c / d0); the bond breaks when
-    // drdivd > thr.
-    auto measure = [&](const double4& xq, double sqv, double d0, double& e0, double& e1,
-                       double& e2, double& dij, double& yd, double& drdivd, double& thr) {
-      bond_dir<SHARED>(pos_p, xq, e0, e1, e2, dij);
-      if constexpr (SHARED) zero_len = zero_len || dij == 0.0;
+    // drdivd > thr.  lg: the caller drops the result of a bond no longer than
+    // SMALL (of which it is told).
+    auto measure = [&](auto lg, const double4& xq, double sqv, double d0, double& e0,
+                       double& e1, double& e2, double& dij, double& yi, double& yd,
+                       double& drdivd, double& thr) {
+      bond_dir<SHARED, lg.value>(pos_p, xq, e0, e1, e2, dij, yi);
+      const bool is_short = SHARED && !((float)dij > small_len());
       yd = 0.0;
       if constexpr (SHARED) yd = rcp_nr(d0);
       drdivd = (SHARED ? div_rcp(dij, d0, yd) : dij / d0) - 1.0;
       // cg_solver.cuh:264: threshold (float)max(s_p, s_q)
       const float sq_f = (float)sqv;
       thr = (double)(stretch_f > sq_f ? stretch_f : sq_f);
+      return is_short;
     };
     // GAP: the bond nearest its threshold so far (the first one on ties)
     auto track_gap = [&](int q, double drdivd, double thr) {
@@ -113,7 +118,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     // A live bond's force, Jacobian, diagonal and residual terms,
     // cg_solver.cuh:277-319.
     auto accumulate = [&](const double4& u, double d0, double e0, double e1, double e2,
-                          double dij, double yd, double drdivd) {
+                          double dij, double yi, double yd, double drdivd) {
       double vscale = 1.0;
       if (d0 > hr)
         vscale = 0.5 + (SHARED ? div_rcp((mt.horizon - d0) / 2.0, mt.radius, yr)
@@ -127,7 +132,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
       f2 += kk * e2;
       double F00, F01, F02, F11, F12, F22;
       const double sc = SHARED ? div_rcp(mt.c_bond, d0, yd) : mt.c_bond / d0;
-      bond_jac_sc<SHARED>(e0, e1, e2, dij, d0, sc, F00, F01, F02, F11, F12, F22);
+      bond_jac_sc<SHARED, false>(e0, e1, e2, dij, yi, d0, sc, F00, F01, F02, F11, F12, F22);
       k00 += F00;
       k01 += F01;
       k02 += F02;
@@ -151,11 +156,15 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     // With shared reciprocals: first an optimistic pass over the list as
     // it stands, OPT slots per trip (independent chains for the
     // scheduler) and no swap-remove.  Breaking bonds are rare (tens per
-    // step among 10^8): a lane stops at the first trip that holds one and
+    // step among 10^8): a lane stops at the first trip that holds one, or
+    // one no longer than SMALL (so no select of the clamped length here), and
     // the sequential pass below takes over at that trip's first slot, with
     // the sums of the slots before it -- those of the sequential pass, which
     // reaches that slot with the same bonds in the same order.
-    constexpr int OPT = SHARED ? 3 : 0;
+    // At 10^6 rows of 112 bonds, two / three / four / five slots per trip:
+    // 0.89 / 0.82 / 0.79 / 0.82 ms (0.84 before the reciprocals came from the
+    // square root); four take 168 registers, three waves per SIMD.
+    constexpr int OPT = SHARED ? 4 : 0;
     if constexpr (OPT > 0) {
       bool brk = false;
       for (; bnd + OPT - 1 <= top; bnd += OPT) {
@@ -169,17 +178,21 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
         }
 #pragma unroll
         for (int k = 0; k < OPT; ++k) gather_asm<FUSE>(a, qv[k], xv[k], sv[k], uv[k]);
-        double e0[OPT], e1[OPT], e2[OPT], dij[OPT], yd[OPT], dr[OPT], th[OPT];
+        // every load before the arithmetic (1.02 ms without at 10^6 rows and
+        // three slots, 0.82 with)
+        __builtin_amdgcn_sched_barrier(0);
+        double e0[OPT], e1[OPT], e2[OPT], dij[OPT], yi[OPT], yd[OPT], dr[OPT], th[OPT];
 #pragma unroll
         for (int k = 0; k < OPT; ++k) {
-          measure(xv[k], sv[k], lv[k], e0[k], e1[k], e2[k], dij[k], yd[k], dr[k], th[k]);
-          brk = brk || dr[k] > th[k];
+          const bool sh = measure(std::true_type{}, xv[k], sv[k], lv[k], e0[k], e1[k], e2[k],
+                                  dij[k], yi[k], yd[k], dr[k], th[k]);
+          brk = brk || sh || dr[k] > th[k];
         }
         if (brk) break;
 #pragma unroll
         for (int k = 0; k < OPT; ++k) {
           track_gap(qv[k], dr[k], th[k]);
-          accumulate(uv[k], lv[k], e0[k], e1[k], e2[k], dij[k], yd[k], dr[k]);
+          accumulate(uv[k], lv[k], e0[k], e1[k], e2[k], dij[k], yi[k], yd[k], dr[k]);
         }
       }
       for (; !brk && bnd <= top; ++bnd) {
@@ -188,12 +201,12 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
         double4 xq, u;
         double sqv;
         gather_asm<FUSE>(a, q, xq, sqv, u);
-        double e0, e1, e2, dij, yd, drdivd, thr;
-        measure(xq, sqv, d0, e0, e1, e2, dij, yd, drdivd, thr);
-        brk = drdivd > thr;
+        double e0, e1, e2, dij, yi, yd, drdivd, thr;
+        brk = measure(std::true_type{}, xq, sqv, d0, e0, e1, e2, dij, yi, yd, drdivd, thr) ||
+              drdivd > thr;
         if (brk) break;
         track_gap(q, drdivd, thr);
-        accumulate(u, d0, e0, e1, e2, dij, yd, drdivd);
+        accumulate(u, d0, e0, e1, e2, dij, yi, yd, drdivd);
       }
     }
     // Sequential pass with swap-remove, in software pipeline: the neighbour
@@ -224,8 +237,9 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
         gather_asm<FUSE>(a, q_n, xq_n, sq_n, us_n);
       }
       if (bnd + 2 <= top) q_nn = a.col[(slot + 2) * 64 + lane];
-      double e0, e1, e2, dij, yd, drdivd, thr;
-      measure(xq, sqv, d0, e0, e1, e2, dij, yd, drdivd, thr);
+      double e0, e1, e2, dij, yi, yd, drdivd, thr;
+      if (measure(std::false_type{}, xq, sqv, d0, e0, e1, e2, dij, yi, yd, drdivd, thr))
+        short_len = true;
       track_gap(q, drdivd, thr);
       if (drdivd > thr) {
         // swap-remove: the last live bond takes this slot, walker stays
@@ -246,7 +260,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
         if (bnd + 1 <= top) q_nn = a.col[(slot + 1) * 64 + lane];
         continue;
       }
-      accumulate(u, d0, e0, e1, e2, dij, yd, drdivd);
+      accumulate(u, d0, e0, e1, e2, dij, yi, yd, drdivd);
       ++bnd;
     }
     // A_pp = K_pp dt^2 + m I
@@ -459,7 +473,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     if (live) atomicAdd(&a.counters->live, live);
   }
   if constexpr (SHARED)
-    if (__any(zero_len) && (threadIdx.x & 63) == 0) atomicOr(&a.counters->range_bad, 2u);
+    if (__any(short_len) && (threadIdx.x & 63) == 0) atomicOr(&a.counters->range_bad, 2u);
 }
 
 template <bool MIXED, bool FUSE, bool GAP>
@@ -734,13 +748,14 @@ __global__ __launch_bounds__(PD_BLOCK) void k_spmv_plain(SpmvView A,
 }
 
 // Self-check of the shared-reciprocal quotients against IEEE division, and
-// of sqrt_nr against IEEE sqrt, over random operands spanning the ranges
-// the range flag admits (odd samples: a coordinate difference over a float
-// bond length; 2 mod 4: a current bond length over a reference length;
-// 0 mod 16: a bond stiffness over a reference length; 8 mod 16: half of a
-// horizon less a reference length over a radius; 4 mod 16: a reference
-// length over a current length; 12 mod 16: the square root of a squared
-// bond length); the exponent ends are drawn often.
+// of sqrt_rcp against IEEE sqrt, over random operands spanning the ranges
+// the range flag admits (odd samples: a squared bond length, its root, a
+// coordinate difference over the root's float and a reference length over
+// the root; 2 mod 4: a current bond length over a reference length; 0 mod
+// 16: a bond stiffness over a reference length; 8 mod 16: half of a horizon
+// less a reference length over a radius; 4 mod 16: the root of the squared
+// length of a bond of any length and a reference length over it; 12 mod 16:
+// a coordinate difference over SMALL); the exponent ends are drawn often.
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   z += 0x9e3779b97f4a7c15ull;
   z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
@@ -760,13 +775,28 @@ __global__ __launch_bounds__(PD_BLOCK) void k_check_division(int64_t samples, ui
   const int64_t i = (int64_t)blockIdx.x * PD_BLOCK + threadIdx.x;
   if (i >= samples) return;
   const uint64_t h1 = mix64(seed ^ (2 * (uint64_t)i)), h2 = mix64(seed ^ (2 * (uint64_t)i + 1));
+  auto differ = [](double u, double v) {
+    return __double_as_longlong(u) != __double_as_longlong(v);
+  };
   double a, b;
-  if (i & 1) {
-    a = (h1 & 15) == 0 ? 0.0 : draw_f64(h1, -352, 100);
-    const float small_f = (float)1.0e-10;
-    float bf = (h2 & 15) == 0 ? small_f : fabsf((float)draw_f64(h2, -34, 101));
-    if (!(bf >= small_f)) bf = small_f;
-    b = (double)bf;
+  bool wrong = false;
+  if ((i & 1) || (i & 15) == 4) {
+    // a bond of length in [1e-10, 2^102] (odd samples) or any
+    const double x = fabs(draw_f64(h1, (i & 1) ? -66 : -704, 203));
+    const uint64_t h3 = mix64(h1 ^ h2);
+    double yi;
+    const double s = sqrt_rcp(x, yi);
+    const double d0 = fabs(draw_f64(h2, -400, 99));
+    wrong = differ(s, sqrt(x)) || differ(d0 / s, div_rcp(d0, s, yi));
+    const float f = (float)s;
+    if ((i & 1) && f > small_len()) {  // a difference is no longer than the bond
+      const double fd = (double)f;
+      a = (h3 & 15) == 0 ? 0.0 : draw_f64(h3, -352, 100);
+      if (fabs(a) > s) a = 0.25 * s;
+      wrong = wrong || differ(a / fd, div_rcp(a, fd, rcp_from(fd, yi)));
+    }
+    if (wrong) atomicAdd(bad, 1ull);
+    return;
   } else if ((i & 3) == 2) {  // a current bond length over a reference length
     a = (h1 & 15) == 0 ? 0.0 : fabs(draw_f64(h1, -537, 101));
     b = fabs(draw_f64(h2, -400, 99));
@@ -776,17 +806,13 @@ __global__ __launch_bounds__(PD_BLOCK) void k_check_division(int64_t samples, ui
   } else if ((i & 15) == 8) {  // (horizon - d0) / 2 over a radius
     a = (h1 & 15) == 0 ? 0.0 : draw_f64(h1, -453, 299);
     b = fabs(draw_f64(h2, -300, 299));
-  } else if ((i & 15) == 4) {  // a reference length over a current length
-    a = fabs(draw_f64(h1, -400, 99));
-    b = fabs(draw_f64(h2, -352, 101));
-  } else {  // the square root of a squared bond length
-    const double x = fabs(draw_f64(h1, -704, 203));
-    if (__double_as_longlong(sqrt(x)) != __double_as_longlong(sqrt_nr(x))) atomicAdd(bad, 1ull);
+  } else {  // a coordinate difference over SMALL
+    a = (h1 & 15) == 0 ? 0.0 : draw_f64(h1, -352, -34);
+    b = (double)small_len();
+    if (differ(a / b, div_rcp(a, b, rcp_from(b, 1.0 / b)))) atomicAdd(bad, 1ull);
     return;
   }
-  const double ieee = a / b;
-  const double shared = div_rcp(a, b, rcp_nr(b));
-  if (__double_as_longlong(ieee) != __double_as_longlong(shared)) atomicAdd(bad, 1ull);
+  if (differ(a / b, div_rcp(a, b, rcp_nr(b)))) atomicAdd(bad, 1ull);
 }
 
 void launch_check_division(int64_t samples, uint64_t seed, unsigned long long* bad,
@@ -988,13 +1014,16 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv(CgArgs a) {
 
 // The matrix-free CG product after an assembly: gathers from the record;
 // with the range flag clear (the common case) shared reciprocals and
-// sqrt_nr, four bonds per trip, else IEEE quotients, two bonds per trip
+// sqrt_rcp, five bonds per trip, else IEEE quotients, two bonds per trip
 // (the general path fits in the common path's registers).
 // The row loop waits on a dependent chain (column, then the neighbour's
 // record) each trip, so the bonds per trip, not the waves per SIMD, hide
-// its latency: at 1M particles 511 us per product with four bonds per trip
-// (126 VGPRs, four waves per SIMD) against 562 with two (76 VGPRs, six
-// waves), 592 with three, 569 with six and 557 with eight.
+// its latency: at 1M particles 480 us per product with five bonds per trip
+// (126 VGPRs, four waves per SIMD) against 504 with three, 492 with four,
+// 481 with six, 500 with seven (164 VGPRs, three waves) and 509 with eight;
+// 504 before 1 / dij came from the square root (12 reciprocal instructions
+// and 372 other FP64 ones per four bonds then, 4 and 348 now).  The columns
+// and lengths of the next trip loaded ahead: 522.
 __global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_mf(CgArgs a) {
   __shared__ double lds4[4];
   const int ntiles = gridDim.x;
@@ -1005,7 +1034,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_mf(CgArgs a) {
   if (p < a.A.n) {
     double y0, y1, y2;
     if (*a.A.range_bad == 0)  // uniform over the grid
-      spmv_row_mf<4, false, true, true>(a.A, a.p, p, y0, y1, y2, a.A.rec);
+      spmv_row_mf<5, false, true, true>(a.A, a.p, p, y0, y1, y2, a.A.rec);
     else
       spmv_row_mf<2, false, true, false>(a.A, a.p, p, y0, y1, y2, a.A.rec);
     a.y[p] = make_double4(y0, y1, y2, 0.0);
@@ -1059,10 +1088,10 @@ __global__ __launch_bounds__(PD_BLOCK) void k_write_blocks(SpmvView A, double* v
   const double dt2 = A.consts ? A.consts->dt2 : A.dt2;
   for (int bnd = 0; bnd <= top; ++bnd) {
     const int64_t i = (base + bnd) * 64 + lane;
-    double e0, e1, e2, dij;
-    bond_dir(pos_p, A.pos[A.col[i]], e0, e1, e2, dij);
+    double e0, e1, e2, dij, yi;
+    bond_dir(pos_p, A.pos[A.col[i]], e0, e1, e2, dij, yi);
     double F00, F01, F02, F11, F12, F22;
-    bond_jac(e0, e1, e2, dij, A.d0[i], cb, F00, F01, F02, F11, F12, F22);
+    bond_jac(e0, e1, e2, dij, yi, A.d0[i], cb, F00, F01, F02, F11, F12, F22);
     store_block(vals, base + bnd, lane, (F00 * -1.0) * dt2, (F01 * -1.0) * dt2,
                 (F02 * -1.0) * dt2, (F11 * -1.0) * dt2, (F12 * -1.0) * dt2, (F22 * -1.0) * dt2);
   }
