@@ -1690,7 +1690,7 @@ int pd_ctx_create(const pd_config* cfg, pd_ctx** out) {
   ALLOC(c->z, n);
   ALLOC(c->p, n);
   ALLOC(c->y, n);
-  ALLOC(c->part, 4 * ntiles);
+  ALLOC(c->part, 8 * ntiles);
   ALLOC(c->st, 1);
   c->state_cap = 1;
   ALLOC(c->counters, 1);

@@ -106,6 +106,9 @@ struct pd_step_counters {
 // this has alpha folded once, by one workgroup, ahead of the update, since
 // the per-workgroup reads grow with the square of its tile count.
 #define PD_ALPHA_FOLD_TILES 8192
+// Largest system, in slices, whose matrix-free product takes four lanes per
+// row (k_cg_spmv_lanes).
+#define PD_LANES_SLICES 1536
 
 __device__ __forceinline__ double4 ld4(const double4* p) { return *p; }
 
@@ -179,11 +182,59 @@ __device__ __forceinline__ double tile_sum(double v, double* lds4) {
   return r;
 }
 
+// Orders a wave's LDS writes before its own lanes' later reads.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc + t[0] + t[1] + .. + t[n - 1], left to right; the next eight terms are
+// on their way from LDS while eight are added.
+__device__ __forceinline__ double chain_add(double acc, const double* t, int n) {
+  double h[8];
+  int e = 0;
+  if (n >= 8) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) h[u] = t[u];
+    for (; e + 16 <= n; e += 8) {
+      double k[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) k[u] = t[e + 8 + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += h[u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) h[u] = k[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += h[u];
+    e += 8;
+  }
+  for (; e < n; ++e) acc += t[e];
+  return acc;
+}
+
 // Final fold of one quantity over the tiles by one 256-thread workgroup:
 // thread t sums part[t], part[t + 256], ... left to right from 0.0, then
 // tile_sum (the oracle's final_combine).
 __device__ __forceinline__ double fold_partials(const double* part, int ntiles, double* lds4) {
   double acc = 0.0;
   for (int k = threadIdx.x; k < ntiles; k += PD_BLOCK) acc = acc + part[k];
+  return tile_sum(acc, lds4);
+}
+
+// The same over tiles t0 .. t0 + nt whose four slices' sums (wave_sum over 64
+// rows each) are given instead: tile_sum's (w0 + w1) + (w2 + w3), slices past
+// the last one summing to +0.
+__device__ __forceinline__ double fold_slices(const double* slices, int nslices, int t0, int nt,
+                                              double* lds4) {
+  double acc = 0.0;
+  for (int k = threadIdx.x; k < nt; k += PD_BLOCK) {
+    const int s = 4 * (t0 + k);
+    const double w0 = slices[s], w1 = s + 1 < nslices ? slices[s + 1] : 0.0;
+    const double w2 = s + 2 < nslices ? slices[s + 2] : 0.0;
+    const double w3 = s + 3 < nslices ? slices[s + 3] : 0.0;
+    acc = acc + ((w0 + w1) + (w2 + w3));
+  }
   return tile_sum(acc, lds4);
 }

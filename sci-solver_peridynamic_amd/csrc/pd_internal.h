@@ -168,7 +168,7 @@ struct CgArgs {
   double4* z;
   double4* p;
   double4* y;
-  double* part;  // [4 * ntiles]
+  double* part;  // [8 * ntiles]: four rows of tiles, then the slices of k_cg_spmv_lanes
   pd_cg_state* st;  // [batch.nspec]
   int32_t precond;
   // stored-block FP64 steps whose assembly left the blocks to the first

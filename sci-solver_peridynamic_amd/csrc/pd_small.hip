@@ -84,12 +84,6 @@ __device__ __forceinline__ double get(const double* p) {
 // whole L2 back on top, 1.5 to 2 us here.
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Fold of NV partial rows over tiles [t0, t0 + nt), nt <= 64 >> K, by one
 // wave: fold_partials' tree.  The units' partials are read 64 at a time, one
 // per lane (a lane per tile reading its units one after another asked for
@@ -143,32 +137,7 @@ __device__ __forceinline__ void fold_units(const double* part, int64_t stride, i
   }
 }
 
-// acc + t[0] + t[1] + .. + t[n - 1], left to right; the next eight terms are
-// on their way from LDS while eight are added.
-__device__ __forceinline__ double chain_add(double acc, const double* t, int n) {
-  double h[8];
-  int e = 0;
-  if (n >= 8) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) h[u] = t[u];
-    for (; e + 16 <= n; e += 8) {
-      double k[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) k[u] = t[e + 8 + u];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) acc += h[u];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) h[u] = k[u];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc += h[u];
-    e += 8;
-  }
-  for (; e < n; ++e) acc += t[e];
-  return acc;
-}
-
-// The same over t[0 .. n), n <= N wave-uniform, in steps of 16 terms with
+// chain_add over t[0 .. n), n <= N wave-uniform, in steps of 16 terms with
 // each term read 16 terms ahead (the terms past a list's end hold -0.0,
 // which changes no sum).  An LDS read costs the same with one lane as with
 // 64: a chain in three lanes of every wave took 32 cycles an addition, all

@@ -1045,6 +1045,122 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_mf(CgArgs a) {
   if (threadIdx.x == 0) a.part[tile] = v;
 }
 
+// Whether the matrix-free product after an assembly takes LANES lanes per
+// row (k_cg_spmv_lanes).
+__host__ __device__ __forceinline__ bool lanes_product(const SpmvView& A) {
+  return A.mf && A.rec && A.range_bad && (A.n + 63) / 64 <= PD_LANES_SLICES;
+}
+
+// The same product for systems whose slices leave the 1024 SIMDs with one
+// wave or two: a lane per row then waits out every trip's chain of column,
+// record and some 90 dependent operations, 20 trips in a row, and one slice
+// more than 1024 doubles the time.  Four lanes share a row, four bonds each
+// per trip, one workgroup per slice; a row's terms pass through LDS and
+// three of its lanes add them in list order, so y keeps its bits.  Partials
+// per slice, joined to the tile's by the fold.
+// us per product, one lane / two / four / eight (106 to 109 bonds a row):
+//   17.6k rows  34 / 24 / 20 / 18      27k  47 / 29 / 23 / 22
+//   65.6k       61 / 45 / 43 / 48     130k  76 / 77 / 82 / 92
+// so four up to PD_LANES_SLICES = 1536 slices (98k rows, where the lines
+// cross), one above.
+__global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_lanes(CgArgs a) {
+  constexpr int L = 4, V = 4, CH = L * V;
+  constexpr int CP = CH + 3;  // odd, so the rows' and components' reads spread over the banks
+  constexpr int RW = 64 / L;  // rows per wave
+  __shared__ double terms[PD_BLOCK / 64][RW * 3 * CP];
+  __shared__ double ts[64];
+  const int ntiles = (a.A.n + PD_BLOCK - 1) / PD_BLOCK;
+  const int s = xcd_tile(blockIdx.x, gridDim.x);
+  if (a.st[spec_of(a.batch, s >> 2)].done) return;
+  double* slice_part = a.part + 4 * (int64_t)ntiles;
+  if (*a.A.range_bad != 0) {  // uniform over the grid; rare: one wave, a lane per row
+    if (threadIdx.x >= 64) return;
+    const int p = s * 64 + threadIdx.x;
+    double t = 0.0;
+    if (p < a.A.n) {
+      double y0, y1, y2;
+      spmv_row_mf<2, false, true, false>(a.A, a.p, p, y0, y1, y2, a.A.rec);
+      a.y[p] = make_double4(y0, y1, y2, 0.0);
+      const double4 pp = rec_vec(a.A.rec, p);
+      t = term3(y0, y1, y2, pp.x, pp.y, pp.z);
+    }
+    const double v = wave_sum(t);
+    if (threadIdx.x == 0) slice_part[s] = v;
+    return;
+  }
+  const int lane = threadIdx.x & 63, r = lane / L, j = lane % L;
+  const int pl = threadIdx.x / L;  // row of the slice
+  const bool row = s * 64 + pl < a.A.n;
+  const int p = row ? s * 64 + pl : a.A.n - 1;
+  const int top = row ? a.A.top[p] : -1;
+  const int64_t base = a.A.slice_off[s];
+  const int* __restrict__ cp = a.A.col + base * 64 + pl;
+  const double* __restrict__ lp = a.A.d0 + base * 64 + pl;
+  // slots past the row's list: the row itself, whose terms are not added
+  auto fetch = [&](int c0, int q[V], double l0[V]) {
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const int k = c0 + u * L + j;
+      const bool in = k <= top;
+      q[u] = in ? ntl(cp + (int64_t)k * 64) : p;
+      l0[u] = in ? ntl(lp + (int64_t)k * 64) : 1.0;
+    }
+  };
+  int q[V];
+  double l0[V];
+  fetch(0, q, l0);
+  const double4 pos_p = a.A.pos[p];
+  const double4 pp = rec_vec(a.A.rec, p);
+  const double cb = a.A.mat[a.A.body[p]].c_bond;
+  const double dt2 = a.A.consts ? a.A.consts->dt2 : a.A.dt2;
+  double acc;  // component j of y (j < 3)
+  {
+    const double* dg = a.A.diag + (int64_t)s * 6 * 64 + pl;
+    double y0, y1, y2;
+    blk6(dg[0], dg[64], dg[128], dg[192], dg[256], dg[320], pp, y0, y1, y2);
+    acc = j == 0 ? y0 : j == 1 ? y1 : y2;
+  }
+  double* tw = terms[threadIdx.x >> 6] + r * 3 * CP;
+  int wtop = top;  // longest list of the wave
+#pragma unroll
+  for (int m = 32; m >= L; m >>= 1) wtop = max(wtop, __shfl_xor(wtop, m, 64));
+  for (int c0 = 0; c0 <= wtop; c0 += CH) {
+    double4 xq[V], vq[V];
+    double lc[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      gather_mf<true>(a.A, a.A.rec, a.p, q[u], xq[u], vq[u]);
+      lc[u] = l0[u];
+    }
+    if (c0 + CH <= wtop) fetch(c0 + CH, q, l0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      double e0, e1, e2, dij, yi;
+      bond_dir<true, true>(pos_p, xq[u], e0, e1, e2, dij, yi);
+      double F00, F01, F02, F11, F12, F22;
+      bond_jac<true, false>(e0, e1, e2, dij, yi, lc[u], cb, F00, F01, F02, F11, F12, F22);
+      double t0, t1, t2;
+      blk6((F00 * -1.0) * dt2, (F01 * -1.0) * dt2, (F02 * -1.0) * dt2, (F11 * -1.0) * dt2,
+           (F12 * -1.0) * dt2, (F22 * -1.0) * dt2, vq[u], t0, t1, t2);
+      tw[u * L + j] = t0;
+      tw[CP + u * L + j] = t1;
+      tw[2 * CP + u * L + j] = t2;
+    }
+    wave_fence();
+    if (j < 3) acc = chain_add(acc, tw + j * CP, min(CH, top + 1 - c0));
+    wave_fence();
+  }
+  if (row) ((double*)(a.y + p))[j] = j < 3 ? acc : 0.0;
+  const double y1 = __shfl_down(acc, 1, 64), y2 = __shfl_down(acc, 2, 64);
+  if (j == 0) ts[pl] = row ? term3(acc, y1, y2, pp.x, pp.y, pp.z) : 0.0;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const double v = wave_sum(ts[threadIdx.x]);
+    if (threadIdx.x == 0) slice_part[s] = v;
+  }
+}
+
 // The first CG product of a stored-block FP64 step whose assembly left the
 // blocks out: every block is recomputed from the gather record (positions
 // and p side by side) exactly as the assembly forms it, written to its slot
@@ -1128,7 +1244,10 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_update(CgArgs a, int it) {
   if (nt > PD_ALPHA_FOLD_TILES) {
     alpha = st->alpha;  // k_cg_alpha folded it ahead of this launch
   } else {
-    const double yp = fold_partials(a.part + t0, nt, lds4);
+    const double yp = lanes_product(a.A)
+                          ? fold_slices(a.part + 4 * (int64_t)ntiles, (a.A.n + 63) / 64, t0, nt,
+                                        lds4)
+                          : fold_partials(a.part + t0, nt, lds4);
     alpha = rz / yp;
     if (tile == t0 && threadIdx.x == 0) {
       st->yp = yp;
@@ -1266,7 +1385,9 @@ void launch_cg_spmv(const CgArgs& a, hipStream_t s) {
   if (!a.A.n) return;
   const int g = tiles_of(a.A.n);
   if (a.A.mf) {
-    if (a.A.rec && a.A.range_bad)  // after an assembly: the record and the range flag
+    if (lanes_product(a.A))
+      hipLaunchKernelGGL(k_cg_spmv_lanes, dim3((a.A.n + 63) / 64), dim3(PD_BLOCK), 0, s, a);
+    else if (a.A.rec && a.A.range_bad)  // after an assembly: the record and the range flag
       hipLaunchKernelGGL(k_cg_spmv_mf, dim3(g), dim3(PD_BLOCK), 0, s, a);
     else
       hipLaunchKernelGGL(k_cg_spmv<0>, dim3(g), dim3(PD_BLOCK), 0, s, a);

@@ -1,0 +1,92 @@
+"""The matrix-free product with four lanes per row (systems up to 1536 slices
+of 64 rows that do not take the resident step: here because they are timed,
+solved on their own or too large for it): row counts at the edges of a wave's
+16 rows, a slice, a tile and of its range, lists of every remainder by its 16
+slots and longer than the resident step's, specimens and a range flag."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as orc
+from pdhelpers import lattice, make_pair, material
+from test_gpu_small import compare, pair
+
+pytestmark = pytest.mark.gpu
+pds = pytest.importorskip("pdsolver")
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def general(S, ctx, steps, **kw):
+    """compare() with the step timed, so that it takes the general kernels."""
+    broken = 0
+    for k in range(1, steps + 1):
+        p = dict(dict(dt=1e-4, clock_scale=min(k, 10) / 10.0, precond=1, rtol=1e-8), **kw)
+        so = S.step(orc.make_params(**p))
+        sg = ctx.step(pds.make_params(matrix_free=1, timing=1, **p))
+        assert (so.cg_iterations, so.broken_bonds, so.residual_norm) == \
+            (sg.cg_iterations, sg.broken_bonds, sg.residual_norm), k
+        for f, want in (("position", S.x), ("velocity", S.v)):
+            assert np.array_equal(ctx.download(f)[:, :3], want[:, :3]), (f, k)
+        broken += sg.broken_bonds
+    assert np.array_equal(ctx.download("bond_top"), S.top)
+    return broken
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 63, 64, 65, 255, 257, 1000, 8193])
+def test_sizes_match_oracle(n):
+    say("case lanes n", n)
+    S, ctx = pair(n)
+    say(dict(broken=general(S, ctx, 8 if n < 4000 else 4)))
+    ctx.close()
+
+
+@pytest.mark.parametrize("factor", [1.1, 1.8, 2.3, 2.9, 4.2])
+def test_list_lengths(factor):
+    say("case lanes factor", factor)
+    S, ctx = pair(1000, pull=2.0, factor=factor)
+    say(dict(longest=int(S.top.max()) + 1, broken=general(S, ctx, 4, precond=0)))
+    ctx.close()
+
+
+def test_first_size_past_the_resident_step():
+    say("case lanes 16385")
+    S, ctx = pair(16385)
+    compare(S, ctx, 3, matrix_free=1)
+    ctx.close()
+
+
+def test_operands_out_of_range_take_ieee_forms():
+    say("case lanes range flag")
+    x4 = lattice(6, 6, 8, 0.01, 0.0, 3)
+    x4[:, :3] -= x4[0, :3]
+    x4[5, 1] = 1e-200
+    S, ctx = make_pair(x4, [material(0.01)])
+    general(S, ctx, 4)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n", [98304, 98305])
+def test_ends_of_the_range_equal_stored(n):
+    """The last size with four lanes and the first with one, against the
+    stored blocks."""
+    say("case lanes n", n)
+    x4 = lattice(48, 48, -(-n // 2304), 0.01, 0.05, n)[:n]
+    v4 = np.zeros((n, 4))
+    v4[:, 2] = np.linspace(-1, 1, n)
+    out = []
+    for mode in (0, 1):
+        ctx = pds.Context(n, [material(0.01, 1.8)])
+        pds.load_state(ctx, x4, v4, np.full(n, 0.02))
+        ctx.build_bonds()
+        st = [ctx.step(pds.make_params(dt=1e-4, precond=1, rtol=1e-8, matrix_free=mode))
+              for _ in range(3)]
+        out.append(([(s.cg_iterations, s.broken_bonds, s.residual_norm) for s in st],
+                    ctx.download("position"), ctx.download("velocity")))
+        ctx.close()
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
