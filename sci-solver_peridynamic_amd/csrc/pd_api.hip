@@ -1814,16 +1814,12 @@ int pd_upload(pd_ctx* c, int32_t field, const void* src, size_t bytes) {
         return fail(c, PD_ERR_ARG, "body index outside [0, num_bodies)");
   }
   HIPCHK(c, hipSetDevice(c->device));
+  HIPCHK(c, hipMemcpyAsync(*fi.dptr, src, bytes, hipMemcpyHostToDevice, c->stream));
   if (fi.vec4) {
-    // the w lane is not part of the state: store it as 0
-    std::vector<double> tmp((const double*)src, (const double*)src + 4 * (size_t)c->n);
-    for (size_t i = 0; i < (size_t)c->n; ++i) tmp[4 * i + 3] = 0.0;
-    HIPCHK(c, hipMemcpyAsync(*fi.dptr, tmp.data(), bytes, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  } else {
-    HIPCHK(c, hipMemcpyAsync(*fi.dptr, src, bytes, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    pd::launch_zero_w((double4*)*fi.dptr, c->n, c->stream);
+    CHECK_LAUNCH(c, "upload");
   }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   return PD_OK;
 }
 

@@ -414,6 +414,7 @@ void launch_update(int32_t n, double4* x, double4* v, const double4* sol,
                    const pd_step_consts* consts, hipStream_t s,
                    const unsigned int* skip = nullptr);
 void launch_copy(double* dst, const double* src, int32_t n, hipStream_t s);
+void launch_zero_w(double4* v, int32_t n, hipStream_t s);
 // Compares shared-reciprocal quotients with IEEE division on `samples`
 // random operand pairs; *bad counts the differing ones.
 void launch_check_division(int64_t samples, uint64_t seed, unsigned long long* bad,
