@@ -1853,7 +1853,8 @@ int pd_build_bonds(pd_ctx* c, pd_bond_stats* stats) {
     // one cell of each other despite rounding in the cell index
     pd::GridView g;
     if (int e = build_grid(c, hmax * (1.0 + 1e-7), &g)) return e;
-    pd::launch_bond_count(n, c->x, c->body, c->act, c->dhorizon, g, c->counts, c->stream);
+    pd::launch_bond_count(n, c->x, c->body, c->act, c->dhorizon, g, c->counts, c->z,
+                          c->stream);
     CHECK_LAUNCH(c, "bond count");
     pd::launch_slice_width(c->counts, n, c->widths, c->stream);
     CHECK_LAUNCH(c, "slice width");
@@ -1871,7 +1872,7 @@ int pd_build_bonds(pd_ctx* c, pd_bond_stats* stats) {
     }
     if (int e = set_slice_offsets(c, widths)) return e;
     pd::launch_bond_fill(n, c->x, c->body, c->act, c->dhorizon, g, c->counts, c->slice_off, c->col,
-                         c->top, c->cap, c->stream);
+                         c->top, c->cap, c->z, mx, c->stream);
     CHECK_LAUNCH(c, "bond fill");
   } else {
     if (int e = set_slice_offsets(c, widths)) return e;

@@ -494,12 +494,12 @@ int launch_small_grid(const double4* x, const int32_t* subset, int32_t m, const 
 // INVISIBLE particles take no bonds and are no one's neighbour
 void launch_bond_count(int32_t n, const double4* x, const int32_t* body, const int32_t* act,
                        const double* horizon, const GridView& g, int32_t* counts,
-                       hipStream_t s);
+                       double4* rec, hipStream_t s);
 void launch_slice_width(const int32_t* counts, int32_t n, int32_t* widths,
                         hipStream_t s);
 void launch_bond_fill(int32_t n, const double4* x, const int32_t* body, const int32_t* act,
                       const double* horizon, const GridView& g, const int32_t* counts,
                       const int64_t* slice_off, int32_t* col, int32_t* top,
-                      int32_t* cap, hipStream_t s);
+                      int32_t* cap, double4* rec, int32_t longest, hipStream_t s);
 
 }  // namespace pd
