@@ -42,12 +42,14 @@ struct pd_cg_state {
   double tol;    // rtol * bnorm
   double rnorm;  // sqrt(rr)
   double rtol;
+  double upd_rz;  // rz and iter as that update found them
   int32_t iter;
   int32_t done;
   int32_t converged;
   int32_t max_iter;
   int32_t upd_it;  // the iteration whose update ran last (-1: none yet)
-  uint32_t pad[3];
+  int32_t upd_iter;
+  uint32_t pad[2];
 };
 
 // Scalars of one mixed-precision solve (iterative refinement around a float
@@ -106,6 +108,11 @@ struct pd_step_counters {
 // this has alpha folded once, by one workgroup, ahead of the update, since
 // the per-workgroup reads grow with the square of its tile count.
 #define PD_ALPHA_FOLD_TILES 8192
+// Largest system, in tiles, whose direction update folds <r, z> and <r, r>
+// itself, in every workgroup, instead of after a one-workgroup kernel: 4.8 us
+// for both against 8.6 at 110 tiles, 5.4 against 8.2 at 510, but 41.8 against
+// 37.2 at 3930, where the workgroups' reads add up to 250 MB.
+#define PD_DIR_FOLD_TILES 1024
 // Largest system, in slices, whose matrix-free product takes four lanes per
 // row (k_cg_spmv_lanes).
 #define PD_LANES_SLICES 1536
@@ -217,10 +224,36 @@ __device__ __forceinline__ double chain_add(double acc, const double* t, int n) 
 // Final fold of one quantity over the tiles by one 256-thread workgroup:
 // thread t sums part[t], part[t + 256], ... left to right from 0.0, then
 // tile_sum (the oracle's final_combine).
-__device__ __forceinline__ double fold_partials(const double* part, int ntiles, double* lds4) {
+// Eight loads are under way at a time (one after another, 4000 tiles took 5 us
+// a fold): the zeros added past the end change no sum, which is never -0.
+__device__ __forceinline__ double fold_strided(const double* part, int ntiles) {
   double acc = 0.0;
-  for (int k = threadIdx.x; k < ntiles; k += PD_BLOCK) acc = acc + part[k];
-  return tile_sum(acc, lds4);
+  for (int k = threadIdx.x; k < ntiles; k += 8 * PD_BLOCK) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = k + u * PD_BLOCK < ntiles ? part[k + u * PD_BLOCK] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = acc + v[u];
+  }
+  return acc;
+}
+__device__ __forceinline__ double fold_partials(const double* part, int ntiles, double* lds4) {
+  return tile_sum(fold_strided(part, ntiles), lds4);
+}
+// Two quantities at once, one exchange.
+__device__ __forceinline__ void fold_pair(const double* part0, const double* part1, int ntiles,
+                                          double* lds8, double& s0, double& s1) {
+  double v0 = fold_strided(part0, ntiles), v1 = fold_strided(part1, ntiles);
+  v0 = wave_sum(v0);
+  v1 = wave_sum(v1);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    lds8[w] = v0;
+    lds8[4 + w] = v1;
+  }
+  __syncthreads();
+  s0 = (lds8[0] + lds8[1]) + (lds8[2] + lds8[3]);
+  s1 = (lds8[4] + lds8[5]) + (lds8[6] + lds8[7]);
 }
 
 // The same over tiles t0 .. t0 + nt whose four slices' sums (wave_sum over 64

@@ -1254,7 +1254,11 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_update(CgArgs a, int it) {
       st->alpha = alpha;
     }
   }
-  if (tile == t0 && threadIdx.x == 0) st->upd_it = it;
+  if (tile == t0 && threadIdx.x == 0) {
+    st->upd_it = it;
+    st->upd_rz = rz;
+    st->upd_iter = st->iter;
+  }
   double t_rz = 0.0, t_rr = 0.0;
   if (row) {
     if (fr) {
@@ -1295,55 +1299,88 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_alpha(CgArgs a, int ntiles) {
 }
 
 // beta = rz' / rz, iteration count and the monitor test ahead of the next
-// iteration (||r|| <= tol converged, iter >= max_iter failed), for every
-// specimen whose update ran in iteration `it`
+// iteration (||r|| <= tol converged, iter >= max_iter failed) of a specimen
+// whose update ran, from what that update found (upd_rz, upd_iter): every
+// workgroup that forms it gets the same, also while one records it.
+struct CgEnd {
+  double beta;
+  bool done;
+};
+__device__ __forceinline__ CgEnd cg_end(pd_cg_state* st, double rz, double rr, bool record) {
+  const double rnorm = sqrt(rr);
+  const int iter = st->upd_iter + 1;
+  const bool converged = rnorm <= st->tol;
+  CgEnd e;
+  e.beta = rz / st->upd_rz;
+  e.done = converged || iter >= st->max_iter;
+  if (record) {
+    st->rz = rz;
+    st->beta = e.beta;
+    st->iter = iter;
+    st->rr = rr;
+    st->rnorm = rnorm;
+    if (converged) st->converged = 1;
+    if (e.done) st->done = 1;
+  }
+  return e;
+}
+
+// The same ahead of k_cg_dir<false>, one workgroup per specimen
 __global__ __launch_bounds__(PD_BLOCK) void k_cg_beta(CgArgs a, int ntiles, int it) {
   if (a.st[blockIdx.x].upd_it != it) return;
-  __shared__ double lds4[4];
+  __shared__ double lds8[8];
   int t0, nt;
   spec_range(a.batch, ntiles, t0, nt);
-  const double rz = fold_partials(a.part + 2 * (int64_t)ntiles + t0, nt, lds4);
-  const double rr = fold_partials(a.part + 3 * (int64_t)ntiles + t0, nt, lds4);
-  if (threadIdx.x == 0) {
-    pd_cg_state* st = a.st + blockIdx.x;
-    const double rz_old = st->rz;
-    st->rz = rz;
-    st->beta = rz / rz_old;
-    st->iter = st->iter + 1;
-    st->rr = rr;
-    const double rnorm = sqrt(rr);
-    st->rnorm = rnorm;
-    if (rnorm <= st->tol) {
-      st->done = 1;
-      st->converged = 1;
-    } else if (st->iter >= st->max_iter) {
-      st->done = 1;
-    }
-  }
+  double rz, rr;
+  fold_pair(a.part + 2 * (int64_t)ntiles + t0, a.part + 3 * (int64_t)ntiles + t0, nt, lds8, rz,
+            rr);
+  if (threadIdx.x == 0) cg_end(a.st + blockIdx.x, rz, rr, true);
 }
 
 // The end of iteration `it` for every specimen whose update ran in it:
-// x += alpha p, and, unless k_cg_beta found the solve ended, p = z + beta p.
+// x += alpha p, and, unless the solve has ended, p = z + beta p.  FOLD: beta
+// and the end are formed here, by every workgroup (PD_DIR_FOLD_TILES), and
+// recorded by the specimen's first.
+template <bool FOLD>
 __global__ __launch_bounds__(PD_BLOCK) void k_cg_dir(CgArgs a, int it) {
-  const int tile = xcd_tile(blockIdx.x, gridDim.x);
-  const pd_cg_state* st = a.st + spec_of(a.batch, tile);
+  __shared__ double lds8[8];
+  const int ntiles = gridDim.x;
+  const int tile = xcd_tile(blockIdx.x, ntiles);
+  const int s = spec_of(a.batch, tile);
+  pd_cg_state* st = a.st + s;
   if (st->upd_it != it) return;  // the solve had ended before this iteration
   const int p = tile * PD_BLOCK + threadIdx.x;
-  if (p >= a.A.n) return;
+  const bool row = p < a.A.n;
   // matrix-free (A.rec set): p lives in the gather record alone
-  double4 pp = a.A.rec ? rec_vec(a.A.rec, p) : a.p[p];
-  double4 xx = a.x[p];
+  double4 pp = make_double4(0.0, 0.0, 0.0, 0.0), xx = pp, zz = pp;
+  if (row) {  // ahead of the fold
+    pp = a.A.rec ? rec_vec(a.A.rec, p) : a.p[p];
+    xx = a.x[p];
+    if (FOLD) zz = a.z[p];
+  }
+  CgEnd e;
+  if constexpr (FOLD) {
+    int t0, nt;
+    spec_range_of(a.batch, s, ntiles, t0, nt);
+    double rz, rr;
+    fold_pair(a.part + 2 * (int64_t)ntiles + t0, a.part + 3 * (int64_t)ntiles + t0, nt, lds8, rz,
+              rr);
+    e = cg_end(st, rz, rr, tile == t0 && threadIdx.x == 0);
+  } else {
+    e.beta = st->beta;
+    e.done = st->done;
+  }
+  if (!row) return;
   const double alpha = st->alpha;
   xx.x = alpha * pp.x + xx.x;
   xx.y = alpha * pp.y + xx.y;
   xx.z = alpha * pp.z + xx.z;
   a.x[p] = xx;
-  if (st->done) return;
-  const double beta = st->beta;
-  const double4 zz = a.z[p];
-  pp.x = zz.x + beta * pp.x;
-  pp.y = zz.y + beta * pp.y;
-  pp.z = zz.z + beta * pp.z;
+  if (e.done) return;
+  if (!FOLD) zz = a.z[p];
+  pp.x = zz.x + e.beta * pp.x;
+  pp.y = zz.y + e.beta * pp.y;
+  pp.z = zz.z + e.beta * pp.z;
   if (a.A.rec)
     rec_p(a.A.rec, p, pp.x, pp.y, pp.z);
   else
@@ -1417,8 +1454,12 @@ void launch_cg_update(const CgArgs& a, int it, hipStream_t s) {
 void launch_cg_dir(const CgArgs& a, int it, hipStream_t s) {
   if (!a.A.n) return;
   const int g = tiles_of(a.A.n);
+  if (g <= PD_DIR_FOLD_TILES) {
+    hipLaunchKernelGGL(k_cg_dir<true>, dim3(g), dim3(PD_BLOCK), 0, s, a, it);
+    return;
+  }
   hipLaunchKernelGGL(k_cg_beta, dim3(a.batch.nspec), dim3(PD_BLOCK), 0, s, a, g, it);
-  hipLaunchKernelGGL(k_cg_dir, dim3(g), dim3(PD_BLOCK), 0, s, a, it);
+  hipLaunchKernelGGL(k_cg_dir<false>, dim3(g), dim3(PD_BLOCK), 0, s, a, it);
 }
 
 // ---------------------------------------------------------------------------
