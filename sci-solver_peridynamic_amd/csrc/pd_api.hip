@@ -611,17 +611,11 @@ int enqueue_contact(pd_ctx* c, const pd_step_params* prm) {
   // same order.
   const double w = prm->contact_radius * (1.0 + 1e-6);
   pd::launch_bbox_bodies(c->x, c->body, c->n, c->nbody, c->bbox_part, c->bbox, c->stream,
-                         c->plan, w);
-  const size_t tw = pd::zone_tile_words(c->n);
-  pd::launch_zone_select(c->x, c->body, c->n, &c->plan->z, c->zone_cnt, c->cand, c->stream,
-                         c->fc);
+                         c->plan, c->h_plan, w);
+  pd::launch_zone_select(c->x, c->body, c->n, &c->plan->z, c->zone_cnt, c->cand,
+                         c->h_zone_count, c->stream, c->fc);
   CHECK_LAUNCH(c, "contact candidates");
-  HIPCHK(c, hipMemcpyAsync(c->h_plan, c->plan, sizeof(pd::ContactPlan), hipMemcpyDeviceToHost,
-                           c->stream));
   uint32_t m = 0;
-  if (c->n > 0)
-    HIPCHK(c, hipMemcpyAsync(c->h_zone_count, c->zone_cnt + tw - 1, sizeof(uint32_t),
-                             hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   const pd::ContactPlan& P = *c->h_plan;
   for (int k = 0; k < 3; ++k)

@@ -9,6 +9,8 @@
 // lists equal the reference's bit for bit once sorted.
 #include <math.h>
 
+#include <algorithm>
+
 #include "pd_internal.h"
 #include "pd_solver.h"  // PD_MAX_BODIES
 
@@ -76,46 +78,51 @@ static const int kBodyBboxBlocks = 1024;
 __device__ __forceinline__ double first_min(double a, double b) { return b < a ? b : a; }
 __device__ __forceinline__ double first_max(double a, double b) { return a < b ? b : a; }
 
-// The contact plan (one thread): the zones are the body boxes widened by
-// w, and the sub-grid box is the bound of every zone's intersection with
-// another body's box, formed in the order of the host loops it replaces.
+// The contact plan (one wave; lane k < 3 forms coordinate k): the zones are the
+// body boxes widened by w, and the sub-grid box is the bound of every zone's
+// intersection with another body's box, formed in the order of the host
+// loops it replaces.
 __device__ void contact_plan(const double* bb, int nb, double w, ContactPlan& P) {
-  for (int k = 0; k < 3; ++k) {
-    P.mn[k] = P.ulo[k] = P.glo[k] = INFINITY;
-    P.mx[k] = P.uhi[k] = P.ghi[k] = -INFINITY;
+  const int k = min((int)(threadIdx.x & 63), 2);
+  double mn = INFINITY, mx = -INFINITY, ulo = INFINITY, uhi = -INFINITY, glo = INFINITY,
+         ghi = -INFINITY;
+  for (int b = 0; b < nb; ++b) {
+    const double lo = bb[6 * b + k], hi = bb[6 * b + 3 + k];
+    mn = first_min(mn, lo);
+    mx = first_max(mx, hi);
+    ulo = first_min(ulo, lo - w);
+    uhi = first_max(uhi, hi + w);
   }
-  for (int b = 0; b < nb; ++b)
-    for (int k = 0; k < 3; ++k) {
-      P.mn[k] = first_min(P.mn[k], bb[6 * b + k]);
-      P.mx[k] = first_max(P.mx[k], bb[6 * b + 3 + k]);
-    }
-  P.z.nbody = nb;
-  for (int b = 0; b < PD_MAX_ZONE_BODIES; ++b)
-    for (int k = 0; k < 3; ++k) {
-      P.z.lo[b][k] = b < nb ? bb[6 * b + k] - w : INFINITY;  // empty bodies: +inf, no zone
-      P.z.hi[b][k] = b < nb ? bb[6 * b + 3 + k] + w : -INFINITY;
-    }
-  for (int b = 0; b < nb; ++b)
-    for (int k = 0; k < 3; ++k) {
-      P.ulo[k] = first_min(P.ulo[k], P.z.lo[b][k]);
-      P.uhi[k] = first_max(P.uhi[k], P.z.hi[b][k]);
-    }
+  for (int b = 0; b < PD_MAX_ZONE_BODIES; ++b) {
+    P.z.lo[b][k] = b < nb ? bb[6 * b + k] - w : INFINITY;  // empty bodies: +inf, no zone
+    P.z.hi[b][k] = b < nb ? bb[6 * b + 3 + k] + w : -INFINITY;
+  }
   for (int b = 0; b < nb; ++b)
     for (int o = 0; o < nb; ++o) {
       if (o == b) continue;
-      double lo[3], hi[3];
-      bool meet = true;
-      for (int k = 0; k < 3; ++k) {
-        lo[k] = first_max(P.z.lo[b][k], bb[6 * o + k]);
-        hi[k] = first_min(P.z.hi[b][k], bb[6 * o + 3 + k]);
-        meet = meet && lo[k] <= hi[k];
-      }
-      if (!meet) continue;
-      for (int k = 0; k < 3; ++k) {
-        P.glo[k] = first_min(P.glo[k], lo[k]);
-        P.ghi[k] = first_max(P.ghi[k], hi[k]);
-      }
+      const double lo = first_max(bb[6 * b + k] - w, bb[6 * o + k]);
+      const double hi = first_min(bb[6 * b + 3 + k] + w, bb[6 * o + 3 + k]);
+      if (!__all(lo <= hi)) continue;
+      glo = first_min(glo, lo);
+      ghi = first_max(ghi, hi);
     }
+  P.z.nbody = nb;
+  P.mn[k] = mn;
+  P.mx[k] = mx;
+  P.ulo[k] = ulo;
+  P.uhi[k] = uhi;
+  P.glo[k] = glo;
+  P.ghi[k] = ghi;
+}
+
+// The smallest (LO) or largest v of the wave.
+template <bool LO, int M>
+__device__ __forceinline__ double wave_extreme(double v) {
+  double a, b;
+  xor_pair<M>(v, a, b);
+  v = LO ? fmin(a, b) : fmax(a, b);
+  if constexpr (M > 1) return wave_extreme<LO, M / 2>(v);
+  return v;
 }
 
 // Bounding boxes of all bodies in one pass: per block (lo xyz, hi xyz) for
@@ -150,12 +157,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_bbox_bodies_partial(const double4*
     if (b >= nbody) break;  // uniform: only the bodies that exist are folded
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      double t = v[b][k];
-#pragma unroll
-      for (int m = 32; m >= 1; m >>= 1) {
-        const double o = __shfl_xor(t, m, 64);
-        t = k < 3 ? fmin(t, o) : fmax(t, o);
-      }
+      const double t = k < 3 ? wave_extreme<true, 32>(v[b][k]) : wave_extreme<false, 32>(v[b][k]);
       if (lane == 0) s[wave][b * 6 + k] = t;
     }
   }
@@ -169,56 +171,61 @@ __global__ __launch_bounds__(PD_BLOCK) void k_bbox_bodies_partial(const double4*
   }
 }
 
-// each thread folds the block partials t, t + 256, ... (g <= 4 PD_BLOCK),
-// then every value of the bodies that exist is folded by wave butterflies
-// and across the four waves; the other bodies' entries are left unwritten.
-// plan non-null: thread 0 then forms the contact plan from the boxes
-// (contact_plan, zones widened by w).
+// Wave w folds the block partials of bodies w, w + 4, ..: a lane blocks lane,
+// lane + 64, .., then a butterfly; the other bodies' entries are left
+// unwritten.  plan non-null: the first wave then forms the contact plan from
+// the boxes (contact_plan, zones widened by w), kept on the device and, for
+// the host's wait, in host memory.
+// One workgroup of latency: 15.8 -> 3.8 us at two bodies and 110 blocks (a value after another
+// over all waves, butterflies through the LDS crossbar, the plan by one
+// thread on LDS).
 __global__ __launch_bounds__(PD_BLOCK) void k_bbox_bodies_final(const double* part, int g,
                                                                int nbody, double* out,
-                                                               ContactPlan* plan, double w) {
-  __shared__ double s[PD_BLOCK / 64][PD_MAX_BODIES * 6];
+                                                               ContactPlan* plan,
+                                                               ContactPlan* hplan, double w) {
   __shared__ double box[PD_MAX_BODIES * 6];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int k = 0; k < nbody * 6; ++k) {
-    const bool lo = (k % 6) < 3;
-    double r = lo ? INFINITY : -INFINITY;
-    for (int i = t; i < g; i += PD_BLOCK) {
-      const double v = part[i * PD_MAX_BODIES * 6 + k];
-      r = lo ? fmin(r, v) : fmax(r, v);
+  for (int b = wave; b < nbody; b += PD_BLOCK / 64) {
+    double r[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) r[k] = k < 3 ? INFINITY : -INFINITY;
+#pragma unroll 4
+    for (int i = lane; i < g; i += 64) {
+      const double* v = part + ((int64_t)i * PD_MAX_BODIES + b) * 6;
+#pragma unroll
+      for (int k = 0; k < 6; ++k) r[k] = k < 3 ? fmin(r[k], v[k]) : fmax(r[k], v[k]);
     }
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      const double o = __shfl_xor(r, m, 64);
-      r = lo ? fmin(r, o) : fmax(r, o);
+    for (int k = 0; k < 6; ++k) {
+      r[k] = k < 3 ? wave_extreme<true, 32>(r[k]) : wave_extreme<false, 32>(r[k]);
+      if (lane == 0) {
+        out[b * 6 + k] = r[k];
+        box[b * 6 + k] = r[k];
+      }
     }
-    if (lane == 0) s[wave][k] = r;
-  }
-  __syncthreads();
-  if (t < nbody * 6) {
-    const bool lo = (t % 6) < 3;
-    double r = s[0][t];
-    for (int w = 1; w < PD_BLOCK / 64; ++w) r = lo ? fmin(r, s[w][t]) : fmax(r, s[w][t]);
-    out[t] = r;
-    box[t] = r;
   }
   if (!plan) return;  // uniform
   __shared__ ContactPlan sp;
   __syncthreads();
-  if (t == 0) contact_plan(box, nbody, w, sp);
+  if (wave == 0) contact_plan(box, nbody, w, sp);
   __syncthreads();
   static_assert(sizeof(ContactPlan) % 8 == 0, "the plan is copied in 8-byte words");
   const uint64_t* src = (const uint64_t*)&sp;
-  uint64_t* dst = (uint64_t*)plan;
-  for (int i = t; i < (int)(sizeof(ContactPlan) / 8); i += PD_BLOCK) dst[i] = src[i];
+  for (int i = t; i < (int)(sizeof(ContactPlan) / 8); i += PD_BLOCK) {
+    ((uint64_t*)plan)[i] = src[i];
+    ((uint64_t*)hplan)[i] = src[i];
+  }
 }
 
 void launch_bbox_bodies(const double4* x, const int32_t* body, int32_t n, int32_t nbody,
-                        double* part, double* out, hipStream_t s, ContactPlan* plan, double w) {
-  hipLaunchKernelGGL(k_bbox_bodies_partial, dim3(kBodyBboxBlocks), dim3(PD_BLOCK), 0, s, x,
-                     body, n, nbody, part);
-  hipLaunchKernelGGL(k_bbox_bodies_final, dim3(1), dim3(PD_BLOCK), 0, s, part, kBodyBboxBlocks,
-                     nbody, out, plan, w);
+                        double* part, double* out, hipStream_t s, ContactPlan* plan,
+                        ContactPlan* hplan, double w) {
+  // a workgroup per 256 particles, at most four per CU
+  const int g = std::max(1, std::min(kBodyBboxBlocks, (n + PD_BLOCK - 1) / PD_BLOCK));
+  hipLaunchKernelGGL(k_bbox_bodies_partial, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, nbody,
+                     part);
+  hipLaunchKernelGGL(k_bbox_bodies_final, dim3(1), dim3(PD_BLOCK), 0, s, part, g, nbody, out,
+                     plan, hplan, w);
 }
 
 void launch_bbox(const double4* x, const int32_t* body, int32_t n, int32_t body_sel,
@@ -230,10 +237,15 @@ void launch_bbox(const double4* x, const int32_t* body, int32_t n, int32_t body_
 
 // ------------------------------------------------------------ compaction
 // Stable selection of the particles inside any zone box of another body:
-// per-tile counts, an exclusive scan of the counts, then each tile writes
-// its selected indices in ascending order.
+// per-tile counts, then each tile writes its selected indices in ascending
+// order, behind the counts of the tiles before it: up to CP_DIRECT tiles of
+// 256 particles every workgroup adds them up itself, more (tiles of 1024)
+// are scanned by a kernel of one workgroup first, whose launch alone takes 4
+// us.  Tiles of 256: count and write of 28k particles 8.0 + 5.4 -> 4.1 + 3.5 us
+// (28 workgroups of four particles a thread left most of the chip idle); at
+// 10^6 particles 14.3 + 10.8 us against 14.4 + 8.3 and 4.2 for the scan.
 #define CP_ITEMS 4
-#define CP_TILE (PD_BLOCK * CP_ITEMS)
+#define CP_DIRECT 4096
 
 __device__ __forceinline__ bool in_zone(const double4 p, int b, const ZoneBoxes* __restrict__ z) {
   for (int k = 0; k < z->nbody; ++k) {
@@ -246,14 +258,14 @@ __device__ __forceinline__ bool in_zone(const double4 p, int b, const ZoneBoxes*
 }
 
 __global__ __launch_bounds__(PD_BLOCK) void k_zone_count(const double4* x, const int32_t* body,
-                                                        int n, const ZoneBoxes* z,
+                                                        int n, int items, const ZoneBoxes* z,
                                                         uint32_t* tile_cnt, double4* fc) {
   __shared__ uint32_t c;
   if (threadIdx.x == 0) c = 0;
   __syncthreads();
   uint32_t mine = 0;
-  for (int j = 0; j < CP_ITEMS; ++j) {
-    const int i = blockIdx.x * CP_TILE + j * PD_BLOCK + threadIdx.x;
+  for (int j = 0; j < items; ++j) {
+    const int i = (blockIdx.x * items + j) * PD_BLOCK + threadIdx.x;
     if (i < n) {
       if (fc) fc[i] = make_double4(0.0, 0.0, 0.0, 0.0);
       if (in_zone(x[i], body[i], z)) ++mine;
@@ -290,18 +302,32 @@ __global__ __launch_bounds__(1024) void k_scan_small(uint32_t* v, int g) {
   if (t == 1023) v[g] = sums[1023];
 }
 
+// tile_cnt: the tiles' counts, SCANNED: their exclusive scan.  The last tile
+// writes the number of candidates to *total (host memory).
+template <bool SCANNED>
 __global__ __launch_bounds__(PD_BLOCK) void k_zone_scatter(const double4* x, const int32_t* body,
-                                                          int n, const ZoneBoxes* z,
-                                                          const uint32_t* tile_off,
-                                                          int32_t* out) {
+                                                          int n, int items, const ZoneBoxes* z,
+                                                          const uint32_t* tile_cnt, int32_t* out,
+                                                          uint32_t* total) {
   __shared__ uint32_t wcnt[4];
   __shared__ uint32_t run;
   const int w = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const unsigned long long lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  if (threadIdx.x == 0) run = tile_off[blockIdx.x];
-  for (int j = 0; j < CP_ITEMS; ++j) {
-    const int i = blockIdx.x * CP_TILE + j * PD_BLOCK + threadIdx.x;
+  if constexpr (SCANNED) {
+    if (threadIdx.x == 0) run = tile_cnt[blockIdx.x];
+  } else {
+    uint32_t acc = 0;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += PD_BLOCK) acc += tile_cnt[k];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, 64);
+    if (lane == 0) wcnt[w] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) run = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
+  }
+  for (int j = 0; j < items; ++j) {
+    const int i = (blockIdx.x * items + j) * PD_BLOCK + threadIdx.x;
     const bool sel = i < n && in_zone(x[i], body[i], z);
     const unsigned long long m = __ballot(sel);
     __syncthreads();
@@ -313,18 +339,28 @@ __global__ __launch_bounds__(PD_BLOCK) void k_zone_scatter(const double4* x, con
     __syncthreads();
     if (threadIdx.x == 0) run += wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
   }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = run;
 }
 
 void launch_zone_select(const double4* x, const int32_t* body, int32_t n, const ZoneBoxes* z,
-                        uint32_t* tile_cnt, int32_t* out, hipStream_t s, double4* fc) {
-  const int g = (n + CP_TILE - 1) / CP_TILE;
-  if (g == 0) return;
-  hipLaunchKernelGGL(k_zone_count, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, z, tile_cnt, fc);
+                        uint32_t* tile_cnt, int32_t* out, uint32_t* total, hipStream_t s,
+                        double4* fc) {
+  if (n <= 0) return;
+  const int items = (n + PD_BLOCK - 1) / PD_BLOCK <= CP_DIRECT ? 1 : CP_ITEMS;
+  const int g = (n + PD_BLOCK * items - 1) / (PD_BLOCK * items);
+  hipLaunchKernelGGL(k_zone_count, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, items, z, tile_cnt,
+                     fc);
+  if (items == 1) {
+    hipLaunchKernelGGL(k_zone_scatter<false>, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, items, z,
+                       tile_cnt, out, total);
+    return;
+  }
   hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, tile_cnt, g);
-  hipLaunchKernelGGL(k_zone_scatter, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, z, tile_cnt, out);
+  hipLaunchKernelGGL(k_zone_scatter<true>, dim3(g), dim3(PD_BLOCK), 0, s, x, body, n, items, z,
+                     tile_cnt, out, total);
 }
 
-size_t zone_tile_words(int32_t n) { return (size_t)(n + CP_TILE - 1) / CP_TILE + 1; }
+size_t zone_tile_words(int32_t n) { return (size_t)(n + PD_BLOCK - 1) / PD_BLOCK + 1; }
 
 // ---------------------------------------------------------------- keys
 __device__ __forceinline__ void cell_of(const double4 p, const double* mn, double cell,

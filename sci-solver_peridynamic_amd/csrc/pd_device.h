@@ -142,16 +142,19 @@ __device__ __forceinline__ double dpp_mov(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
   return __longlong_as_double(((int64_t)hi << 32) | (uint32_t)lo);
 }
+// v and the v of the lane M away by xor (a, b: in either order, the same in
+// both lanes of a pair when M >= 16)
 template <int M>
-__device__ __forceinline__ double xor_add(double v) {
-  if constexpr (M == 1) return v + dpp_mov<0xb1>(v);                  // quad_perm 1 0 3 2
-  if constexpr (M == 2) return v + dpp_mov<0x4e>(v);                  // quad_perm 2 3 0 1
-  if constexpr (M == 4) return v + dpp_mov<0x1b>(dpp_mov<0x141>(v));  // i ^ 7, then i ^ 3
-  if constexpr (M == 8) return v + dpp_mov<0x128>(v);                 // row_ror 8
+__device__ __forceinline__ void xor_pair(double v, double& a, double& b) {
+  a = v;
+  if constexpr (M == 1) b = dpp_mov<0xb1>(v);                  // quad_perm 1 0 3 2
+  if constexpr (M == 2) b = dpp_mov<0x4e>(v);                  // quad_perm 2 3 0 1
+  if constexpr (M == 4) b = dpp_mov<0x1b>(dpp_mov<0x141>(v));  // i ^ 7, then i ^ 3
+  if constexpr (M == 8) b = dpp_mov<0x128>(v);                 // row_ror 8
   if constexpr (M >= 16) {
-    const int64_t b = __double_as_longlong(v);
+    const int64_t bits = __double_as_longlong(v);
     typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-    const unsigned int l = (unsigned int)b, h = (unsigned int)(b >> 32);
+    const unsigned int l = (unsigned int)bits, h = (unsigned int)(bits >> 32);
     u2 sl, sh;
     if constexpr (M == 16) {
       sl = __builtin_amdgcn_permlane16_swap(l, l, false, false);
@@ -160,10 +163,15 @@ __device__ __forceinline__ double xor_add(double v) {
       sl = __builtin_amdgcn_permlane32_swap(l, l, false, false);
       sh = __builtin_amdgcn_permlane32_swap(h, h, false, false);
     }
-    const double a = __longlong_as_double(((int64_t)sh.x << 32) | sl.x);
-    const double c = __longlong_as_double(((int64_t)sh.y << 32) | sl.y);
-    return a + c;
+    a = __longlong_as_double(((int64_t)sh.x << 32) | sl.x);
+    b = __longlong_as_double(((int64_t)sh.y << 32) | sl.y);
   }
+}
+template <int M>
+__device__ __forceinline__ double xor_add(double v) {
+  double a, b;
+  xor_pair<M>(v, a, b);
+  return a + b;
 }
 
 // Sum of a double over the 64 lanes by the xor butterfly m = 32..1; every

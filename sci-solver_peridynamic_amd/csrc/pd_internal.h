@@ -454,18 +454,20 @@ struct ContactPlan {
 // the bounding boxes of bodies 0 .. nbody - 1: out[b * 6 + k] (lo xyz, hi
 // xyz; +inf / -inf for bodies without particles); part holds
 // 1024 * PD_MAX_BODIES * 6
-// plan non-null: the contact plan of the boxes too, zones widened by w
+// plan non-null: the contact plan of the boxes too, zones widened by w, there
+// and in hplan (host memory)
 void launch_bbox_bodies(const double4* x, const int32_t* body, int32_t n, int32_t nbody,
                         double* part, double* out, hipStream_t s,
-                        ContactPlan* plan = nullptr, double w = 0.0);
+                        ContactPlan* plan = nullptr, ContactPlan* hplan = nullptr,
+                        double w = 0.0);
 void launch_bbox(const double4* x, const int32_t* body, int32_t n, int32_t body_sel,
                  double* part, double* out6, hipStream_t s);
-// stable (ascending) list of contact candidates; the count lands in
-// tile_cnt[zone_tile_words(n) - 1]
+// stable (ascending) list of contact candidates; the count lands in *total
+// (host memory)
 // (fc non-null: every particle's contact force is cleared on the way)
 void launch_zone_select(const double4* x, const int32_t* body, int32_t n,
                         const ZoneBoxes* z, uint32_t* tile_cnt, int32_t* out,
-                        hipStream_t s, double4* fc = nullptr);
+                        uint32_t* total, hipStream_t s, double4* fc = nullptr);
 
 size_t zone_tile_words(int32_t n);
 // keys of the cells (sub-grid origin cell c0, dims) of particles subset[i]
