@@ -229,6 +229,23 @@ __device__ __forceinline__ double chain_add(double acc, const double* t, int n) 
   return acc;
 }
 
+// tile_sum of N quantities, one exchange; lds: [4 N], not to be reused before
+// the next barrier.
+template <int N>
+__device__ __forceinline__ void tile_sums(double (&v)[N], double* lds) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = wave_sum(v[k]);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) lds[4 * k + w] = v[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    v[k] = (lds[4 * k] + lds[4 * k + 1]) + (lds[4 * k + 2] + lds[4 * k + 3]);
+}
+
 // Final fold of one quantity over the tiles by one 256-thread workgroup:
 // thread t sums part[t], part[t + 256], ... left to right from 0.0, then
 // tile_sum (the oracle's final_combine).
@@ -251,17 +268,10 @@ __device__ __forceinline__ double fold_partials(const double* part, int ntiles, 
 // Two quantities at once, one exchange.
 __device__ __forceinline__ void fold_pair(const double* part0, const double* part1, int ntiles,
                                           double* lds8, double& s0, double& s1) {
-  double v0 = fold_strided(part0, ntiles), v1 = fold_strided(part1, ntiles);
-  v0 = wave_sum(v0);
-  v1 = wave_sum(v1);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    lds8[w] = v0;
-    lds8[4 + w] = v1;
-  }
-  __syncthreads();
-  s0 = (lds8[0] + lds8[1]) + (lds8[2] + lds8[3]);
-  s1 = (lds8[4] + lds8[5]) + (lds8[6] + lds8[7]);
+  double v[2] = {fold_strided(part0, ntiles), fold_strided(part1, ntiles)};
+  tile_sums(v, lds8);
+  s0 = v[0];
+  s1 = v[1];
 }
 
 // The same over tiles t0 .. t0 + nt whose four slices' sums (wave_sum over 64

@@ -50,14 +50,14 @@ __device__ __forceinline__ void gather_asm(const AsmArgs& a, int q, double4& xq,
 // the quotients by the float-rounded length (bond_dir), by the reference
 // length (dij / d0, c / d0), by the current length (d0 / dij) and by the
 // radius (the volume scale) share reciprocals and the square root is
-// sqrt_rcp; both variants are launched and the one that does not match bit 0
-// of the range flag (k_asm_prep) returns at once.  The SHARED variant sets
+// sqrt_rcp; bit 0 of the range flag (k_asm_prep) tells which of the two
+// runs, in one kernel (the general form fits in the common one's registers; a
+// launch of its own, which returned at once, took 4.8 us a step).  SHARED sets
 // bit 1 when a live bond is no longer than SMALL (the matrix-free products
 // then leave the shared forms).
 // FUSE and GAP: a.fuse and a.track_gap as compile-time choices.
 template <bool MIXED, bool SHARED, bool FUSE, bool GAP>
-__global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
-  if (((a.counters->range_bad & 1u) == 0) != SHARED) return;
+__device__ __forceinline__ void assemble_tile(AsmArgs a, double* lds) {
   if (a.consts) {
     a.dt = a.consts->dt;
     a.dt2 = a.consts->dt2;
@@ -161,23 +161,36 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     // the sequential pass below takes over at that trip's first slot, with
     // the sums of the slots before it -- those of the sequential pass, which
     // reaches that slot with the same bonds in the same order.
-    // At 10^6 rows of 112 bonds, two / three / four / five slots per trip:
-    // 0.89 / 0.82 / 0.79 / 0.82 ms (0.84 before the reciprocals came from the
-    // square root); four take 168 registers, three waves per SIMD.
+    // The next trip's columns and lengths are loaded a trip ahead.  Three /
+    // four / five slots per trip, us: 64 / 61 / 60 at 28k rows of 106 bonds,
+    // 80 / 76 / 76 at 66k, 867 / 801 / 801 at 10^6 (four without the loads
+    // ahead: 69, 81 and 815; three waves per SIMD instead of two do not
+    // make up for them).
     constexpr int OPT = SHARED ? 4 : 0;
     if constexpr (OPT > 0) {
       bool brk = false;
+      int qn[OPT];
+      double ln[OPT];
+      auto fetch = [&](int at) {
+#pragma unroll
+        for (int k = 0; k < OPT; ++k) {
+          qn[k] = ntl(a.col + (base + at + k) * 64 + lane);
+          ln[k] = ntl(a.d0 + (base + at + k) * 64 + lane);
+        }
+      };
+      if (OPT - 1 <= top) fetch(0);
       for (; bnd + OPT - 1 <= top; bnd += OPT) {
         int qv[OPT];
         double lv[OPT], sv[OPT];
         double4 xv[OPT], uv[OPT];
 #pragma unroll
         for (int k = 0; k < OPT; ++k) {
-          qv[k] = ntl(a.col + (base + bnd + k) * 64 + lane);
-          lv[k] = ntl(a.d0 + (base + bnd + k) * 64 + lane);
+          qv[k] = qn[k];
+          lv[k] = ln[k];
         }
 #pragma unroll
         for (int k = 0; k < OPT; ++k) gather_asm<FUSE>(a, qv[k], xv[k], sv[k], uv[k]);
+        if (bnd + 2 * OPT - 1 <= top) fetch(bnd + OPT);
         // every load before the arithmetic (1.02 ms without at 10^6 rows and
         // three slots, 0.82 with)
         __builtin_amdgcn_sched_barrier(0);
@@ -438,28 +451,22 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
     }
   }
   if constexpr (FUSE) {  // the start kernel's tile partials, all threads
-    __shared__ double lds4[4];
-    const int ntiles = gridDim.x;
+    constexpr int NV = MIXED ? 4 : 3;
+    double v[NV];
     if constexpr (MIXED) {
-      const double v0 = tile_sum(t_rr, lds4);
-      const double v1 = tile_sum(t_rz, lds4);
-      const double v2 = tile_sum(t_r32, lds4);
-      const double v3 = tile_sum(t_bb, lds4);
-      if (threadIdx.x == 0) {
-        a.part[tile] = v0;
-        a.part[ntiles + tile] = v1;
-        a.part[2 * (int64_t)ntiles + tile] = v2;
-        a.part[3 * (int64_t)ntiles + tile] = v3;
-      }
+      v[0] = t_rr;
+      v[1] = t_rz;
+      v[2] = t_r32;
+      v[3] = t_bb;
     } else {
-      const double v0 = tile_sum(t_rz, lds4);
-      const double v1 = tile_sum(t_rr, lds4);
-      const double v2 = tile_sum(t_bb, lds4);
-      if (threadIdx.x == 0) {
-        a.part[tile] = v0;
-        a.part[ntiles + tile] = v1;
-        a.part[2 * (int64_t)ntiles + tile] = v2;
-      }
+      v[0] = t_rz;
+      v[1] = t_rr;
+      v[2] = t_bb;
+    }
+    tile_sums(v, lds);
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) a.part[k * (int64_t)gridDim.x + tile] = v[k];
     }
   }
   // integer counters: order-free
@@ -477,12 +484,18 @@ __global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
 }
 
 template <bool MIXED, bool FUSE, bool GAP>
+__global__ __launch_bounds__(PD_BLOCK) void k_assemble(AsmArgs a) {
+  __shared__ double lds[16];
+  if ((a.counters->range_bad & 1u) == 0)  // uniform over the grid
+    assemble_tile<MIXED, true, FUSE, GAP>(a, lds);
+  else
+    assemble_tile<MIXED, false, FUSE, GAP>(a, lds);
+}
+
+template <bool MIXED, bool FUSE, bool GAP>
 void launch_assemble_t(const AsmArgs& a, int nb, hipStream_t s) {
-  // both variants; the one the range flag does not select returns at once
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_assemble<MIXED, true, FUSE, GAP>), dim3(nb), dim3(PD_BLOCK),
-                     0, s, a);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_assemble<MIXED, false, FUSE, GAP>), dim3(nb), dim3(PD_BLOCK),
-                     0, s, a);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_assemble<MIXED, FUSE, GAP>), dim3(nb), dim3(PD_BLOCK), 0, s,
+                     a);
 }
 
 void launch_assemble(const AsmArgs& a, hipStream_t s) {
@@ -1221,7 +1234,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_write_blocks(SpmvView A, double* v
 // k_cg_dir, which reads p anyway.  The specimen's first workgroup records
 // alpha and that the update of iteration `it` ran.
 __global__ __launch_bounds__(PD_BLOCK) void k_cg_update(CgArgs a, int it) {
-  __shared__ double lds4[4];
+  __shared__ double lds4[4], lds8[8];
   const int ntiles = gridDim.x;
   const int tile = xcd_tile(blockIdx.x, ntiles);
   const int s = spec_of(a.batch, tile);
@@ -1274,11 +1287,11 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_update(CgArgs a, int it) {
     t_rz = term3(rr.x, rr.y, rr.z, z0, z1, z2);
     t_rr = term3(rr.x, rr.y, rr.z, rr.x, rr.y, rr.z);
   }
-  const double v0 = tile_sum(t_rz, lds4);
-  const double v1 = tile_sum(t_rr, lds4);
+  double v[2] = {t_rz, t_rr};
+  tile_sums(v, lds8);
   if (threadIdx.x == 0) {
-    a.part[2 * (int64_t)ntiles + tile] = v0;
-    a.part[3 * (int64_t)ntiles + tile] = v1;
+    a.part[2 * (int64_t)ntiles + tile] = v[0];
+    a.part[3 * (int64_t)ntiles + tile] = v[1];
   }
 }
 
