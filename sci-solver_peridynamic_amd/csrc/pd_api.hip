@@ -195,6 +195,7 @@ struct pd_trainer {
   int64_t count = 0;
   float *p = nullptr, *m = nullptr, *v = nullptr;  // parameters, Adam moments
   __bf16* w = nullptr;
+  __bf16* wt = nullptr;  // W2 and W3 by columns
   float* partial = nullptr;
   int32_t partial_waves = 0;
   float* loss = nullptr;
@@ -2387,7 +2388,7 @@ int pd_learned_set(pd_ctx* c, const float* params, int32_t count) {
   }
   HIPCHK(c, hipMemcpyAsync(c->pc_p, params, sizeof(float) * PC_NPARAM, hipMemcpyHostToDevice,
                            c->stream));
-  pd::launch_pc_to_bf16(c->pc_p, c->pc_w, c->stream);
+  pd::launch_pc_to_bf16(c->pc_p, c->pc_w, nullptr, c->stream);
   CHECK_LAUNCH(c, "bf16 weights");
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->pc_loaded = true;
@@ -2499,7 +2500,8 @@ int pd_trainer_create(int32_t device, int64_t capacity, uint64_t seed, pd_traine
       hipMalloc((void**)&t->p, sizeof(float) * PC_NPARAM) != hipSuccess ||
       hipMalloc((void**)&t->m, sizeof(float) * PC_NWEIGHT) != hipSuccess ||
       hipMalloc((void**)&t->v, sizeof(float) * PC_NWEIGHT) != hipSuccess ||
-      hipMalloc((void**)&t->w, sizeof(__bf16) * PC_NWEIGHT) != hipSuccess)
+      hipMalloc((void**)&t->w, sizeof(__bf16) * PC_NWEIGHT) != hipSuccess ||
+      hipMalloc((void**)&t->wt, sizeof(__bf16) * PC_NWT) != hipSuccess)
     return bail(tfail(t, PD_ERR_HIP, "hipMalloc failed"));
   // He-uniform weights from a seeded splitmix64, zero biases, a small last
   // layer (S starts near I: block Jacobi), eps 1e-3
@@ -2526,7 +2528,7 @@ int pd_trainer_create(int32_t device, int64_t capacity, uint64_t seed, pd_traine
       hipMemset(t->m, 0, sizeof(float) * PC_NWEIGHT) != hipSuccess ||
       hipMemset(t->v, 0, sizeof(float) * PC_NWEIGHT) != hipSuccess)
     return bail(tfail(t, PD_ERR_HIP, "trainer initialisation failed"));
-  pd::launch_pc_to_bf16(t->p, t->w, t->stream);
+  pd::launch_pc_to_bf16(t->p, t->w, t->wt, t->stream);
   if (hipStreamSynchronize(t->stream) != hipSuccess)
     return bail(tfail(t, PD_ERR_HIP, "trainer initialisation failed"));
   *out = t;
@@ -2537,7 +2539,7 @@ int pd_trainer_destroy(pd_trainer* t) {
   if (!t) return PD_OK;
   (void)hipSetDevice(t->device);
   if (t->stream) (void)hipStreamSynchronize(t->stream);
-  for (void* q : {(void*)t->samples, (void*)t->p, (void*)t->m, (void*)t->v, (void*)t->w,
+  for (void* q : {(void*)t->samples, (void*)t->p, (void*)t->m, (void*)t->v, (void*)t->w, (void*)t->wt,
                   (void*)t->partial, (void*)t->loss})
     if (q) (void)hipFree(q);
   if (t->stream) (void)hipStreamDestroy(t->stream);
@@ -2627,10 +2629,11 @@ int run_fit(pd_trainer* t, int32_t steps, int32_t batch, float lr, uint64_t seed
     a.seed = seed;
     a.step = t->steps_done;
     a.w = t->w;
+    a.wt = t->wt;
     a.p = t->p;
     a.partial = partial;
     pd::launch_pc_train(a, t->stream);
-    pd::launch_pc_adam(partial, waves, t->p, t->m, t->v, t->w, t->steps_done, lr, loss + k,
+    pd::launch_pc_adam(partial, waves, t->p, t->m, t->v, t->w, t->wt, t->steps_done, lr, loss + k,
                        t->stream);
     ++t->steps_done;
   }

@@ -261,6 +261,7 @@ void launch_small_undo(int32_t n, const double* arec, double4* x, hipStream_t s)
 #define PC_OFF_EPS (PC_OFF_ISTD + PC_NIN)
 #define PC_NPARAM (PC_OFF_EPS + 1)
 #define PC_NWEIGHT PC_OFF_MEAN  // trainable entries (weights and biases)
+#define PC_NWT (PC_NH * PC_NH + PC_NOUT * PC_NH)  // W2 and W3 by columns
 
 struct PcNet {
   const __bf16* w;     // [PC_NWEIGHT] bf16 copy (biases unused in this copy)
@@ -332,15 +333,18 @@ struct PcTrainArgs {
   int32_t batch;  // multiple of 32
   uint64_t seed;
   int32_t step;
-  const __bf16* w;  // bf16 weights
-  const float* p;   // FP32 parameters (biases, normalisation, eps)
+  const __bf16* w;   // bf16 weights
+  const __bf16* wt;  // [PC_NWT] W2, then W3, by columns
+  const float* p;    // FP32 parameters (biases, normalisation, eps)
   float* partial;   // [batch / 32][PC_NWEIGHT + 1] per-wave gradients + loss
 };
 void launch_pc_train(const PcTrainArgs& a, hipStream_t s);
 // fold the partial gradients, Adam update of p (weights and biases), refresh w
 void launch_pc_adam(const float* partial, int32_t nwaves, float* p, float* m, float* v,
-                    __bf16* w, int32_t step, float lr, float* loss_out, hipStream_t s);
-void launch_pc_to_bf16(const float* p, __bf16* w, hipStream_t s);
+                    __bf16* w, __bf16* wt, int32_t step, float lr, float* loss_out,
+                    hipStream_t s);
+// wt: null, or the trainer's copy by columns
+void launch_pc_to_bf16(const float* p, __bf16* w, __bf16* wt, hipStream_t s);
 // per-feature mean and 1/std over the samples' raw features into p
 void launch_pc_norm(const float* samples, int64_t nsamples, float* p, hipStream_t s);
 

@@ -27,6 +27,7 @@ namespace pd {
 
 namespace {
 
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
@@ -199,22 +200,62 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_features(PcFeatArgs a) {
 
 // One wave evaluates the MLP for 32 rows (its part of a 128-row tile); the
 // outputs land in outs[w][row][0..7].  hs is the wave's activation tile.
-__device__ __forceinline__ void mlp_forward(const bf16x8& x, const __bf16* w, const float* P,
+// The lane's share of the network: issued together ahead of the first
+// layer, since a load behind one of the layers' barriers waits its whole
+// latency there (weights that another kernel has just written come from
+// beyond the L2, about 1 us each time).
+struct Layers {
+  bf16x8 w1[2], w2[4][2], w3[4];
+  float b1[2], b2[2], b3;
+};
+__device__ __forceinline__ Layers load_layers(const __bf16* w, const float* P) {
+  const int l = threadIdx.x & 63;
+  const int r = l & 31, kh = l >> 5;
+  Layers n;
+  // 16-byte loads: every operand row starts on a multiple of 8 elements
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    n.w1[nt] = *(const bf16x8*)(w + PC_OFF_W1 + (nt * 32 + r) * PC_NIN + 8 * kh);
+    n.b1[nt] = P[PC_OFF_B1 + nt * 32 + r];
+    n.b2[nt] = P[PC_OFF_B2 + nt * 32 + r];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      n.w2[ks][nt] =
+          *(const bf16x8*)(w + PC_OFF_W2 + (nt * 32 + r) * PC_NH + ks * 16 + 8 * kh);
+  }
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) n.w3[ks][i] = (__bf16)0.0f;
+    if (r < PC_NOUT) n.w3[ks] = *(const bf16x8*)(w + PC_OFF_W3 + r * PC_NH + ks * 16 + 8 * kh);
+  }
+  n.b3 = r < PC_NOUT ? P[PC_OFF_B3 + r] : 0.0f;
+  return n;
+}
+
+// h1T, h2T (trainer): the activations by feature too.
+constexpr int kT = 32 + 8;  // LDS row of a feature over a chunk's 32 samples
+typedef __bf16 FeatureRow[kT];
+__device__ __forceinline__ void mlp_forward(const bf16x8& x, const Layers& n,
                                             __bf16 (*h1)[kH], __bf16 (*h2)[kH],
-                                            float (*outs)[PC_NOUT]) {
+                                            float (*outs)[PC_NOUT], FeatureRow* h1T = nullptr,
+                                            FeatureRow* h2T = nullptr) {
   const int l = threadIdx.x & 63;
   const int r = l & 31, kh = l >> 5;
   // layer 1: K = 16
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
-    // 16-byte loads: every operand row starts on a multiple of 8 elements
-    const bf16x8 b = *(const bf16x8*)(w + PC_OFF_W1 + (nt * 32 + r) * PC_NIN + 8 * kh);
-    const floatx16 c = mfma(x, b, zero16());
+    const floatx16 c = mfma(x, n.w1[nt], zero16());
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int col = nt * 32 + r;
-      const float v = c[j] + P[PC_OFF_B1 + col];
-      h1[crow(j, kh)][col] = (__bf16)(v > 0.0f ? v : 0.0f);
+    for (int q = 0; q < 4; ++q) {
+      bf16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float v = c[4 * q + i] + n.b1[nt];
+        o[i] = (__bf16)(v > 0.0f ? v : 0.0f);
+        h1[crow(4 * q + i, kh)][nt * 32 + r] = o[i];
+      }
+      if (h1T) *(bf16x4*)&h1T[nt * 32 + r][8 * q + 4 * kh] = o;
     }
   }
   __syncthreads();
@@ -223,17 +264,25 @@ __device__ __forceinline__ void mlp_forward(const bf16x8& x, const __bf16* w, co
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     const bf16x8 av = *(const bf16x8*)&h1[r][ks * 16 + 8 * kh];
-    const bf16x8 b0 = *(const bf16x8*)(w + PC_OFF_W2 + r * PC_NH + ks * 16 + 8 * kh);
-    const bf16x8 b1 = *(const bf16x8*)(w + PC_OFF_W2 + (32 + r) * PC_NH + ks * 16 + 8 * kh);
-    c0 = mfma(av, b0, c0);
-    c1 = mfma(av, b1, c1);
+    c0 = mfma(av, n.w2[ks][0], c0);
+    c1 = mfma(av, n.w2[ks][1], c1);
   }
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const float v0 = c0[j] + P[PC_OFF_B2 + r];
-    const float v1 = c1[j] + P[PC_OFF_B2 + 32 + r];
-    h2[crow(j, kh)][r] = (__bf16)(v0 > 0.0f ? v0 : 0.0f);
-    h2[crow(j, kh)][32 + r] = (__bf16)(v1 > 0.0f ? v1 : 0.0f);
+  for (int q = 0; q < 4; ++q) {
+    bf16x4 o0, o1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float v0 = c0[4 * q + i] + n.b2[0];
+      const float v1 = c1[4 * q + i] + n.b2[1];
+      o0[i] = (__bf16)(v0 > 0.0f ? v0 : 0.0f);
+      o1[i] = (__bf16)(v1 > 0.0f ? v1 : 0.0f);
+      h2[crow(4 * q + i, kh)][r] = o0[i];
+      h2[crow(4 * q + i, kh)][32 + r] = o1[i];
+    }
+    if (h2T) {
+      *(bf16x4*)&h2T[r][8 * q + 4 * kh] = o0;
+      *(bf16x4*)&h2T[32 + r][8 * q + 4 * kh] = o1;
+    }
   }
   __syncthreads();
   // layer 3: N = 8 (of a 32-wide tile), K = 64
@@ -241,15 +290,11 @@ __device__ __forceinline__ void mlp_forward(const bf16x8& x, const __bf16* w, co
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) {
     const bf16x8 av = *(const bf16x8*)&h2[r][ks * 16 + 8 * kh];
-    bf16x8 bv;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) bv[i] = (__bf16)0.0f;
-    if (r < PC_NOUT) bv = *(const bf16x8*)(w + PC_OFF_W3 + r * PC_NH + ks * 16 + 8 * kh);
-    c3 = mfma(av, bv, c3);
+    c3 = mfma(av, n.w3[ks], c3);
   }
   if (r < PC_NOUT) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j) outs[crow(j, kh)][r] = c3[j] + P[PC_OFF_B3 + r];
+    for (int j = 0; j < 16; ++j) outs[crow(j, kh)][r] = c3[j] + n.b3;
   }
   __syncthreads();
 }
@@ -310,8 +355,9 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_infer(int n, const float* feat,
   // the lane's eight features straight from memory (a row past the end
   // reads the last row; its outputs are dropped below)
   const int pr = row0 + r < n ? row0 + r : n - 1;
+  const Layers net_l = load_layers(net.w, P);
   const bf16x8 x = load_x(feat + (int64_t)pr * PC_NIN, P);
-  mlp_forward(x, net.w, P, h1[w], h2[w], outs[w]);
+  mlp_forward(x, net_l, h1[w], h2[w], outs[w]);
   if (l >= 32) return;
   const int p = row0 + l;
   if (p >= n || act[p] == PD_INVISIBLE) return;
@@ -339,11 +385,12 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_infer_start(PcInferStartArgs a)
   const int row0 = tile * PD_BLOCK + w * 64;
   const int n = a.n;
   const float* P = a.net.p;
+  const Layers net_l = load_layers(a.net.w, P);
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     const int pr = row0 + 32 * half + r < n ? row0 + 32 * half + r : n - 1;
     const bf16x8 x = load_x(a.feat + (int64_t)pr * PC_NIN, P);
-    mlp_forward(x, a.net.w, P, h1[w], h2[w], outs[w] + 32 * half);
+    mlp_forward(x, net_l, h1[w], h2[w], outs[w] + 32 * half);
   }
   const int p = row0 + l;
   double t = 0.0;
@@ -472,40 +519,89 @@ __device__ void sample_grad(const float* o, const float* smp, float eps, float* 
   dout[5] = cl[2] ? 0.0f : GL[2][2] * Lc[5];
 }
 
-// C tile (32x32) of A^T-style products from LDS: A[i][k] = src_a(k, i), etc.
 // Forward, loss, backward of one 32-sample chunk per wave; per-wave
 // gradients (and the loss sum) go to partial[global wave].
-__global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
-  __shared__ __bf16 xs[4][32][PC_NIN + kPad];
-  __shared__ __bf16 h1[4][32][kH];
-  __shared__ __bf16 h2[4][32][kH];
-  __shared__ __bf16 g[4][32][kH];  // dH2, then dH1
-  __shared__ float outs[4][32][PC_NOUT];
-  __shared__ float smp[4][32][PC_SAMPLE];
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+// One wave per workgroup: 256 chunks reach 256 CUs, and a chunk has an LDS to
+// itself.  Bound by the latency of its one chain, so whatever can be is under
+// way early (the samples' gather, then every weight, W2 and W3 by columns from
+// their transposed copy wt), and every matrix operand that runs over the
+// samples is read 16 bytes at a time from activations kept in LDS by feature
+// as well (C tiles hold four consecutive samples per register quad, so those
+// copies cost a quarter of the stores): 13.8 us per step of 8192 samples, 18.5
+// with operands gathered two bytes at a time, four waves a workgroup.
+// Four samples (rows 8 q + 4 kh ..) of feature f into its row.
+__device__ __forceinline__ void put4(__bf16 (*t)[kT], int f, int q, int kh, const float v[4]) {
+  bf16x4 o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = (__bf16)v[i];
+  *(bf16x4*)&t[f][8 * q + 4 * kh] = o;
+}
+// Sum over the chunk's samples of feature f, in order.
+__device__ __forceinline__ float row_sum(const __bf16 (*t)[kT], int f) {
+  float s = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const bf16x8 v = *(const bf16x8*)&t[f][8 * q];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s += (float)v[i];
+  }
+  return s;
+}
+
+__global__ __launch_bounds__(64) void k_pc_train(PcTrainArgs a) {
+  __shared__ __attribute__((aligned(16))) __bf16 xT[PC_NIN][kT];
+  __shared__ __attribute__((aligned(16))) __bf16 h1[32][kH], h1T[PC_NH][kT];
+  __shared__ __attribute__((aligned(16))) __bf16 h2[32][kH], h2T[PC_NH][kT];
+  __shared__ __attribute__((aligned(16))) __bf16 g[32][kH], gT[PC_NH][kT];  // dH2, then dH1
+  __shared__ __attribute__((aligned(16))) float outs[32][PC_NOUT], dOT[PC_NOUT][32 + 4];
+  __shared__ __attribute__((aligned(16))) float smp[32][PC_SAMPLE];
+  const int l = threadIdx.x;
   const int r = l & 31, kh = l >> 5;
-  const int gw = blockIdx.x * 4 + w;
+  const int gw = blockIdx.x;
   const float* P = a.p;
   // draw the samples (with replacement)
+  static_assert(PC_SAMPLE % 4 == 0, "a sample is read 16 bytes at a time");
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  f4 drawn[PC_SAMPLE / 8 + 1];
   {
     const uint64_t h = mix64(a.seed ^ mix64((uint64_t)a.step * 0x100000001B3ull + gw * 32 + r));
     const int64_t idx = (int64_t)(h % (uint64_t)a.nsamples);
-    const float* src = a.samples + idx * PC_SAMPLE;
-    for (int k = kh; k < PC_SAMPLE; k += 2) smp[w][r][k] = src[k];
-  }
-  __syncthreads();
-  const bf16x8 x = load_x(smp[w][r], P);
+    const f4* src = (const f4*)(a.samples + idx * PC_SAMPLE);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) xs[w][r][8 * kh + i] = x[i];
-  mlp_forward(x, a.w, P, h1[w], h2[w], outs[w]);
+    for (int k = 0; k < PC_SAMPLE / 8 + 1; ++k)
+      if (2 * k + kh < PC_SAMPLE / 4) drawn[k] = src[2 * k + kh];
+  }
+  // the weights, for the backward pass too
+  const Layers net = load_layers(a.w, P);
+  const float eps = P[PC_OFF_EPS];
+  bf16x8 w2a[4], w2b[4], w3a, w3b;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    w2a[ks] = *(const bf16x8*)(a.wt + r * PC_NH + ks * 16 + 8 * kh);
+    w2b[ks] = *(const bf16x8*)(a.wt + (32 + r) * PC_NH + ks * 16 + 8 * kh);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) w3a[i] = w3b[i] = (__bf16)0.0f;
+  if (kh == 0) {  // output index < 8
+    w3a = *(const bf16x8*)(a.wt + PC_NH * PC_NH + r * PC_NOUT);
+    w3b = *(const bf16x8*)(a.wt + PC_NH * PC_NH + (32 + r) * PC_NOUT);
+  }
+#pragma unroll
+  for (int k = 0; k < PC_SAMPLE / 8 + 1; ++k)
+    if (2 * k + kh < PC_SAMPLE / 4) *(f4*)&smp[r][4 * (2 * k + kh)] = drawn[k];
+  __syncthreads();
+  const bf16x8 x = load_x(smp[r], P);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) xT[8 * kh + i][r] = x[i];
+  mlp_forward(x, net, h1, h2, outs, h1T, h2T);
   // loss and output gradients (lanes 0..31, one sample each)
   const float scale = 1.0f / (3.0f * (float)a.batch);
   float loss = 0.0f;
   if (l < 32) {
     float o[PC_NOUT], dout[PC_NOUT];
-    for (int k = 0; k < PC_NOUT; ++k) o[k] = outs[w][l][k];
-    sample_grad(o, smp[w][l], P[PC_OFF_EPS], dout, loss);
-    for (int k = 0; k < PC_NOUT; ++k) outs[w][l][k] = dout[k] * scale;
+    for (int k = 0; k < PC_NOUT; ++k) o[k] = outs[l][k];
+    sample_grad(o, smp[l], eps, dout, loss);
+    for (int k = 0; k < PC_NOUT; ++k) outs[l][k] = dOT[k][l] = dout[k] * scale;
   }
   __syncthreads();
   float* part = a.partial + (int64_t)gw * (PC_NWEIGHT + 1);
@@ -514,16 +610,13 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
     floatx16 c0 = zero16(), c1 = zero16();
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      bf16x8 av, b0, b1;
+      bf16x8 av;
+      const int k0 = ks * 16 + 8 * kh;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int k = ks * 16 + 8 * kh + i;
-        av[i] = r < PC_NOUT ? (__bf16)outs[w][k][r] : (__bf16)0.0f;
-        b0[i] = h2[w][k][r];
-        b1[i] = h2[w][k][32 + r];
-      }
-      c0 = mfma(av, b0, c0);
-      c1 = mfma(av, b1, c1);
+      for (int i = 0; i < 8; ++i)
+        av[i] = r < PC_NOUT ? (__bf16)dOT[r % PC_NOUT][k0 + i] : (__bf16)0.0f;
+      c0 = mfma(av, *(const bf16x8*)&h2T[r][k0], c0);
+      c1 = mfma(av, *(const bf16x8*)&h2T[32 + r][k0], c1);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {  // rows 4 kh + j < 8
@@ -533,28 +626,33 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
     }
     if (l < PC_NOUT) {
       float s = 0.0f;
-      for (int k = 0; k < 32; ++k) s += outs[w][k][l];
+#pragma unroll
+      for (int k = 0; k < 32; ++k) s += dOT[l][k];
       part[PC_OFF_B3 + l] = s;
     }
   }
   // dH2 = dO W3, masked by H2 > 0
   {
-    floatx16 c0 = zero16(), c1 = zero16();
-    bf16x8 av, b0, b1;
+    bf16x8 av;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = 8 * kh + i;  // output index, < 8 only for kh = 0
-      av[i] = k < PC_NOUT ? (__bf16)outs[w][r][k] : (__bf16)0.0f;
-      b0[i] = k < PC_NOUT ? a.w[PC_OFF_W3 + k * PC_NH + r] : (__bf16)0.0f;
-      b1[i] = k < PC_NOUT ? a.w[PC_OFF_W3 + k * PC_NH + 32 + r] : (__bf16)0.0f;
-    }
-    c0 = mfma(av, b0, c0);
-    c1 = mfma(av, b1, c1);
+    for (int i = 0; i < 8; ++i)  // output index 8 kh + i, < 8 only for kh = 0
+      av[i] = kh == 0 ? (__bf16)outs[r][i] : (__bf16)0.0f;
+    const floatx16 c0 = mfma(av, w3a, zero16()), c1 = mfma(av, w3b, zero16());
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int row = crow(j, kh);
-      g[w][row][r] = (float)h2[w][row][r] > 0.0f ? (__bf16)c0[j] : (__bf16)0.0f;
-      g[w][row][32 + r] = (float)h2[w][row][32 + r] > 0.0f ? (__bf16)c1[j] : (__bf16)0.0f;
+    for (int q = 0; q < 4; ++q) {
+      const bf16x4 m0 = *(const bf16x4*)&h2T[r][8 * q + 4 * kh];
+      const bf16x4 m1 = *(const bf16x4*)&h2T[32 + r][8 * q + 4 * kh];
+      float v0[4], v1[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = crow(4 * q + i, kh);
+        v0[i] = (float)m0[i] > 0.0f ? c0[4 * q + i] : 0.0f;
+        v1[i] = (float)m1[i] > 0.0f ? c1[4 * q + i] : 0.0f;
+        g[row][r] = (__bf16)v0[i];
+        g[row][32 + r] = (__bf16)v1[i];
+      }
+      put4(gT, r, q, kh, v0);
+      put4(gT, 32 + r, q, kh, v1);
     }
   }
   __syncthreads();
@@ -562,50 +660,40 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
   floatx16 d1a = zero16(), d1b = zero16();
   {
 #pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      const bf16x8 av = *(const bf16x8*)&g[r][ks * 16 + 8 * kh];
+      d1a = mfma(av, w2a[ks], d1a);
+      d1b = mfma(av, w2b[ks], d1b);
+    }
+#pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) {
         floatx16 c = zero16();
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-          bf16x8 av, bv;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const int k = ks * 16 + 8 * kh + i;
-            av[i] = g[w][k][mt * 32 + r];
-            bv[i] = h1[w][k][nt * 32 + r];
-          }
-          c = mfma(av, bv, c);
+          const int k0 = ks * 16 + 8 * kh;
+          c = mfma(*(const bf16x8*)&gT[mt * 32 + r][k0], *(const bf16x8*)&h1T[nt * 32 + r][k0], c);
         }
 #pragma unroll
         for (int j = 0; j < 16; ++j)
           part[PC_OFF_W2 + (mt * 32 + crow(j, kh)) * PC_NH + nt * 32 + r] = c[j];
       }
-    {
-      float s = 0.0f;
-      for (int k = 0; k < 32; ++k) s += (float)g[w][k][l];
-      part[PC_OFF_B2 + l] = s;
-    }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      bf16x8 av, b0, b1;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int k = ks * 16 + 8 * kh + i;  // H2 index
-        av[i] = g[w][r][k];
-        b0[i] = a.w[PC_OFF_W2 + k * PC_NH + r];
-        b1[i] = a.w[PC_OFF_W2 + k * PC_NH + 32 + r];
-      }
-      d1a = mfma(av, b0, d1a);
-      d1b = mfma(av, b1, d1b);
-    }
+    part[PC_OFF_B2 + l] = row_sum(gT, l);
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int row = crow(j, kh);
-    g[w][row][r] = (float)h1[w][row][r] > 0.0f ? (__bf16)d1a[j] : (__bf16)0.0f;
-    g[w][row][32 + r] = (float)h1[w][row][32 + r] > 0.0f ? (__bf16)d1b[j] : (__bf16)0.0f;
+  for (int q = 0; q < 4; ++q) {
+    const bf16x4 m0 = *(const bf16x4*)&h1T[r][8 * q + 4 * kh];
+    const bf16x4 m1 = *(const bf16x4*)&h1T[32 + r][8 * q + 4 * kh];
+    float v0[4], v1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v0[i] = (float)m0[i] > 0.0f ? d1a[4 * q + i] : 0.0f;
+      v1[i] = (float)m1[i] > 0.0f ? d1b[4 * q + i] : 0.0f;
+    }
+    put4(gT, r, q, kh, v0);
+    put4(gT, 32 + r, q, kh, v1);
   }
   __syncthreads();
   // dW1 = dH1^T X, db1
@@ -615,29 +703,39 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
       floatx16 c = zero16();
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        bf16x8 av, bv;
+        const int k0 = ks * 16 + 8 * kh;
+        bf16x8 bv = *(const bf16x8*)&xT[r % PC_NIN][k0];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int k = ks * 16 + 8 * kh + i;
-          av[i] = g[w][k][mt * 32 + r];
-          bv[i] = r < PC_NIN ? xs[w][k][r] : (__bf16)0.0f;
-        }
-        c = mfma(av, bv, c);
+        for (int i = 0; i < 8; ++i) bv[i] = r < PC_NIN ? bv[i] : (__bf16)0.0f;
+        c = mfma(*(const bf16x8*)&gT[mt * 32 + r][k0], bv, c);
       }
       if (r < PC_NIN) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) part[PC_OFF_W1 + (mt * 32 + crow(j, kh)) * PC_NIN + r] = c[j];
       }
     }
-    float s = 0.0f;
-    for (int k = 0; k < 32; ++k) s += (float)g[w][k][l];
-    part[PC_OFF_B1 + l] = s;
+    part[PC_OFF_B1 + l] = row_sum(gT, l);
   }
   // loss of the wave's samples
   float ls = l < 32 ? loss : 0.0f;
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) ls += __shfl_xor(ls, m, 64);
   if (l == 0) part[PC_NWEIGHT] = ls;
+}
+
+// A weight's bf16 copies: w in the parameters' order, wt (trainer) with W2 and
+// W3 by columns.
+__device__ __forceinline__ void put_weight(__bf16* w, __bf16* wt, int i, float v) {
+  const __bf16 b = (__bf16)v;
+  w[i] = b;
+  if (!wt) return;
+  if (i >= PC_OFF_W2 && i < PC_OFF_B2) {
+    const int k = i - PC_OFF_W2;
+    wt[k % PC_NH * PC_NH + k / PC_NH] = b;
+  } else if (i >= PC_OFF_W3 && i < PC_OFF_B3) {
+    const int k = i - PC_OFF_W3;
+    wt[PC_NH * PC_NH + k % PC_NH * PC_NOUT + k / PC_NH] = b;
+  }
 }
 
 // Fold the per-wave gradients in wave order, Adam, bf16 refresh; the last
@@ -648,8 +746,8 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_train(PcTrainArgs a) {
 // the latency of the loads; this takes 7.)
 #define ADAM_COLS 32
 __global__ __launch_bounds__(PD_BLOCK) void k_pc_adam(const float* partial, int nwaves, float* p,
-                                                     float* m, float* v, __bf16* w, int step,
-                                                     float lr, float* loss_out) {
+                                                     float* m, float* v, __bf16* w, __bf16* wt,
+                                                     int step, float lr, float* loss_out) {
   __shared__ float rows[PD_BLOCK][ADAM_COLS + 1];
   constexpr int STEP = PD_BLOCK / ADAM_COLS;  // rows per pass
   const int c = threadIdx.x % ADAM_COLS, r0 = threadIdx.x / ADAM_COLS;
@@ -692,12 +790,12 @@ __global__ __launch_bounds__(PD_BLOCK) void k_pc_adam(const float* partial, int 
   const float vh = vi / (1.0f - powf(b2, t));
   const float pi = p[i] - lr * mh / (sqrtf(vh) + 1e-8f);
   p[i] = pi;
-  w[i] = (__bf16)pi;
+  put_weight(w, wt, i, pi);
 }
 
-__global__ __launch_bounds__(PD_BLOCK) void k_pc_to_bf16(const float* p, __bf16* w) {
+__global__ __launch_bounds__(PD_BLOCK) void k_pc_to_bf16(const float* p, __bf16* w, __bf16* wt) {
   const int i = blockIdx.x * PD_BLOCK + threadIdx.x;
-  if (i < PC_NWEIGHT) w[i] = (__bf16)p[i];
+  if (i < PC_NWEIGHT) put_weight(w, wt, i, p[i]);
 }
 
 // feature means and inverse standard deviations, a workgroup per feature
@@ -754,15 +852,15 @@ void launch_pc_samples(const PcSampleArgs& a, hipStream_t s) {
   if (a.n) hipLaunchKernelGGL(k_pc_samples, dim3(blocks_of(a.n)), dim3(PD_BLOCK), 0, s, a);
 }
 void launch_pc_train(const PcTrainArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_pc_train, dim3(a.batch / 128), dim3(PD_BLOCK), 0, s, a);
+  hipLaunchKernelGGL(k_pc_train, dim3(a.batch / 32), dim3(64), 0, s, a);
 }
 void launch_pc_adam(const float* partial, int32_t nwaves, float* p, float* m, float* v, __bf16* w,
-                    int32_t step, float lr, float* loss_out, hipStream_t s) {
+                    __bf16* wt, int32_t step, float lr, float* loss_out, hipStream_t s) {
   hipLaunchKernelGGL(k_pc_adam, dim3((PC_NWEIGHT + 1 + ADAM_COLS - 1) / ADAM_COLS),
-                     dim3(PD_BLOCK), 0, s, partial, nwaves, p, m, v, w, step, lr, loss_out);
+                     dim3(PD_BLOCK), 0, s, partial, nwaves, p, m, v, w, wt, step, lr, loss_out);
 }
-void launch_pc_to_bf16(const float* p, __bf16* w, hipStream_t s) {
-  hipLaunchKernelGGL(k_pc_to_bf16, dim3(blocks_of(PC_NWEIGHT)), dim3(PD_BLOCK), 0, s, p, w);
+void launch_pc_to_bf16(const float* p, __bf16* w, __bf16* wt, hipStream_t s) {
+  hipLaunchKernelGGL(k_pc_to_bf16, dim3(blocks_of(PC_NWEIGHT)), dim3(PD_BLOCK), 0, s, p, w, wt);
 }
 void launch_pc_norm(const float* samples, int64_t nsamples, float* p, hipStream_t s) {
   hipLaunchKernelGGL(k_pc_norm, dim3(PC_NIN), dim3(PD_BLOCK), 0, s, samples, nsamples, p);
