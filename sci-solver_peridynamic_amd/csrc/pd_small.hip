@@ -137,6 +137,59 @@ __device__ __forceinline__ void fold_units(const double* part, int64_t stride, i
   }
 }
 
+// Two of them side by side.
+__device__ __forceinline__ void chain_add2(double (&acc)[2], const double* t0, const double* t1,
+                                           int n) {
+  double a0 = acc[0], a1 = acc[1];
+  int e = 0;
+  if (n >= 8) {
+    double h0[8], h1[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      h0[u] = t0[u];
+      h1[u] = t1[u];
+    }
+    for (; e + 16 <= n; e += 8) {
+      double k0[8], k1[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        k0[u] = t0[e + 8 + u];
+        k1[u] = t1[e + 8 + u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        a0 += h0[u];
+        a1 += h1[u];
+        h0[u] = k0[u];
+        h1[u] = k1[u];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      a0 += h0[u];
+      a1 += h1[u];
+    }
+    e += 8;
+  }
+  for (; e < n; ++e) {
+    a0 += t0[e];
+    a1 += t1[e];
+  }
+  acc[0] = a0;
+  acc[1] = a1;
+}
+
+// The smallest and the largest over the L lanes of a row.
+template <int L>
+__device__ __forceinline__ void row_extremes(double& lo, double& hi) {
+#pragma unroll
+  for (int m = L / 2; m >= 1; m >>= 1) {
+    const double l = __shfl_xor(lo, m, 64), h = __shfl_xor(hi, m, 64);
+    lo = l < lo ? l : lo;
+    hi = h > hi ? h : hi;
+  }
+}
+
 // chain_add over t[0 .. n), n <= N wave-uniform, in steps of 16 terms with
 // each term read 16 terms ahead (the terms past a list's end hold -0.0,
 // which changes no sum).  An LDS read costs the same with one lane as with
@@ -173,7 +226,11 @@ __device__ __forceinline__ double chain_wide(double acc, const double* t, int n)
 // bonds of the rest of the list are flagged in parallel, one lane walks the
 // flags as the sequential pass walks the list, and the row's lanes apply
 // the permutation.  Bound by latency: a chunk is a column load, a gather and
-// 2 L additions in a row.
+// 2 L additions in a row.  The stretch extremes are kept per lane: as chains of
+// compares through LDS behind the sums they took a third of the kernel (288
+// rows 21.8 -> 12.3 us, 8k 30.2 -> 22.3, 13k 37.3 -> 26.3).  Columns and records
+// loaded a chunk ahead gained nothing (8k rows 13.1 us to the unit's end
+// against 12.1, at 256 registers).
 // ---------------------------------------------------------------------------
 template <int L, bool SHARED>
 __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs& g,
@@ -181,8 +238,9 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
   constexpr int R = Unit<L>::R, K = Unit<L>::K;
   constexpr int CH = 2 * L, CP = CH + 1;  // slots per chunk and its padded stride
   constexpr int ROW = 13 * CP;            // LDS doubles per row
-  constexpr int ROLES = 15;               // 13 sums, the smallest and the largest stretch
-  constexpr int NR = (ROLES + L - 1) / L;
+  constexpr int ROLES = 13;               // sums
+  constexpr int NR = (ROLES + L - 1) / L;  // per lane
+  static_assert(NR <= 2, "two chains side by side at most");
   const int unit = xcd_tile(blockIdx.x, gridDim.x);
   const int s = unit >> K;
   const int i = threadIdx.x / L, j = threadIdx.x % L;  // row of the unit, lane of the row
@@ -206,9 +264,8 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
   const double hr = mt.horizon - mt.radius;
   const double yr = SHARED ? rcp_nr(mt.radius) : 0.0;
   bool short_len = false;
-  double acc[NR];
-#pragma unroll
-  for (int k = 0; k < NR; ++k) acc[k] = j + k * L == 14 ? -INFINITY : 0.0;
+  double acc[2] = {0.0, 0.0};
+  double smin = 0.0, smax = -INFINITY;  // of this lane's bonds
 
   // geometry, stretch and breaking test of slot k (k <= top)
   struct Bond {
@@ -368,26 +425,18 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
       o[10 * CP] = b01 * t.u.x + b11 * t.u.y + b12 * t.u.z;
       o[11 * CP] = b02 * t.u.x + b12 * t.u.y + b22 * t.u.z;
       o[12 * CP] = t.dr;
+      if (c0 + u * L + j <= top) {
+        smin = t.dr < smin ? t.dr : smin;
+        smax = t.dr > smax ? t.dr : smax;
+      }
     }
     wave_fence();
     const int m = min(CH, top + 1 - c0);
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      const int role = j + k * L;
-      if (role < ROLES) {
-        const double* t = tr + min(role, 12) * CP;
-        double v = acc[k];
-        int e = 0;
-        if (role < 13) {
-          v = chain_add(v, t, m);
-        } else if (role == 13) {
-          for (; e < m; ++e) v = t[e] < v ? t[e] : v;
-        } else {
-          for (; e < m; ++e) v = t[e] > v ? t[e] : v;
-        }
-        acc[k] = v;
-      }
-    }
+    // lane j adds terms j and j + L (lanes past the last repeat it)
+    if constexpr (NR == 2)
+      chain_add2(acc, tr + j * CP, tr + min(j + L, ROLES - 1) * CP, m);
+    else
+      acc[0] = chain_add(acc[0], tr + min(j, ROLES - 1) * CP, m);
     wave_fence();
   }
   // the row's sums to the unit's owner lanes (the first R threads)
@@ -396,6 +445,11 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
 #pragma unroll
   for (int k = 0; k < NR; ++k)
     if (j + k * L < ROLES) sum[i * 16 + j + k * L] = acc[k];
+  row_extremes<L>(smin, smax);
+  if (j == 0) {
+    sum[i * 16 + 13] = smin;
+    sum[i * 16 + 14] = smax;
+  }
   int* tops = (int*)(lds + R * 16);  // [R]
   if (j == 0) tops[i] = top;
   const bool zany = __any(short_len);
