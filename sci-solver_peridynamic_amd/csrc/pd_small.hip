@@ -623,7 +623,7 @@ template <int L, int M, int MR, int MC>
 __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g) {
   constexpr int R = Unit<L>::R, K = Unit<L>::K;
   constexpr int CH = MC * L, CP = CH + 3;  // slots per chunk, padded stride
-  __shared__ double T[R * 3 * CP];  // terms
+  __shared__ __attribute__((aligned(16))) double T[R * 3 * CP];  // terms
   __shared__ double Y[3 * R];
   __shared__ double Di[6 * R];  // the rows' diagonal blocks
   __shared__ int longest;
@@ -716,26 +716,41 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
       }
     }
   }
-  // the union of the gathered rows as a bitmap, its ranks the local indices
+  // the union of the gathered rows as a bitmap, its ranks the local indices.
+  // The rows are marked by a byte each, stored plainly: a bit each, by LDS
+  // atomics, had most of a wave's lanes queue at a few words (the neighbours
+  // of neighbouring rows): 24 thousand cycles of a solve's set-up at 13k rows
+  // against 12.
   int own_at, nlist;
   unsigned int at2[(M + 1) / 2];  // slots' places in V, two to a word
   static_assert(3 * small_union(L) <= 65536, "16-bit places");
   {
-    unsigned int* bits = (unsigned int*)T;       // [kThreads]: 16,384 rows
-    unsigned int* rank = bits + kThreads;        // [kThreads] ones before the word
-    unsigned int* wsum = rank + kThreads;        // [kThreads / 64]
-    static_assert(sizeof(T) >= (2 * kThreads + kThreads / 64) * sizeof(unsigned int), "scratch");
-    static_assert(PD_SMALL_UNITS * 64 <= kThreads * 32, "a bit per row");
+    typedef unsigned int u4v __attribute__((ext_vector_type(4)));
+    typedef unsigned int u2v __attribute__((ext_vector_type(2)));
+    u4v* marks = (u4v*)T;                                // [2 kThreads]: 16,384 rows
+    u2v* words = (u2v*)(marks + 2 * kThreads);           // [kThreads] bits, ones before the word
+    unsigned int* wsum = (unsigned int*)(words + kThreads);  // [kThreads / 64]
+    static_assert(sizeof(T) >= 2 * kThreads * 16 + kThreads * 8 + kThreads / 64 * 4, "scratch");
+    static_assert(PD_SMALL_UNITS * 64 <= kThreads * 32, "a byte per row");
     const int t = threadIdx.x, wl = t & 63;
     const int pc = row ? p : 0;
-    bits[t] = 0u;
+    marks[t] = u4v{0u, 0u, 0u, 0u};
+    marks[kThreads + t] = u4v{0u, 0u, 0u, 0u};
     if (t == 0) longest = 0;
     __syncthreads();
+    unsigned char* mark = (unsigned char*)marks;
 #pragma unroll
-    for (int m = 0; m < M; ++m) atomicOr(bits + (q[m] >> 5), 1u << (q[m] & 31));
-    if (j == 0) atomicOr(bits + (pc >> 5), 1u << (pc & 31));
+    for (int m = 0; m < M; ++m) mark[q[m]] = 1;
+    if (j == 0) mark[pc] = 1;
     __syncthreads();
-    const unsigned int mine = bits[t];
+    unsigned int mine = 0u;  // rows 32 t ..
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const u4v v = marks[2 * t + h];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)  // four bytes of 0 or 1 to four bits
+        mine |= ((v[k] * 0x01020408u) >> 24 & 0xfu) << (16 * h + 4 * k);
+    }
     int incl = __popc(mine);
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -752,7 +767,7 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
       nlist += wsum[k];
     }
     const int ex0 = before + incl - __popc(mine);
-    rank[t] = ex0;
+    words[t] = u2v{mine, (unsigned int)ex0};
     unsigned int left = mine;
     for (int k = ex0; left; ++k) {
       if (k < UC) list[k] = (unsigned short)(t * 32 + __ffs((int)left) - 1);
@@ -760,7 +775,8 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
     }
     __syncthreads();
     auto local = [&](int r) {
-      return 3 * (int)(rank[r >> 5] + __popc(bits[r >> 5] & ((1u << (r & 31)) - 1u)));
+      const u2v w = words[r >> 5];
+      return 3 * (int)(w.y + __popc(w.x & ((1u << (r & 31)) - 1u)));
     };
 #pragma unroll
     for (int m = 0; m < M; m += 2) {
