@@ -18,7 +18,7 @@ namespace pd {
 // + core/implicit_euler.cuh:19-86 / core/newmark_beta.cuh:19-86 (fill A, b)
 // + the block-Jacobi inverse of A_pp.  One lane per particle; a wave is one
 // 64-row slice, so every slot read / write is 64 consecutive words.  With
-// shared reciprocals a lane first takes its list three slots per trip
+// shared reciprocals a lane first takes its list four slots per trip
 // without swap-remove, up to the first trip holding a breaking bond; the
 // sequential pass (the next bond's column and neighbour data fetched while
 // the current bond is computed) does the rest.  FP64 bond blocks are not
@@ -854,8 +854,9 @@ void launch_spmv_plain(const SpmvView& A, const double4* x, double4* y, hipStrea
 // kept on the device.  Every streaming kernel writes one partial sum per
 // 256-row tile; the partials of a specimen are folded in the fixed order of
 // the oracle's orc_dot, by a fold kernel with one workgroup per specimen
-// (the start, beta plus the monitor test) or by every workgroup of the
-// update for itself (alpha).  Kernel boundaries order the writes, so no
+// (the start; beta and the monitor test of large systems) or by every
+// workgroup of the update (alpha) and of the direction update (beta) for
+// itself.  Kernel boundaries order the writes, so no
 // fences are needed.  The kernels of a tile or specimen return at once when
 // its solve is done.
 // ---------------------------------------------------------------------------

@@ -90,3 +90,33 @@ def test_ends_of_the_range_equal_stored(n):
         ctx.close()
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_captured_steps_equal_eager(mode):
+    """Past the resident step, captured: the folds inside the direction update
+    and the per-slice partials on every replay."""
+    say("case lanes captured", mode)
+    n = 17000
+    ends = []
+    for graph in (0, 1):
+        x4 = lattice(26, 26, 26, 0.01, 0.05, n)[:n]
+        k = np.arange(n) // 676
+        bc = ((k == 0) | (k == k[-1])).astype(np.int32)
+        vbc = np.zeros((n, 4))
+        vbc[k == k[-1], 2] = 6.0
+        ctx = pds.Context(n, [material(0.01)])
+        pds.load_state(ctx, x4, vbc.copy(), np.full(n, 0.01), bc=bc, vbc=vbc)
+        ctx.build_bonds()
+        out = []
+        for step in range(1, 9):
+            st = ctx.step(pds.make_params(dt=1e-4, clock_scale=step / 8.0, precond=1, rtol=1e-8,
+                                          matrix_free=mode, graph=graph))
+            out.append((st.cg_iterations, st.broken_bonds, st.live_bonds, st.residual_norm))
+            if step % 3 == 0:
+                ctx.download("velocity")  # the program's own work between replays
+        ends.append((out, ctx.download("position"), ctx.download("bond_top")))
+        ctx.close()
+    say(dict(its=[o[0] for o in ends[0][0]], broken=sum(o[1] for o in ends[0][0])))
+    assert ends[0][0] == ends[1][0]
+    assert np.array_equal(ends[0][1], ends[1][1]) and np.array_equal(ends[0][2], ends[1][2])
