@@ -113,9 +113,10 @@ struct pd_step_counters {
 // for both against 8.6 at 110 tiles, 5.4 against 8.2 at 510, but 41.8 against
 // 37.2 at 3930, where the workgroups' reads add up to 250 MB.
 #define PD_DIR_FOLD_TILES 1024
-// Largest system, in slices, whose matrix-free product takes four lanes per
-// row (k_cg_spmv_lanes).
+// Largest systems, in slices, whose matrix-free product takes four and eight
+// lanes per row (k_cg_spmv_lanes).
 #define PD_LANES_SLICES 1536
+#define PD_LANES8_SLICES 512
 
 __device__ __forceinline__ double4 ld4(const double4* p) { return *p; }
 

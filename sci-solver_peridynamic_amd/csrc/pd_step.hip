@@ -1068,20 +1068,22 @@ __host__ __device__ __forceinline__ bool lanes_product(const SpmvView& A) {
 // The same product for systems whose slices leave the 1024 SIMDs with one
 // wave or two: a lane per row then waits out every trip's chain of column,
 // record and some 90 dependent operations, 20 trips in a row, and one slice
-// more than 1024 doubles the time.  Four lanes share a row, four bonds each
-// per trip, one workgroup per slice; a row's terms pass through LDS and
-// three of its lanes add them in list order, so y keeps its bits.  Partials
-// per slice, joined to the tile's by the fold.
+// more than 1024 doubles the time.  L lanes share a row, V bonds each per
+// trip, one workgroup per slice; a row's terms pass through LDS and three of
+// its lanes add them in list order, so y keeps its bits.  Partials per slice,
+// joined to the tile's by the fold.
 // us per product, one lane / two / four / eight (106 to 109 bonds a row):
 //   17.6k rows  34 / 24 / 20 / 18      27k  47 / 29 / 23 / 22
 //   65.6k       61 / 45 / 43 / 48     130k  76 / 77 / 82 / 92
-// so four up to PD_LANES_SLICES = 1536 slices (98k rows, where the lines
-// cross), one above.
-__global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_lanes(CgArgs a) {
-  constexpr int L = 4, V = 4, CH = L * V;
+// so eight up to PD_LANES8_SLICES = 512 slices (28k rows in a step: 25.2
+// against 28.0 with four), four up to PD_LANES_SLICES = 1536 (98k rows, where
+// the lines cross), one above.
+template <int L, int V>
+__global__ __launch_bounds__(64 * L) void k_cg_spmv_lanes(CgArgs a) {
+  constexpr int CH = L * V;
   constexpr int CP = CH + 3;  // odd, so the rows' and components' reads spread over the banks
   constexpr int RW = 64 / L;  // rows per wave
-  __shared__ double terms[PD_BLOCK / 64][RW * 3 * CP];
+  __shared__ double terms[L][RW * 3 * CP];
   __shared__ double ts[64];
   const int ntiles = (a.A.n + PD_BLOCK - 1) / PD_BLOCK;
   const int s = xcd_tile(blockIdx.x, gridDim.x);
@@ -1165,7 +1167,7 @@ __global__ __launch_bounds__(PD_BLOCK) void k_cg_spmv_lanes(CgArgs a) {
     if (j < 3) acc = chain_add(acc, tw + j * CP, min(CH, top + 1 - c0));
     wave_fence();
   }
-  if (row) ((double*)(a.y + p))[j] = j < 3 ? acc : 0.0;
+  if (row && j < 4) ((double*)(a.y + p))[j] = j < 3 ? acc : 0.0;
   const double y1 = __shfl_down(acc, 1, 64), y2 = __shfl_down(acc, 2, 64);
   if (j == 0) ts[pl] = row ? term3(acc, y1, y2, pp.x, pp.y, pp.z) : 0.0;
   __syncthreads();
@@ -1432,12 +1434,19 @@ void launch_cg_init_fold(const CgArgs& a, double rtol, int32_t max_iter, hipStre
   else
     launch_cg_setup(a.st, a.batch.nspec, rtol, max_iter, s);
 }
+static void launch_spmv_lanes(const CgArgs& a, hipStream_t s) {
+  const int slices = (a.A.n + 63) / 64;
+  if (slices <= PD_LANES8_SLICES)
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cg_spmv_lanes<8, 2>), dim3(slices), dim3(64 * 8), 0, s, a);
+  else
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_cg_spmv_lanes<4, 4>), dim3(slices), dim3(64 * 4), 0, s, a);
+}
 void launch_cg_spmv(const CgArgs& a, hipStream_t s) {
   if (!a.A.n) return;
   const int g = tiles_of(a.A.n);
   if (a.A.mf) {
     if (lanes_product(a.A))
-      hipLaunchKernelGGL(k_cg_spmv_lanes, dim3((a.A.n + 63) / 64), dim3(PD_BLOCK), 0, s, a);
+      launch_spmv_lanes(a, s);
     else if (a.A.rec && a.A.range_bad)  // after an assembly: the record and the range flag
       hipLaunchKernelGGL(k_cg_spmv_mf, dim3(g), dim3(PD_BLOCK), 0, s, a);
     else

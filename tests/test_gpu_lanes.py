@@ -1,8 +1,9 @@
-"""The matrix-free product with four lanes per row (systems up to 1536 slices
-of 64 rows that do not take the resident step: here because they are timed,
-solved on their own or too large for it): row counts at the edges of a wave's
-16 rows, a slice, a tile and of its range, lists of every remainder by its 16
-slots and longer than the resident step's, specimens and a range flag."""
+"""The matrix-free product with eight lanes per row (up to 512 slices of 64
+rows) and with four (up to 1536), on systems that do not take the resident
+step (here because they are timed, solved on their own or too large for it):
+row counts at the edges of a wave's rows, a slice, a tile and of the ranges,
+lists of every remainder by its 16 slots and longer than the resident step's,
+specimens and a range flag."""
 import sys
 
 import numpy as np
@@ -70,17 +71,18 @@ def test_operands_out_of_range_take_ieee_forms():
     ctx.close()
 
 
-@pytest.mark.parametrize("n", [98304, 98305])
-def test_ends_of_the_range_equal_stored(n):
-    """The last size with four lanes and the first with one, against the
-    stored blocks."""
-    say("case lanes n", n)
+@pytest.mark.parametrize("n,factor", [(32768, 3.0), (32769, 3.0), (40001, 2.3), (98304, 1.8),
+                                      (98305, 1.8)])
+def test_ends_of_the_ranges_equal_stored(n, factor):
+    """The last size with eight lanes, the first with four, the last with four
+    and the first with one, against the stored blocks."""
+    say("case lanes n", n, factor)
     x4 = lattice(48, 48, -(-n // 2304), 0.01, 0.05, n)[:n]
     v4 = np.zeros((n, 4))
     v4[:, 2] = np.linspace(-1, 1, n)
     out = []
     for mode in (0, 1):
-        ctx = pds.Context(n, [material(0.01, 1.8)])
+        ctx = pds.Context(n, [material(0.01, factor)])
         pds.load_state(ctx, x4, v4, np.full(n, 0.02))
         ctx.build_bonds()
         st = [ctx.step(pds.make_params(dt=1e-4, precond=1, rtol=1e-8, matrix_free=mode))
