@@ -650,8 +650,10 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
   int t0, nt;
   spec_range_of(a.batch, spec, (a.A.n + PD_BLOCK - 1) / PD_BLOCK, t0, nt);
   if (unit == 0 && threadIdx.x == 0) *g.h_cnt = *g.counters;
-  // a tile between specimens: its rows are invisible, nobody awaits its sums
-  if ((s >> 2) >= t0 + nt) return;
+  // a tile before the first specimen, between two or behind the last: its rows
+  // are invisible and nobody awaits its sums, so it may not await others' (they
+  // are unset again as soon as the specimen's own units have read them)
+  if ((s >> 2) < t0 || (s >> 2) >= t0 + nt) return;
   // the slots' blocks (past the list's end anything: nothing adds them)
   int q[M];
   double B[MR][6];

@@ -75,3 +75,67 @@ def deformed_pair(nx=10, ny=9, nz=8, amp=0.03, seed=0, s_fixed=0.02):
         sys_.s[:] = s_fixed
         ctx.upload("stretch", sys_.s)
     return sys_, ctx
+
+
+def specimen_pair(sizes, lead=0, pull=6.0, factor=3.0, s0=0.02):
+    """Independent tension specimens in one GPU context, `lead` rows of
+    INVISIBLE padding before the first, and each of them alone in the oracle;
+    returns (first rows, oracle systems, gpu context)."""
+    import pdsolver as pds
+    mats = [material(0.01, factor)]
+    far = np.array([[-1.0, -1.0, -1.0, 0.0]])
+    parts, first, alone = [], [], []
+
+    def padding(m):
+        return (np.tile(far, (m, 1)), np.zeros((m, 4)), np.zeros(m, np.int32), np.full(m, s0),
+                np.full(m, 3, np.int32))
+
+    if lead:
+        parts.append(padding(lead))
+    row = lead
+    for i, n in enumerate(sizes):
+        w = 4 if n < 2000 else 12
+        x4 = lattice(w, w, -(-n // (w * w)), 0.01, 0.05, 7 * n + i, origin=(0.5 * i, 0.0, 0.0))[:n]
+        k = np.arange(n) // (w * w)
+        bc = ((k == 0) | (k == k[-1])).astype(np.int32)
+        vbc = np.zeros((n, 4))
+        vbc[k == k[-1], 2] = pull * (1.0 + 0.3 * i)
+        sys_ = make_system(x4, mats, s0=s0, seed=11 + i, v4=vbc.copy(), bc=bc, vbc=vbc)
+        parts.append((x4, vbc, bc, sys_.s00.copy(), np.zeros(n, np.int32)))
+        alone.append(sys_)
+        first.append(row)
+        pad = -n % 256
+        if pad:
+            parts.append(padding(pad))
+        row += n + pad
+    x4, vbc, bc, s00, act = (np.concatenate(c) for c in zip(*parts))
+    ctx = pds.Context(row, mats)
+    pds.load_state(ctx, x4, vbc.copy(), s00, act=act, bc=bc, vbc=vbc)
+    ctx.build_bonds()
+    ctx.set_specimens(np.array(first, np.int32), np.array(sizes, np.int32))
+    return first, alone, ctx
+
+
+def compare_specimens(first, alone, ctx, step, kw, steps):
+    """Steps the context by step(kw) and every specimen alone in the oracle:
+    the same bits, counts and residuals; returns the broken bonds."""
+    broken = 0
+    for k in range(1, steps + 1):
+        q = dict(dict(dt=1e-4, clock_scale=min(k, 10) / 10.0, precond=1, rtol=1e-8), **kw)
+        o = {a: b for a, b in q.items() if a not in ("matrix_free", "graph", "timing")}
+        sg = step(q)
+        per = ctx.specimen_stats(len(alone))
+        xg, vg = ctx.download("position"), ctx.download("velocity")
+        tops = ctx.download("bond_top")
+        br = 0
+        for i, (f, S) in enumerate(zip(first, alone)):
+            so = S.step(orc.make_params(**o))
+            br += so.broken_bonds
+            assert per[i]["cg_iterations"] == so.cg_iterations, (k, i)
+            assert per[i]["residual_norm"] == so.residual_norm, (k, i)
+            assert np.array_equal(xg[f:f + S.n, :3], S.x[:, :3]), (k, i)
+            assert np.array_equal(vg[f:f + S.n, :3], S.v[:, :3]), (k, i)
+            assert np.array_equal(tops[f:f + S.n], S.top), (k, i)
+        assert sg.broken_bonds == br, k
+        broken += br
+    return broken

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from pdhelpers import lattice, make_pair, material
+from pdhelpers import compare_specimens, lattice, make_pair, material, specimen_pair
 
 pytestmark = pytest.mark.gpu
 pds = pytest.importorskip("pdsolver")
@@ -116,4 +116,24 @@ def test_operands_out_of_range_take_ieee_forms():
     x4[5, 1] = 1e-200
     S, ctx = make_pair(x4, [material(0.01)])
     compare(S, ctx, 6)
+    ctx.close()
+
+
+# 32, 16 and 8 lanes per row; rows of padding before the first specimen
+@pytest.mark.parametrize("lead", [0, 256, 512])
+@pytest.mark.parametrize("sizes", [(300, 700), (2500, 3000), (5000, 1, 4000)])
+def test_specimens_match_oracle(sizes, lead):
+    """Every specimen as if alone, in one resident launch (one wait a step)."""
+    say("case small specimens", sizes, lead)
+    first, alone, ctx = specimen_pair(sizes, lead)
+    syncs = []
+
+    def step(q):
+        sg = ctx.step(pds.make_params(**q))
+        syncs.append(sg.host_syncs)
+        return sg
+
+    broken = compare_specimens(first, alone, ctx, step, {}, 12)
+    say(dict(broken=broken, syncs=syncs))
+    assert broken > 0 and syncs == [1] * 12
     ctx.close()
