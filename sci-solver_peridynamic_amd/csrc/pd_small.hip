@@ -22,6 +22,7 @@
 #include <math.h>
 
 #include "pd_bond.h"
+#include "pd_resident.h"
 
 namespace pd {
 
@@ -90,17 +91,18 @@ __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)
 // eight times the lines, 5 us a fold at 250 units); the lanes of a slice,
 // then those of a tile join through xor levels (2^(K-1) .. 1 within the
 // slice, then (w0 + w1) + (w2 + w3)), and tile t's sum moves to lane t.
-// WAIT: the partials are written by running workgroups, each is awaited
-// until it is set, `until` (100 MHz clock) has passed or another unit has
-// given up (*aborted); then *late is raised.
+// WAIT: the partials are written by running workgroups and awaited until all
+// are set, the limit (ticks of the 100 MHz clock) has passed or another unit
+// has given up (*aborted); then *late is raised.
 template <int K, int NV, bool WAIT>
 __device__ __forceinline__ void fold_units(const double* part, int64_t stride, int t0, int nt,
-                                           int nslices, int lane, unsigned long long until,
+                                           int nslices, int lane, unsigned long long limit,
                                            const unsigned int* aborted, bool* late,
                                            double* out) {
   const int first = (t0 * 4) << K;
   const int nu = min(nt * 4, nslices - t0 * 4) << K;  // at most 256
   double v[NV][4];
+  WaitLimit wait(limit);
   for (unsigned spin = 0;; ++spin) {
     bool ready = true;
 #pragma unroll
@@ -112,8 +114,8 @@ __device__ __forceinline__ void fold_units(const double* part, int64_t stride, i
         if (WAIT) ready = ready && !is_unset(v[k][r]);
       }
     if (!WAIT || __all(ready)) break;
-    if ((spin & 15) == 15 &&
-        (wall_clock64() > until ||
+    if (WaitLimit::due(spin) &&
+        (wait.over(spin, wall_clock64()) ||
          __hip_atomic_load(aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
       *late = true;
       break;
@@ -612,8 +614,8 @@ __global__ __launch_bounds__(kThreads) void k_small_assemble(AsmArgs a, SmallArg
 // acquire after the wait, by one wave per workgroup (fences in all eight
 // took 30 to 60 us per round; in one they are not seen).
 //
-// Every wait ends: after g.spin_ticks of the 100 MHz clock a workgroup
-// raises *g.aborted and leaves.  The position update behind it then does
+// Every wait ends: after g.spin_ticks of the 100 MHz clock, counted anew in
+// each wait, a workgroup raises *g.aborted and leaves.  The position update behind it then does
 // nothing, and the host puts the start values back (the assembly record
 // holds them) and solves with the general kernels.
 // ---------------------------------------------------------------------------
@@ -645,7 +647,6 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
   const int p = s * 64 + pl;
   const bool row = p < a.A.n;
   const int top = row ? a.A.top[p] : -1;
-  const unsigned long long until = wall_clock64() + g.spin_ticks;
   const int spec = spec_of(a.batch, s >> 2);
   int t0, nt;
   spec_range_of(a.batch, spec, (a.A.n + PD_BLOCK - 1) / PD_BLOCK, t0, nt);
@@ -950,7 +951,7 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
         put(e + 4, p1);
         put(e + 5, p2);
       }
-      fold_units<K, 1, true>(P_yp + b * PR, 0, t0, nt, g.nslices, lane, until, g.aborted,
+      fold_units<K, 1, true>(P_yp + b * PR, 0, t0, nt, g.nslices, lane, g.spin_ticks, g.aborted,
                              &late, &yp);
       alpha = rz / yp;
       double t_rz = 0.0, t_rr = 0.0;
@@ -992,7 +993,7 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
         put(P_rz + (2 + b) * PR + at, vr);
       }
       double sums[2];
-      fold_units<K, 2, true>(P_rz + b * PR, 2 * PR, t0, nt, g.nslices, lane, until,
+      fold_units<K, 2, true>(P_rz + b * PR, 2 * PR, t0, nt, g.nslices, lane, g.spin_ticks,
                              g.aborted, &late, sums);
       const double nrz = sums[0];
       rr = sums[1];

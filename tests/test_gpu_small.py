@@ -5,6 +5,7 @@ lists broken in the middle and to the end, both integrators and operators,
 specimens, and a wait that runs out."""
 import ctypes
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -137,3 +138,48 @@ def test_specimens_match_oracle(sizes, lead):
     say(dict(broken=broken, syncs=syncs))
     assert broken > 0 and syncs == [1] * 12
     ctx.close()
+
+
+def test_limit_counts_from_each_wait():
+    """A solve that makes progress outlasts the limit and is not given up,
+    also while another context's kernels slow some of its workgroups down:
+    40,000 iterations of 8 us or more, 0.1 s a wait."""
+    say("case small long solve")
+    L = pds.lib()
+    L.pd_set_wait_limit.argtypes = [ctypes.c_void_p, ctypes.c_double]
+
+    def bar(n, w):
+        x4 = lattice(w, w, -(-n // (w * w)), 0.01, 0.05, n)[:n]
+        v4 = np.zeros((n, 4))
+        v4[:, :3] = np.random.default_rng(n).uniform(-1, 1, (n, 3))
+        ctx = pds.Context(n, [material(0.01)])
+        pds.load_state(ctx, x4, v4, np.full(n, 1e9))
+        ctx.build_bonds()
+        return ctx
+
+    other, stop = bar(100000, 40), threading.Event()
+
+    def load():
+        while not stop.is_set():
+            other.step(pds.make_params(dt=1e-6, matrix_free=1, rtol=1e-12))
+
+    out = []
+    for limit in (2.0, 0.1):
+        ctx = bar(13225, 4)
+        assert L.pd_set_wait_limit(ctx._h, limit) == pds.PD_OK
+        stop.clear()
+        t = threading.Thread(target=load)
+        t.start()
+        try:
+            st = ctx.step(pds.make_params(dt=1.0, precond=0, rtol=0.0, max_iter=40000),
+                          allow_fail=True)
+        finally:
+            stop.set()
+            t.join()
+        out.append((st.cg_iterations, st.host_syncs, st.residual_norm,
+                    ctx.download("position").tobytes()))
+        ctx.close()
+    other.close()
+    say([o[:3] for o in out])
+    assert out[0][0] == 40000 and out[0][1] == 1
+    assert out[0] == out[1]
