@@ -301,7 +301,8 @@ int pd_restore(pd_ctx* ctx);
  * run at once and await each other's sums.  Where a wait runs out (another
  * process holds the device's room) the step is solved by the general
  * kernels, with identical results, and so are the context's later steps
- * until this is called again. */
+ * until this is called again.  0: nothing is awaited, the next step is handed
+ * to them. */
 int pd_set_wait_limit(pd_ctx* ctx, double seconds);
 
 /* Wait for all work on the context stream. */

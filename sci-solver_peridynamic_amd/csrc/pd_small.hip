@@ -615,9 +615,10 @@ __global__ __launch_bounds__(kThreads) void k_small_assemble(AsmArgs a, SmallArg
 // took 30 to 60 us per round; in one they are not seen).
 //
 // Every wait ends: after g.spin_ticks of the 100 MHz clock, counted anew in
-// each wait, a workgroup raises *g.aborted and leaves.  The position update behind it then does
-// nothing, and the host puts the start values back (the assembly record
-// holds them) and solves with the general kernels.
+// each wait, a workgroup raises *g.aborted and leaves (0 ticks: before the
+// first iteration, whatever the others do).  The position update behind it
+// then does nothing, and the host puts the start values back (the assembly
+// record holds them) and solves with the general kernels.
 // ---------------------------------------------------------------------------
 // M slots per lane, the blocks of the first MR in registers and of the rest
 // in LDS; MC slots per chunk.
@@ -853,9 +854,10 @@ __global__ __launch_bounds__(kThreads) void k_small_solve(CgArgs a, SmallArgs g)
     } else if (g.max_iter <= 0) {
       done = true;
     }
+    late = g.spin_ticks == 0;  // no wait at all
     if (threadIdx.x == 0) {
       ctl[0] = 0.0;
-      ctl[1] = done ? 0.0 : 1.0;
+      ctl[1] = done || late ? 0.0 : 1.0;
     }
   }
   __syncthreads();

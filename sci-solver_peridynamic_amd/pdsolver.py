@@ -147,6 +147,7 @@ def lib():
         L.pd_get_matrix.argtypes = [vp, vp, vp, C.c_int32]
         for name in ("pd_step", "pd_assemble", "pd_solve"):
             getattr(L, name).argtypes = [vp, C.POINTER(StepParams), C.POINTER(StepStats)]
+        L.pd_set_wait_limit.argtypes = [vp, C.c_double]
         L.pd_update.argtypes = [vp, C.POINTER(StepParams)]
         L.pd_commit_stretch.argtypes = [vp]
         L.pd_spmv.argtypes = [vp, vp, vp]
@@ -173,6 +174,7 @@ def lib():
         for name in ("pd_ctx_create", "pd_ctx_destroy", "pd_upload", "pd_download",
                      "pd_build_bonds", "pd_set_bonds", "pd_get_bonds", "pd_get_matrix",
                      "pd_step", "pd_assemble", "pd_solve", "pd_update", "pd_commit_stretch",
+                     "pd_set_wait_limit",
                      "pd_spmv", "pd_backup", "pd_restore", "pd_synchronize", "pd_bench_spmv",
                      "pd_spmv_bytes", "pd_check_division", "pd_set_specimens", "pd_get_specimen_stats",
                      "pd_tune_spmv", "pd_learned_set", "pd_get_precond", "pd_trainer_create",
@@ -284,6 +286,11 @@ class Context:
         if not (allow_fail and rc == PD_ERR_NOT_CONVERGED):
             self._check(rc)
         return st
+
+    def set_wait_limit(self, seconds):
+        """Longest wait of the resident solve of small systems (pd_set_wait_limit); 0 leaves it to
+        the general kernels."""
+        self._check(lib().pd_set_wait_limit(self._h, seconds))
 
     def update(self, prm):
         self._check(lib().pd_update(self._h, C.byref(prm)))

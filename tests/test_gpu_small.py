@@ -183,3 +183,34 @@ def test_limit_counts_from_each_wait():
     say([o[:3] for o in out])
     assert out[0][0] == 40000 and out[0][1] == 1
     assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("kw", [dict(matrix_free=0), dict(matrix_free=1), dict(matrix_free=2),
+                                dict(matrix_free=1, integrator=1), dict(precond=0),
+                                dict(matrix_free=0, graph=1), dict(rtol=1e10)])
+@pytest.mark.parametrize("lead", [0, 256])
+def test_fallback_matches_oracle(lead, kw):
+    """A limit of zero gives the solve up before its first iteration, also one
+    that would end there: that step and the next ones come from the general
+    kernels (more than one host wait; a general step after that has the
+    previous one's count), a new limit takes the resident solve up again."""
+    say("case small fallback", lead, kw)
+    first, alone, ctx = specimen_pair((300, 700), lead)
+    syncs = []
+
+    def step(q):
+        if len(syncs) == 3:
+            ctx.set_wait_limit(0.0)
+        if len(syncs) == 6:
+            ctx.set_wait_limit(2.0)
+        sg = ctx.step(pds.make_params(**q))
+        syncs.append(sg.host_syncs)
+        return sg
+
+    compare_specimens(first, alone, ctx, step, kw, 9)
+    say(syncs)
+    assert syncs[:3] == [1] * 3 and syncs[6:] == [1] * 3
+    assert syncs[3] > 1
+    with pytest.raises(pds.PDError):
+        ctx.set_wait_limit(-1.0)
+    ctx.close()
