@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "pd_internal.h"
+#include "pd_resident.h"
 #include "../../include/pd_solver.h"
 
 static_assert(PD_LEARNED_PARAMS == PC_NPARAM, "learned parameter layout");
@@ -181,10 +182,7 @@ struct pd_ctx {
   int small_fit = -1;              // the units' neighbours fit LDS (-1: not counted yet)
   bool small_off = false;          // a wait ran out in this context: not again
   unsigned long long spin_ticks = 200000000ull;  // 2 s of the 100 MHz clock
-  double* small_ex = nullptr;      // [2][n][6]
-  double* small_part = nullptr;    // [9][PD_SMALL_ROW]
-  unsigned int* small_abort = nullptr;
-  unsigned int* h_small_abort = nullptr;  // pinned
+  pd::SmallScratch small;
 };
 
 struct pd_trainer {
@@ -673,26 +671,44 @@ int small_step_lanes(pd_ctx* c, const pd_step_params* prm) {
   return lanes != 8 || c->small_fit == 1 ? lanes : 0;
 }
 
-int small_args(pd_ctx* c, const pd_step_params* prm, int lanes, pd::SmallArgs* g) {
-  if (!c->small_ex) {
-    if (int e = dalloc(c, &c->small_ex, (size_t)c->n * 12)) return e;
-    if (int e = dalloc(c, &c->small_part, 9 * PD_SMALL_ROW)) return e;
-    if (int e = dalloc(c, &c->small_abort, 1)) return e;
-    if (hipHostMalloc((void**)&c->h_small_abort, sizeof(unsigned int), hipHostMallocDefault) !=
-        hipSuccess)
-      return fail(c, PD_ERR_HIP, "hipHostMalloc failed");
+// SmallScratch's memory
+struct SmallAlloc {
+  pd_ctx* c;
+  template <typename T>
+  int device(T** p, size_t count) {
+    return dalloc(c, p, count);
   }
+  template <typename T>
+  int pinned(T** p) {
+    if (hipHostMalloc((void**)p, sizeof(T), hipHostMallocDefault) == hipSuccess) return PD_OK;
+    *p = nullptr;
+    return fail(c, PD_ERR_HIP, "hipHostMalloc failed");
+  }
+  template <typename T>
+  void device_free(T*& p) {
+    dfree(p);
+  }
+  template <typename T>
+  void pinned_free(T*& p) {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+  }
+};
+
+int small_args(pd_ctx* c, const pd_step_params* prm, int lanes, pd::SmallArgs* g) {
+  SmallAlloc al{c};
+  if (int e = c->small.ensure(al, (size_t)c->n, PD_SMALL_ROW)) return e;
   g->units = c->nslices * (lanes / 8);
   g->nslices = c->nslices;
-  g->ex = c->small_ex;
-  g->start = c->small_part;
-  g->part = c->small_part + 3 * PD_SMALL_ROW;
+  g->ex = c->small.ex;
+  g->start = c->small.part;
+  g->part = c->small.part + 3 * PD_SMALL_ROW;
   g->rtol = prm->rtol;
   g->max_iter = prm->max_iter;
   g->spin_ticks = c->spin_ticks;
   g->counters = c->counters;
-  g->aborted = c->small_abort;
-  g->h_aborted = c->h_small_abort;
+  g->aborted = c->small.aborted;
+  g->h_aborted = c->small.h_aborted;
   g->h_st = c->h_st;
   g->h_cnt = c->h_cnt;
   return PD_OK;
@@ -1538,18 +1554,18 @@ int run_step_small(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int 
   if (int e = small_args(c, prm, lanes, &g)) return e;
   pd::CgArgs a = cg_args(c, prm->precond);
   if (prm->matrix_free) a.vals = nullptr;  // else the blocks are written on the way
-  *c->h_small_abort = 0u;
+  *c->small.h_aborted = 0u;
   const bool deferred = c->blocks_deferred;
   {
     std::lock_guard<std::mutex> lock(g_small_mu[c->device]);
     pd::launch_small_solve(lanes, a, g, c->stream);
     CHECK_LAUNCH(c, "resident solve");
     c->blocks_deferred = false;
-    if (int e = enqueue_update(c, prm, nullptr, c->small_abort)) return e;
+    if (int e = enqueue_update(c, prm, nullptr, c->small.aborted)) return e;
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
   int syncs = 1;
-  if (*c->h_small_abort) {  // no room for all its workgroups at once
+  if (*c->small.h_aborted) {  // no room for all its workgroups at once
     c->small_off = true;
     c->blocks_deferred = deferred;
     pd::launch_small_undo(c->n, c->arec, c->sol, c->stream);
@@ -1766,8 +1782,8 @@ int pd_ctx_destroy(pd_ctx* c) {
   destroy_graphs(c);
   dfree(c->consts);
   if (c->h_consts) (void)hipHostFree(c->h_consts);
-  dfree(c->small_ex); dfree(c->small_part); dfree(c->small_abort);
-  if (c->h_small_abort) (void)hipHostFree(c->h_small_abort);
+  SmallAlloc small_alloc{c};
+  c->small.release(small_alloc);
   dfree(c->bond_stats); dfree(c->pc_feat); dfree(c->pc_p); dfree(c->pc_w);
   dfree(c->pc_minv); dfree(c->pc_minv32);
   if (c->h_mx) (void)hipHostFree(c->h_mx);

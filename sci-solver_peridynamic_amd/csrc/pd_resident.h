@@ -2,6 +2,8 @@
 // device: plain C++, also compiled by the tests for the host.
 #pragma once
 
+#include <cstddef>
+
 #if defined(__HIPCC__)
 #define PD_HD __host__ __device__ __forceinline__
 #else
@@ -22,6 +24,33 @@ struct WaitLimit {
   PD_HD bool over(unsigned poll, unsigned long long now) {
     if (poll == 15) since = now;
     return now - since > limit;
+  }
+};
+
+// A context's scratch for the resident step, there as a whole or not at all:
+// a step that could not allocate it reports that, and so does the next one.
+// Alloc: int device(T**, count), int pinned(T**), 0 on success, and
+// device_free(T*&), pinned_free(T*&), which take null.
+struct SmallScratch {
+  double* ex = nullptr;               // [2][n][6]
+  double* part = nullptr;             // [9][row]
+  unsigned int* aborted = nullptr;    // device word
+  unsigned int* h_aborted = nullptr;  // pinned
+  template <class Alloc>
+  int ensure(Alloc& al, size_t n, size_t row) {
+    if (h_aborted) return 0;  // allocated last
+    int e;
+    if ((e = al.device(&ex, 12 * n)) || (e = al.device(&part, 9 * row)) ||
+        (e = al.device(&aborted, 1)) || (e = al.pinned(&h_aborted)))
+      release(al);
+    return e;
+  }
+  template <class Alloc>
+  void release(Alloc& al) {
+    al.device_free(ex);
+    al.device_free(part);
+    al.device_free(aborted);
+    al.pinned_free(h_aborted);
   }
 };
 

@@ -1,5 +1,6 @@
 // Host checks of csrc/pd_resident.h: prints one line per check that fails.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 
 #include "pd_resident.h"
@@ -39,8 +40,61 @@ static void wait_limit() {
   CHECK(!wait(limit, 1400, &clock));
 }
 
+// Counts what is held; the allocation number `fail_at` fails, once, after
+// its memory was taken when `late` (a device allocation is cleared after it).
+struct Alloc {
+  int fail_at, late, calls = 0, held = 0;
+  template <typename T>
+  int device(T** p, size_t n) {
+    *p = nullptr;
+    const bool fails = calls++ == fail_at;
+    if (fails && !late) return 2;
+    *p = (T*)malloc(n * sizeof(T));
+    ++held;
+    return fails ? 2 : 0;
+  }
+  template <typename T>
+  int pinned(T** p) {
+    *p = nullptr;
+    if (calls++ == fail_at) return 2;
+    *p = (T*)malloc(sizeof(T));
+    ++held;
+    return 0;
+  }
+  template <typename T>
+  void device_free(T*& p) {
+    if (p) --held;
+    free(p);
+    p = nullptr;
+  }
+  template <typename T>
+  void pinned_free(T*& p) {
+    device_free(p);
+  }
+};
+
+static void scratch() {
+  for (int late = 0; late < 2; ++late)
+    for (int k = -1; k < 4; ++k) {
+      Alloc al{k, late};
+      pd::SmallScratch s;
+      const int first = s.ensure(al, 7, 5);
+      CHECK((first != 0) == (k >= 0));
+      if (first) {
+        CHECK(al.held == 0 && !s.ex && !s.part && !s.aborted && !s.h_aborted);
+        CHECK(s.ensure(al, 7, 5) == 0);  // memory is there again
+      }
+      CHECK(al.held == 4 && s.ex && s.part && s.aborted && s.h_aborted);
+      const int calls = al.calls;
+      CHECK(s.ensure(al, 7, 5) == 0 && al.calls == calls);
+      s.release(al);
+      CHECK(al.held == 0 && !s.h_aborted);
+    }
+}
+
 int main(int argc, char** argv) {
   if (argc > 1 && !strcmp(argv[1], "wait_limit")) wait_limit();
+  else if (argc > 1 && !strcmp(argv[1], "scratch")) scratch();
   else return 2;
   return bad ? 1 : 0;
 }
