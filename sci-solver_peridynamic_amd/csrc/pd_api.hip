@@ -640,9 +640,14 @@ int enqueue_contact(pd_ctx* c, const pd_step_params* prm) {
   return PD_OK;
 }
 
-// One resident solve at a time per device: two of them could each hold part
-// of the chip and wait for workgroups that find no room.
-std::mutex g_small_mu[64];
+// The resident solves of a device's contexts run side by side as far as there
+// is room for all of their workgroups (one per CU): two solves that each held
+// part of the chip would wait for workgroups that find none.
+constexpr int kXcds = 8, kSmallDevices = 64;
+struct SmallPlaces : pd::Places {
+  SmallPlaces() : Places(PD_SMALL_UNITS / kXcds) {}
+};
+SmallPlaces g_small_places[kSmallDevices];
 
 // Lanes per row of the small-system step, or 0: the general kernels.  They
 // stay for mixed precision, the learned preconditioner, gap tracking and
@@ -650,7 +655,7 @@ std::mutex g_small_mu[64];
 // where a row per lane fills the chip.
 int small_step_lanes(pd_ctx* c, const pd_step_params* prm) {
   if (c->small_off || c->n <= 0 || prm->precision != 0 || prm->precond == 2 || prm->track_gap ||
-      prm->timing || c->device >= 64)
+      prm->timing || c->device >= kSmallDevices)
     return 0;
   const int lanes = pd::small_lanes(c->nslices, c->max_cap);
   if (!lanes) return 0;
@@ -1557,7 +1562,7 @@ int run_step_small(pd_ctx* c, const pd_step_params* prm, pd_step_stats* st, int 
   *c->small.h_aborted = 0u;
   const bool deferred = c->blocks_deferred;
   {
-    std::lock_guard<std::mutex> lock(g_small_mu[c->device]);
+    const pd::PlacesHeld places(g_small_places[c->device], pd::Places::needed(g.units, kXcds));
     pd::launch_small_solve(lanes, a, g, c->stream);
     CHECK_LAUNCH(c, "resident solve");
     c->blocks_deferred = false;

@@ -2,6 +2,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <atomic>
+#include <chrono>
+#include <thread>
+#include <vector>
 
 #include "pd_resident.h"
 
@@ -92,9 +96,56 @@ static void scratch() {
     }
 }
 
+// `solves` threads of `workgroups` each, two turns apiece: the most at a time.
+static int most_at_once(pd::Places& p, int solves, int workgroups) {
+  const int k = pd::Places::needed(workgroups, 8);
+  std::atomic<int> now{0}, most{0};
+  std::vector<std::thread> t;
+  for (int i = 0; i < solves; ++i)
+    t.emplace_back([&] {
+      for (int turn = 0; turn < 2; ++turn) {
+        pd::PlacesHeld held(p, k);
+        const int mine = ++now;
+        for (int m = most; mine > m && !most.compare_exchange_weak(m, mine);) {
+        }
+        std::this_thread::sleep_for(std::chrono::milliseconds(20));
+        --now;
+      }
+    });
+  for (auto& th : t) th.join();
+  return most;
+}
+
+static void places() {
+  CHECK(pd::Places::needed(1, 8) == 1 && pd::Places::needed(8, 8) == 1);
+  CHECK(pd::Places::needed(20, 8) == 3 && pd::Places::needed(256, 8) == 32);
+  pd::Places p(32);
+  CHECK(most_at_once(p, 16, 20) == 10);   // 288 rows: 3 places each
+  CHECK(most_at_once(p, 5, 128) == 2);
+  CHECK(most_at_once(p, 5, 129) == 1);    // 17 + 17 > 32
+  CHECK(most_at_once(p, 3, 256) == 1);
+  // a solve of the whole device comes to its turn among small ones
+  std::atomic<bool> stop{false};
+  std::vector<std::thread> small;
+  for (int i = 0; i < 4; ++i)
+    small.emplace_back([&] {
+      while (!stop) {
+        pd::PlacesHeld held(p, 3);
+        std::this_thread::sleep_for(std::chrono::milliseconds(1));
+      }
+    });
+  std::this_thread::sleep_for(std::chrono::milliseconds(5));
+  { pd::PlacesHeld held(p, 32); }
+  stop = true;
+  for (auto& th : small) th.join();
+  p.take(32);  // everything was given back
+  p.give(32);
+}
+
 int main(int argc, char** argv) {
   if (argc > 1 && !strcmp(argv[1], "wait_limit")) wait_limit();
   else if (argc > 1 && !strcmp(argv[1], "scratch")) scratch();
+  else if (argc > 1 && !strcmp(argv[1], "places")) places();
   else return 2;
   return bad ? 1 : 0;
 }

@@ -6,6 +6,7 @@ specimens, and a wait that runs out."""
 import ctypes
 import sys
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -214,3 +215,59 @@ def test_fallback_matches_oracle(lead, kw):
     with pytest.raises(pds.PDError):
         ctx.set_wait_limit(-1.0)
     ctx.close()
+
+
+def test_contexts_step_side_by_side():
+    """A short system's steps end while another context's long solve (126 of the
+    256 workgroups, 40,000 iterations) is still under way, each with the bits
+    of a run of its own."""
+    say("case small side by side")
+
+    def bar(n, seed):
+        x4 = lattice(4, 4, -(-n // 16), 0.01, 0.05, seed)[:n]
+        v4 = np.zeros((n, 4))
+        v4[:, :3] = np.random.default_rng(seed).uniform(-1, 1, (n, 3))
+        ctx = pds.Context(n, [material(0.01)])
+        pds.load_state(ctx, x4, v4, np.full(n, 1e9))
+        ctx.build_bonds()
+        return ctx
+
+    def long_solve(ctx):
+        st = ctx.step(pds.make_params(dt=100.0, precond=0, rtol=0.0, max_iter=40000),
+                      allow_fail=True)
+        say(dict(iterations=st.cg_iterations))
+        assert st.cg_iterations > 30000 and st.host_syncs == 1
+
+    def short_steps(ctx):
+        for _ in range(20):
+            ctx.step(pds.make_params(dt=1e-4))
+
+    want = []
+    for n, work in ((2000, long_solve), (300, short_steps)):
+        ctx = bar(n, n)
+        work(ctx)
+        want.append(ctx.download("position"))
+        ctx.close()
+    a, b = bar(2000, 2000), bar(300, 300)
+    errors = []
+
+    def run():
+        try:
+            long_solve(a)
+        except Exception as e:  # noqa: BLE001 -- told to the test's thread
+            errors.append(e)
+
+    t = threading.Thread(target=run)
+    t.start()
+    time.sleep(0.05)  # the long solve (0.3 s) has its workgroups
+    t0 = time.perf_counter()
+    short_steps(b)
+    spent = time.perf_counter() - t0
+    still = t.is_alive()
+    t.join()
+    say(dict(short=spent, still=still))
+    assert not errors and still
+    assert np.array_equal(a.download("position"), want[0])
+    assert np.array_equal(b.download("position"), want[1])
+    a.close()
+    b.close()

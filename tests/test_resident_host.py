@@ -17,7 +17,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["wait_limit", "scratch"])
+@pytest.mark.parametrize("check", ["wait_limit", "scratch", "places"])
 def test_rule(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
