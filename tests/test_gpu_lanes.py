@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from pdhelpers import lattice, make_pair, material
+from pdhelpers import compare_specimens, lattice, make_pair, material, specimen_pair
 from test_gpu_small import compare, pair
 
 pytestmark = pytest.mark.gpu
@@ -122,3 +122,34 @@ def test_captured_steps_equal_eager(mode):
     say(dict(its=[o[0] for o in ends[0][0]], broken=sum(o[1] for o in ends[0][0])))
     assert ends[0][0] == ends[1][0]
     assert np.array_equal(ends[0][1], ends[1][1]) and np.array_equal(ends[0][2], ends[1][2])
+
+
+# 18,176 rows, the first tile padding: eight lanes per row; 34,304: four
+@pytest.mark.parametrize("sizes,lead", [((300, 9000, 8000), 256), ((9000, 1, 8500, 16000), 0)])
+def test_specimens_match_oracle(sizes, lead):
+    """Specimens past the resident step, stored and recomputed, eager and
+    captured: each as if alone in the oracle, also beside ones that have ended."""
+    say("case lanes specimens", sizes, lead)
+    first, alone, ctx = specimen_pair(sizes, lead, pull=9.0)
+    others = [(dict(matrix_free=m, graph=g), specimen_pair(sizes, lead, pull=9.0)[2])
+              for m, g in ((0, 1), (1, 0), (1, 1))]
+    ends = set()
+
+    def step(q):
+        sg = ctx.step(pds.make_params(**q))
+        per = ctx.specimen_stats(len(sizes))
+        ends.add(tuple(s["cg_iterations"] for s in per))
+        for kw, o in others:
+            so = o.step(pds.make_params(**dict(q, **kw)))
+            assert (so.cg_iterations, so.broken_bonds, so.live_bonds) == \
+                (sg.cg_iterations, sg.broken_bonds, sg.live_bonds), kw
+            assert o.specimen_stats(len(sizes)) == per, kw
+            for f in ("position", "velocity", "bond_top"):
+                assert np.array_equal(o.download(f), ctx.download(f)), (f, kw)
+        return sg
+
+    broken = compare_specimens(first, alone, ctx, step, {}, 10)
+    say(dict(broken=broken, iterations=sorted(ends)))
+    assert broken > 0 and any(len(set(e)) > 1 for e in ends)
+    for c in [ctx] + [o for _, o in others]:
+        c.close()
