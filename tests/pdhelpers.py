@@ -21,11 +21,14 @@ def material(h, horizon_factor=3.0, stiffness=1e4, mass=1e-3):
     return (horizon_factor * h, 0.5 * h, stiffness * h, mass)
 
 
-def make_system(x4, materials, body=None, s0=0.02, seed=1973, v4=None, **kw):
+def make_system(x4, materials, body=None, s0=0.02, seed=1973, v4=None, lists=None, **kw):
     n = x4.shape[0]
     hs = [m[0] for m in materials]
-    counts, lists, total = orc.bonds_brute(x4, hs, body=body)
-    assert total >= 0
+    if lists is None:
+        counts, lists, total = orc.bonds_brute(x4, hs, body=body)
+        assert total >= 0
+    else:  # (counts, padded rows)
+        counts, lists = lists
     rs, col = orc.lists_to_csr(counts, lists)
     s00 = orc.stretch_init(n, s0, seed)
     v4 = np.zeros((n, 4)) if v4 is None else v4

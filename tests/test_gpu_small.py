@@ -12,7 +12,8 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from pdhelpers import compare_specimens, lattice, make_pair, material, specimen_pair
+from pdhelpers import (compare_specimens, lattice, make_pair, make_system, material,
+                       specimen_pair)
 
 pytestmark = pytest.mark.gpu
 pds = pytest.importorskip("pdsolver")
@@ -271,3 +272,78 @@ def test_contexts_step_side_by_side():
     assert np.array_equal(b.download("position"), want[1])
     a.close()
     b.close()
+
+
+def listed_pair(x4, counts, lists, factor, s0, **kw):
+    """make_pair with the lists given (counts, padded rows)."""
+    mats = [material(0.01, factor)]
+    S = make_system(x4, mats, s0=s0, lists=(counts, lists), **kw)
+    ctx = pds.Context(len(x4), mats)
+    pds.load_state(ctx, x4, S.v, S.s00, bc=kw.get("bc"), vbc=kw.get("vbc"))
+    ctx.set_bonds(counts, lists)
+    return S, ctx
+
+
+def compare_limited(S, ctx, steps, **kw):
+    """compare() of solves that may end at the iteration limit (a list cut off
+    leaves no symmetric matrix); returns the first step's host waits."""
+    syncs = []
+    for k in range(1, steps + 1):
+        p = dict(dict(dt=1e-4, clock_scale=k / 10.0, precond=1, rtol=1e-8, max_iter=30), **kw)
+        so = S.step(orc.make_params(**p))
+        sg = ctx.step(pds.make_params(**p), allow_fail=True)
+        syncs.append(sg.host_syncs)
+        assert so.cg_iterations > 1
+        assert (so.cg_iterations, so.broken_bonds, so.residual_norm) == \
+            (sg.cg_iterations, sg.broken_bonds, sg.residual_norm), k
+        assert np.isfinite(S.x).all()
+        assert np.array_equal(ctx.download("position")[:, :3], S.x[:, :3]), k
+    assert np.array_equal(ctx.download("bond_top"), S.top)
+    return syncs[0]
+
+
+# 32, 16 and 8 lanes per row
+@pytest.mark.parametrize("layers", [7, 90, 180])
+@pytest.mark.parametrize("longest", [119, 120, 121, 128, 129])
+def test_longest_list(layers, longest):
+    """Lists of exactly the longest that the resident step takes, one fewer and
+    more (rows well inside the lattice have 146 neighbours, cut off here)."""
+    say("case small longest list", layers, longest)
+    x4 = lattice(7, 7, layers, 0.01, 0.01, layers)
+    n = len(x4)
+    counts, lists, _ = orc.bonds_brute(x4, [0.0324])
+    assert counts.max() == 146
+    counts = np.minimum(counts, longest).astype(np.int32)
+    k = np.arange(n) // 49
+    bc = ((k == 0) | (k == layers - 1)).astype(np.int32)
+    vbc = np.zeros((n, 4))
+    vbc[k == layers - 1, 2] = 12.0
+    S, ctx = listed_pair(x4, counts, lists[:, :longest], 3.24, 0.02, v4=vbc.copy(), bc=bc, vbc=vbc)
+    first = compare_limited(S, ctx, 6)
+    say(dict(waits=first, broken=int(counts.sum() - (S.top + 1).sum())))
+    assert (first == 1) == (longest <= 120)
+    ctx.close()
+
+
+@pytest.mark.parametrize("others", [1823, 1824])
+def test_neighbours_of_a_unit(others):
+    """Eight lanes per row: rows 64 .. 127 have this many neighbours outside;
+    with themselves and one more the first are the 1888 that the solve holds in
+    LDS, the second one too many."""
+    say("case small neighbours of a unit", others)
+    n = 8256
+    x4 = lattice(12, 12, 58, 0.01, 0.05, 3)[:n]
+    rows = [[q for q in (p - 1, p + 1) if 0 <= q < n] for p in range(n)]
+    for i in range(64):
+        rows[64 + i] = list(range(128 + i, 128 + others, 64))
+    counts = np.array([len(r) for r in rows], np.int32)
+    lists = np.zeros((n, counts.max()), np.int32)
+    for p, r in enumerate(rows):
+        lists[p, :len(r)] = r
+    v4 = np.zeros((n, 4))
+    v4[:, :3] = np.random.default_rng(n).uniform(-1, 1, (n, 3))
+    S, ctx = listed_pair(x4, counts, lists, 3.0, 1e9, v4=v4)
+    first = compare_limited(S, ctx, 3)
+    say(dict(waits=first))
+    assert (first == 1) == (others == 1823)
+    ctx.close()
