@@ -31,9 +31,21 @@ typedef double vpair __attribute__((ext_vector_type(2)));
 // an excess of 2^-16 ulp, so quotients by one denominator can share y, which
 // may come from any such refinement.  No scaling happens when b and
 // 1/b are normal, a is 0 or |a| >= 2^-969, a / b is normal and exponent(a) -
-// exponent(b) < 768.  (Two refinements can only give different quotients for
-// a / b within 1.5 2^-53 ulp of a rounding boundary, a few numerators in 2^52
-// for each b, and only where the two y differ, 2^-16 of all b or fewer.)
+// exponent(b) < 768.
+//
+// What any such y gives is the IEEE quotient for every b whose mantissa is
+// below 2 (1 - 2^-15).  With b in (1, 2) and a / b in (1, 2): the last fma
+// rounds a / b + r (y - 1 / b), r = a - b q, which goes wrong only if a
+// rounding boundary m lies in between.  a - b m is a multiple of 2^-105 and
+// not 0, so |a / b - m| >= 2^-105 / b, while |y - 1 / b| <= 2^-54 (1 + 2^-15).
+// If q is next to m, |r| is about b 2^-53 and b^2 (1 + 2^-15) >= 4 would be
+// needed; q is further off only if a |y - 1 / b| >= 2^-52, so again for a b
+// within 2^-15 of 2.  There two refinements can differ, by an ulp, for a few
+// numerators each.  Of the 4.2 million nearest to a boundary for b = 2 - B
+// 2^-52, B odd below 2^22, this one's y is wrong for none, that of sqrt_rcp
+// for 2 / (2 - 2^-52), and the division's own two Newton steps for three
+// (B = 5, 11, 13).  "Identical" below means up to that.
+//
 // Every denominator here is positive: then a = +0 gives
 // +0 as IEEE division does, but a = -0 would give +0 where it gives -0, so no
 // caller passes -0 (a coordinate difference is -0 only for a -0 coordinate
