@@ -95,7 +95,11 @@ typedef struct pd_step_params {
   double contact_volume;    /* PD_V divisor */
   double contact_cell;      /* grid cell edge for contact, >= Rc */
   int32_t track_gap;        /* 1: report the bond closest to breaking */
-  int32_t timing;           /* 1: time phases and SpMV launches */
+  int32_t timing;           /* 1: time phases and SpMV launches.  A step of a
+                               small system (pd_set_wait_limit), which has no
+                               such launches, is then taken by the general
+                               kernels: same results, other and longer times
+                               than those of its untimed steps */
   /* Solver precision (not in the reference, which is FP64 only).
    * 0: FP64 CG.  1: the assembly also rounds the bond blocks, the diagonal
    * and its block-Jacobi inverse to float, and the solve is iterative
