@@ -10,15 +10,17 @@
 //   * the lanes of a row evaluate its bonds side by side into LDS and a few
 //     of them then add the terms in list order, so every sum has the order,
 //     and the bits, of the one-lane walk;
-//   * each lane keeps the 3x3 blocks of its slots in registers for the whole
-//     solve (at most 15 blocks, 180 VGPRs): a product gathers 48 bytes per
-//     bond and multiplies;
+//   * each lane keeps the 3x3 blocks of its slots on the chip for the whole
+//     solve (with 8 lanes up to 15 of them, 13 in registers and two in LDS),
+//     and the workgroup keeps p of its rows' neighbours in LDS: a product
+//     multiplies from registers and LDS;
 //   * the workgroups exchange z, p and the partial sums through global
 //     memory without leaving the kernel.
-// Measured at 8,000 rows, 11 iterations: assembly 93 -> 31 us, solve about
-// 590 (44 launches) -> 140 us, the step 744 -> 217 us; at 288 rows the step
-// 400 -> 124 us.  An iteration at 4,553 rows (143 workgroups): 9.1 us, of
-// which the products and their sums 2.9, the waits for the two sums 3.9.
+// Steps before -> now: 288 rows 410 -> 114 us (assembly 13, solve 66), 8,000
+// rows 755 -> 205 (assembly 93 -> 23; the solve, 149, was some 60 launches),
+// 13,225 rows, Newmark, 504 -> 148 (26 and 96).  An iteration at 4,553 rows
+// (143 workgroups): 9.1 us, of which the products and their sums 2.9, the
+// waits for the two sums 3.9.
 #include <math.h>
 
 #include "pd_bond.h"
@@ -30,17 +32,17 @@ namespace {
 
 constexpr int kThreads = PD_SMALL_THREADS;
 
-// Unit u of a solve with L lanes per row: slice u >> K, and of it the rows
-// whose low K bits equal u's (K = log2(L / 8)), row i of the unit being row
-// (i << K) + c of the slice.  The xor butterfly of a slice's wave sum pairs
-// lanes 32, 16, .. 1 apart; a unit holds whole subtrees of its first 6 - K
-// levels, and the remaining K levels join the slice's units.
 // Longest neighbour list of a unit that the solve keeps in LDS.  With 16 and
 // 32 lanes no unit can have more (its rows, their bonds and row 0).
 constexpr int small_union(int lanes) {
   return lanes == 8 ? PD_SMALL_UNION : kThreads / lanes * (PD_SMALL_MAX_BONDS + 1) + 1;
 }
 
+// Unit u of a solve with L lanes per row: slice u >> K, and of it the rows
+// whose low K bits equal u's (K = log2(L / 8)), row i of the unit being row
+// (i << K) + c of the slice.  The xor butterfly of a slice's wave sum pairs
+// lanes 32, 16, .. 1 apart; a unit holds whole subtrees of its first 6 - K
+// levels, and the remaining K levels join the slice's units.
 template <int L>
 struct Unit {
   static constexpr int R = kThreads / L;
@@ -139,7 +141,7 @@ __device__ __forceinline__ void fold_units(const double* part, int64_t stride, i
   }
 }
 
-// Two of them side by side.
+// chain_add (pd_device.h) over two lists of n terms side by side.
 __device__ __forceinline__ void chain_add2(double (&acc)[2], const double* t0, const double* t1,
                                            int n) {
   double a0 = acc[0], a1 = acc[1];
@@ -252,7 +254,6 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
   double* tr = lds + i * ROW;
   const int64_t base = a.slice_off[s];
   int top = vis ? a.top[p] : -1;
-  const int otop = top;
   pd_mat_dev mt = {1.0, 1.0, 1.0, 1.0};
   double4 pos_p = make_double4(0.0, 0.0, 0.0, 0.0);
   float stretch_f = 0.0f;
@@ -567,7 +568,6 @@ __device__ __forceinline__ void small_assemble(const AsmArgs& a, const SmallArgs
       ex[2] = 0.0;
     }
   }
-  (void)otop;
   const double v0 = unit_sum<R>(t_rz), v1 = unit_sum<R>(t_rr), v2 = unit_sum<R>(t_bb);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
@@ -1107,8 +1107,10 @@ void launch_small_assemble(int lanes, const AsmArgs& a, const SmallArgs& g, hipS
 }
 
 // slots per lane (L * M >= PD_SMALL_MAX_BONDS), those in registers, slots
-// per chunk (its gathers are in flight together).  More than eleven slots in
-// registers spill beside a chunk's gathers, so four go to LDS.
+// per chunk (its gathers are in flight together).  With 8 lanes not all
+// fifteen fit the 256 registers beside a chunk's gathers (all in registers 32
+// spill, fourteen 17), and LDS has room for two slots beside the rest (163,040
+// of 163,840 bytes), so thirteen stay in registers (4 spill).
 #define SOLVE8 k_small_solve<8, 15, 13, 4>
 #define SOLVE16 k_small_solve<16, 8, 8, 4>
 #define SOLVE32 k_small_solve<32, 4, 4, 4>
